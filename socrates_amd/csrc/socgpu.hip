@@ -162,8 +162,7 @@ struct CallDims {
   int mcica, mode;   // McICA on, sampling table (0 single, 1 optimal)
   int drop;          // droplet type index (0-based; the stratiform type)
   int nwpc;          // waves per column of the triple-column solve
-  int n_items;       // lanes per column of the packed solve (its g-points, at least kMinItems)
-  int n_waves;       // waves of the packed solve
+  int nw, rpw;       // waves per column of the solve, and rounds of g-points per wave
   int n_gen, n_fill, ipph, ioverlap;
   int triple, drop2; // triple-column representation; convective droplet type
   int raw_range;     // cloud range on the fractions as given (kernel-level cloud_gen)
@@ -1054,19 +1053,23 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
                                            Coef &o) {
 #pragma clang fp contract(off)
   double kgas = (!GEN || t.fnc == SG_FNC_POWER_LAW) ? k_term(t, x.lnp, x.lnt, x.mmr) : x.kx;
-  const double frac1 = x.frac1, kgt = x.kgt, csub = x.cv;
-  if (csub * frac1 > 0.0) {
+  const double kgt = x.kgt, csub = x.cv;
+  const bool cloudy = csub * x.frac1 > 0.0;
+  double tau, om, pf = 0.0, frac1 = 1.0;
+  if (cloudy) {
     // the sub-column's cloudy totals (mcica_sample.F90:614-640): each
     // component, droplets then ice, scaled by c_sub and added in turn
     const double cs = csub;
-    double kg = kgt + x.co[0] * cs, ks = x.ksa + x.co[1] * cs;
-    double pf = x.pfa + x.co[2] * cs, fw = x.fwa + x.co[3] * cs;
+    double kg = kgt + x.co[0] * cs, ks = x.ksa + x.co[1] * cs, fw;
+    pf = x.pfa + x.co[2] * cs;
+    fw = x.fwa + x.co[3] * cs;
     if (c.ice) {
       kg = kg + x.ci[0] * cs;
       ks = ks + x.ci[1] * cs;
       pf = pf + x.ci[2] * cs;
       fw = fw + x.ci[3] * cs;
     }
+    frac1 = x.frac1;
     if (c.nosc) {
       // single_scattering.F90:132-158, mcica_column.F90:509-522
       const double kt = kg + kgas;
@@ -1077,21 +1080,18 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
     pf = (pf - fw) / fmax(ks - fw, kEps);
     fw = fw / fmax(ks, kEps);
     double ktot = kg + kgas;
-    double tau = ktot * x.mass;
-    double om = fmin(ks / (ktot + kTiny), 1.0 - 32.0 * kEps);
+    tau = ktot * x.mass;
+    om = fmin(ks / (ktot + kTiny), 1.0 - 32.0 * kEps);
     tau = tau * (1.0 - om * fw);
     om = om * (1.0 - fw) / (1.0 - om * fw);
-    two_coeff(c.solar, tau, om, pf, c.sec0, o);
-    o.T *= frac1; o.R *= frac1; o.T0 *= frac1; o.s1 *= frac1; o.s2 *= frac1;
   } else {
     double ktot = kgt + kgas;
     if (c.nosc) {
       two_coeff_fast_lw((c.nosc == SOCGPU_SCATTER_NONE ? ktot - x.ksa : ktot) * x.mass, o);
       return;
     }
-    double tau = ktot * x.mass;
-    double om = fmin(x.ksa / (ktot + kTiny), 1.0 - 32.0 * kEps);
-    double pf = 0.0;
+    tau = ktot * x.mass;
+    om = fmin(x.ksa / (ktot + kTiny), 1.0 - 32.0 * kEps);
     if (GEN && c.aer) {
       // clear air with aerosols: moments over the scattering
       // (grey_opt_prop.F90:1360-1440), the phase function delta-rescaled
@@ -1107,8 +1107,10 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
       tau = tau * (1.0 - om * fw);
       om = om * (1.0 - fw) / (1.0 - om * fw);
     }
-    two_coeff(c.solar, tau, om, pf, c.sec0, o);
   }
+  // (one evaluation for the lanes of both kinds: the lanes of a wave differ)
+  two_coeff(c.solar, tau, om, pf, c.sec0, o);
+  if (cloudy) { o.T *= frac1; o.R *= frac1; o.T0 *= frac1; o.s1 *= frac1; o.s2 *= frac1; }
 }
 
 // Mixed form of layer_coef: gas k-term, cloud optics, single scattering and
@@ -1224,564 +1226,24 @@ __device__ __forceinline__ void elim_step(const Coef &o, double su, double sd, d
   rho = rho_n;
 }
 
-// One layer of the top-down elimination for one lane: the layer's
-// coefficients (FP64 layer_coef or the mixed layer_coef_mixed), its sources
-// (solar_source.F90:104-162 with the k_eqv direct-beam adjustment, or
-// ir_source.F90:93-120), and the update of the reflectance of the atmosphere
-// above (rho) and the diffuse flux it sends down (dn). Returns the
-// back-substitution pair fu(i) = a fu(i+1) + bb.
-template <bool MIXED, bool GEN>
-__device__ __forceinline__ void layer_step(const LaneCtx &c, const SgTerm &t, const LayerIn &x,
-                                           double &fdir, double &rho, double &dn, double &a,
-                                           double &bb) {
-#pragma clang fp contract(on)
-  Coef o;
-  if (MIXED) layer_coef_mixed<GEN>(c, t, x, o);
-  else layer_coef<GEN>(c, t, x, o);
-  double su, sd;
-  if (c.solar) {
-    double fnew = fdir * o.T0 * x.q1;
-    su = o.s1 * fdir;
-    sd = (o.s2 - o.T0) * fdir + fnew;
-    fdir = fnew;
-  } else {
-    su = o.s1 * x.q2 + o.s2 * x.q1;
-    sd = -o.s1 * x.q2 + o.s2 * x.q1;
-  }
-  elim_step<MIXED>(o, su, sd, rho, dn, a, bb);
-}
-
-// The column solve, one lane per (column, g-point): the g-point's clear-sky
-// solve (weight w_k (1 - frac_cloudy)) and its McICA sub-column samples
-// (weight w_k frac_cloudy / subcol_k each) (mcica_sample.F90:453-930;
-// monochromatic_radiance.F90:429-691; mcica_column.F90:255-622;
-// solver_homogen_direct.F90:93-127). The lanes of a call are numbered column
-// by column (n_items per column: its g-points) and cut into waves of 64, so a
-// wave spans up to kMaxSeg columns ("segments") and no lane idles between
-// columns. The two-stream system is eliminated top-down (reflectance of the
-// atmosphere above and the downward diffuse flux it emits) and
-// back-substituted bottom-up.
-//
-// Above the column's first cloudy layer (ic) every sample is clear, so its
-// layers, its elimination and its direct beam there are those of the clear
-// solve, to the bit. The lane therefore
-//  1. eliminates the clear layers 0..ic-1 once;
-//  2. for each of its solves, continues from that state through layers
-//     ic..L-1, applies the surface condition and back-substitutes up to
-//     level ic, adding the weighted fluxes of levels ic..L into acc;
-//  3. back-substitutes the layers above ic once for all its solves together:
-//     they share fu(i) = a(i) fu(i+1) + bb(i), so the weighted sum
-//     X(i) = sum_j w_j fu_j(i) obeys X(i) = a(i) X(i+1) + bb(i) W with
-//     W = sum_j w_j, and the downward flux sum is rho(i) X(i) + dn(i) W.
-// This does the work of the reference's clear layers once per g-point
-// instead of once per sample (mcica_column.F90:266-298 recomputes them for
-// every sample); the sums associate differently from a sum of separate
-// solves, by rounding only.
-//
-// Output: partial[wave][segment][3][L+1] (up, down, direct) of the segment's
-// weighted sums, formed by butterflies over the wave with the other
-// segments' lanes masked.
-//
-// RECOMP = false keeps the elimination state of every clear layer above ic
-// (a, bb, rho, dn and the direct flux) in lane-private memory between the
-// sweeps. RECOMP = true keeps only (fdir, rho, dn) at the top of every
-// kSeg-th layer and recomputes each segment's layers (coefficients and
-// elimination, bit-identical to the first sweep) into registers on the way
-// up: a second pass of arithmetic in place of the memory traffic. The layers
-// below ic are few (the cloud sits in the lowest of the log-spaced layers)
-// and are kept in private memory for each solve in turn.
-constexpr int kSeg = 4;
-constexpr int kMaxSeg = 4;     // columns a wave can span (n_items >= kMinItems)
-constexpr int kMinItems = 22;  // floor(63 / 22) + 2 = 4
-
-// Sum over the lanes of segment s of each of v[0..7] (other lanes count
-// zero); lanes 8j (j = 0..7) receive the sum of v[j].
-__device__ __forceinline__ void seg_reduce8(const double (&v)[8], int seg, int s, int nseg, double (&o)[8],
-                                            int lane) {
-#pragma unroll
-  for (int k = 0; k < 8; k++) o[k] = (nseg == 1 || seg == s) ? v[k] : 0.0;
-  reduce8(o, lane);
-}
-
-template <bool MIXED, bool RECOMP, bool GEN>
-__device__ __forceinline__ void solve_body(const CallDims &d, const SgSpec *__restrict__ spec,
-                                           int l_rayleigh, const double *__restrict__ colrec,
-                                           const double *__restrict__ grec,
-                                           const double *__restrict__ colscal,
-                                           const double *__restrict__ bandrec,
-                                           const double *__restrict__ bandscal,
-                                           const double *__restrict__ c_sub,
-                                           const double *__restrict__ cldopt,
-                                           const double *__restrict__ aerrec,
-                                           double *__restrict__ partial, int wave, int lane) {
-#pragma clang fp contract(on)
-  static_assert(kSeg == 4, "checkpoints and output blocks share the 4-layer grid");
-  const int L = d.L, NB = d.NB, IM = d.n_items;
-  const long long g0 = (long long)wave * kWave, gmax = (long long)d.P * IM;
-  if (g0 >= gmax) return;
-  const int colA = (int)(g0 / IM);
-  const long long glast = (g0 + kWave < gmax ? g0 + kWave : gmax) - 1;
-  const int nseg = (int)(glast / IM) - colA + 1;  // wave-uniform, 1..kMaxSeg
-  const long long g = g0 + lane;
-  const bool inrange = g < gmax;
-  const int col = inrange ? (int)(g / IM) : colA;
-  const int item = inrange ? (int)(g - (long long)col * IM) : 0;
-  const int seg = col - colA;
-  const bool solar = d.isolir == SOCGPU_SOURCE_SOLAR;
-  const double *cs = colscal + (size_t)col * SG_NS;
-  const double fc = d.mcica ? cs[SG_S_FC] : 0.0;
-  const bool act = inrange && item < spec->n_g;
-  const int gi = act ? item : 0;
-  const SgTerm t = spec->g[gi];
-  // the lane's solves: the clear one unless every sub-column is cloudy, then
-  // the g-point's samples if any sub-column is
-  const bool clear_on = act && fc < 1.0;
-  const int n_s = (act && d.mcica && fc > 0.0) ? spec->g_n_sub[d.mode][gi] : 0;
-  const int s0 = n_s > 0 ? spec->g_sub0[d.mode][gi] : 0;
-  const int n_solve = act ? (clear_on ? 1 : 0) + n_s : 0;
-  // first layer of the column with cloud (every layer above is clear in
-  // every sub-column); L where the lane has no sample
-  const int ic = n_s > 0 ? min(max((int)cs[SG_S_CT], 0), L) : L;
-  const int b = t.band;
-  double *out = partial + (size_t)wave * kMaxSeg * 3 * (L + 1);
-  const double *rec = colrec + (size_t)col * L * SG_NQ;
-  const double *br = bandrec + ((size_t)col * NB + b) * L * SG_NBQ;
-  const double *bs = bandscal + ((size_t)col * NB + b) * SG_NBQ;
-  LaneCtx c;
-  c.solar = solar;
-  c.sec0 = cs[SG_S_SEC0];
-  c.ksc_clear = (solar && l_rayleigh) ? spec->band[b].rayleigh : 0.0;
-  c.ice = d.ice && !MIXED;
-  c.nosc = term_nosc(d.scat, t.iscat);
-  c.aer = GEN && aerrec != nullptr;
-  LaneSrc src;
-  src.aer = c.aer ? aerrec + ((size_t)col * NB + b) * L * 4 : nullptr;
-  src.rec = rec;
-  src.br = br;
-  src.cop = d.mcica ? cldopt + ((size_t)col * NB + b) * L * d.co_stride : nullptr;
-  src.co_stride = d.co_stride;
-  src.ice = d.ice && !MIXED;
-  src.ksc_clear = c.ksc_clear;
-  src.copf = d.mcica ? (const float *)cldopt + ((size_t)col * NB + b) * L * 4 : nullptr;
-  src.csub = c_sub + (size_t)col * L * SG_MAXSUBCOL;
-  src.csubf = (const float *)c_sub + (size_t)col * L * SG_MAXSUBCOL;
-  src.gas = t.gas;
-  src.isub = 0;
-  src.fnc = t.fnc;
-  src.term = spec->g + gi;
-  src.spec = spec;
-  src.grec = grec ? grec + (size_t)col * L * SG_NGQ : nullptr;
-  const double alb_diff = bs[2], alb_dir = bs[3];
-  const double finc = solar ? bs[0] / c.sec0 : -bs[0];  // flux_inc_down, flux_inc_direct
-
-  // 1. the clear layers above ic, once. Every load and store of the loop is
-  // unconditional (the prefetch index clamped, the checkpoint of a layer
-  // that starts no segment written to a spare row), so the compiler's wait
-  // counts see one path and the prefetch of layer i+1 stays in flight while
-  // layer i is computed.
-  constexpr int kNst = RECOMP ? (SG_MAXL + kSeg - 1) / kSeg : SG_MAXL;
-  double st[kNst + 1][RECOMP ? 3 : 5];
-  double fdir = solar ? finc : 0.0, rho = 0.0, dn = finc;
-  const int ic1 = act ? ic : 0;
-  {
-    LayerIn cur, nxt;
-    load_layer<MIXED, GEN, true>(src, 0, cur);
-    for (int i = 0; i < ic1; i++) {
-      load_layer<MIXED, GEN, true>(src, min(i + 1, ic1 - 1), nxt);
-      if (RECOMP) {
-        const int row = i % kSeg == 0 ? i / kSeg : kNst;
-        st[row][0] = fdir; st[row][1] = rho; st[row][2] = dn;
-      } else {
-        st[i][4] = fdir;
-      }
-      double a, bb;
-      const double rho0 = rho, dn0 = dn;
-      layer_step<MIXED, GEN>(c, t, cur, fdir, rho, dn, a, bb);
-      if (!RECOMP) {
-        st[i][0] = a; st[i][1] = bb; st[i][2] = rho0; st[i][3] = dn0;
-      }
-      cur = nxt;
-    }
-  }
-
-  // 2. each solve from level ic down, back to level ic; weighted fluxes of
-  // levels ic..L in acc[lev - ic]. The downward sweep's loop loads and
-  // stores unconditionally (as step 1); the direct flux at each level is kept
-  // with the layer's elimination pair and added to acc on the way back up.
-  double acc[SG_MAXL + 1][3];
-  const int nacc = act ? L - ic : -1;
-  for (int k = 0; k <= nacc; k++) { acc[k][0] = 0.0; acc[k][1] = 0.0; acc[k][2] = 0.0; }
-  double W = 0.0;
-  {
-    double st2[SG_MAXL][5];
-    const double sg_lw = (1.0 - alb_diff) * (bs[1] - br[(L - 1) * SG_NBQ + 3]);
-    for (int j = 0; j < n_solve; j++) {
-      const bool clr = clear_on && j == 0;
-      const int sI = s0 + j - (clear_on ? 1 : 0);
-      const int isub = clr ? 0 : spec->sub_isub[d.mode][sI];
-      const double wj = clr ? t.w * (1.0 - fc) : t.w * (fc * spec->sub_inv_s[d.mode][sI]);
-      W = W + wj;
-      LaneSrc sj = src;
-      sj.isub = isub;
-      sj.csub = src.csub + (isub > 0 ? isub - 1 : 0);
-      sj.csubf = src.csubf + (isub > 0 ? isub - 1 : 0);
-      double f2 = fdir, r2 = rho, d2 = dn;
-      LayerIn cur, nxt;
-      load_layer<MIXED, GEN>(sj, min(ic, L - 1), cur);
-      for (int i = ic; i < L; i++) {
-        load_layer<MIXED, GEN>(sj, min(i + 1, L - 1), nxt);
-        double a, bb;
-        const double r0 = r2, d0 = d2, f0 = f2;
-        layer_step<MIXED, GEN>(c, t, cur, f2, r2, d2, a, bb);
-        st2[i - ic][0] = a; st2[i - ic][1] = bb; st2[i - ic][2] = r0; st2[i - ic][3] = d0;
-        st2[i - ic][4] = f0;
-        cur = nxt;
-      }
-      if (L > ic) acc[L - ic][2] += wj * f2;
-      const double sgs = solar ? (alb_dir - alb_diff) * f2 : sg_lw;
-      double fu = (alb_diff * d2 + sgs) / (1.0 - alb_diff * r2);
-      double fd = r2 * fu + d2;
-      acc[L - ic][0] += wj * fu;
-      acc[L - ic][1] += wj * fd;
-      for (int lev = L - 1; lev >= ic; lev--) {
-        fu = st2[lev - ic][0] * fu + st2[lev - ic][1];
-        fd = st2[lev - ic][2] * fu + st2[lev - ic][3];
-        acc[lev - ic][0] += wj * fu;
-        acc[lev - ic][1] += wj * fd;
-        if (lev > ic) acc[lev - ic][2] += wj * st2[lev - ic][4];
-      }
-    }
-    if (act) acc[0][2] = W * fdir;   // the direct beam at level ic, common to all
-  }
-
-  // 3. levels L..0 in blocks of 4: below ic from acc, above it the joint
-  // back-substitution of the lane's solves; sums over the segment's lanes
-  double x = act ? acc[0][0] : 0.0;
-  double vdir[8], o8[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) vdir[k] = 0.0;
-  for (int blk = L / kSeg; blk >= 0; blk--) {
-    const int l0 = blk * kSeg;
-    double sa[kSeg], sb[kSeg], sr[kSeg], sd[kSeg], sf[kSeg];
-#pragma unroll
-    for (int k = 0; k < kSeg; k++) { sa[k] = 0.0; sb[k] = 0.0; sr[k] = 0.0; sd[k] = 0.0; sf[k] = 0.0; }
-    if (l0 < ic1) {
-      if (RECOMP) {
-        // the segment's layers again from its checkpoint, each layer's
-        // inputs loaded (unconditionally, index clamped) while the one above
-        // is computed
-        double fs = st[blk][0], rs = st[blk][1], ds = st[blk][2];
-        LayerIn xa, xb;
-        load_layer<MIXED, GEN, true>(src, l0, xa);
-#pragma unroll
-        for (int k = 0; k < kSeg; k++) {
-          const int i = l0 + k;
-          if (k + 1 < kSeg) load_layer<MIXED, GEN, true>(src, min(i + 1, ic1 - 1), xb);
-          sr[k] = rs; sd[k] = ds; sf[k] = fs;
-          if (i < ic1) layer_step<MIXED, GEN>(c, t, xa, fs, rs, ds, sa[k], sb[k]);
-          xa = xb;
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < kSeg; k++) {
-          const int i = l0 + k;
-          if (i < ic1) { sa[k] = st[i][0]; sb[k] = st[i][1]; sr[k] = st[i][2]; sd[k] = st[i][3]; sf[k] = st[i][4]; }
-        }
-      }
-    }
-    double v[8];
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-      const int k = kSeg - 1 - m;   // levels l0+3 .. l0
-      const int lev = l0 + k;
-      double up = 0.0, dw = 0.0, dr = 0.0;
-      if (act && lev <= L) {
-        if (lev >= ic) {
-          up = acc[lev - ic][0]; dw = acc[lev - ic][1]; dr = acc[lev - ic][2];
-        } else {
-          x = sa[k] * x + sb[k] * W;
-          up = x;
-          dw = sr[k] * x + sd[k] * W;
-          dr = W * sf[k];
-        }
-      }
-      v[2 * m] = up;
-      v[2 * m + 1] = dw;
-      if (solar) vdir[(blk & 1) * 4 + k] = dr;
-    }
-    for (int sg = 0; sg < nseg; sg++) {
-      seg_reduce8(v, seg, sg, nseg, o8, lane);
-      if ((lane & 7) == 0) {
-        const int jj = lane >> 3, lev = l0 + kSeg - 1 - (jj >> 1);
-        if (lev <= L) out[(sg * 3 + (jj & 1)) * (L + 1) + lev] = o8[0];
-      }
-    }
-    if (solar && (blk & 1) == 0) {
-      // direct flux of levels l0 .. l0+7
-      for (int sg = 0; sg < nseg; sg++) {
-        seg_reduce8(vdir, seg, sg, nseg, o8, lane);
-        if ((lane & 7) == 0 && l0 + (lane >> 3) <= L) out[(sg * 3 + 2) * (L + 1) + l0 + (lane >> 3)] = o8[0];
-      }
-#pragma unroll
-      for (int k = 0; k < 8; k++) vdir[k] = 0.0;
-    }
-  }
-  if (!solar) {
-    for (int sg = 0; sg < nseg; sg++)
-      for (int i = lane; i <= L; i += kWave) out[(sg * 3 + 2) * (L + 1) + i] = 0.0;
-  }
-}
-
-// The same solve with one lane per item (a clear k-term or one McICA
-// sample, each over the whole column): the layout the mixed form keeps for
-// spectra with the general gas optics. The per-g-point layout above faulted
-// on the device in that one combination (mixed form, general gas optics,
-// stored elimination state) for a cause not yet found; every other
-// combination runs the per-g-point layout.
-template <bool MIXED, bool RECOMP, bool GEN>
-__device__ __forceinline__ void solve_body_items(const CallDims &d, const SgSpec *__restrict__ spec,
-                                           int l_rayleigh, const double *__restrict__ colrec,
-                                           const double *__restrict__ grec,
-                                           const double *__restrict__ colscal,
-                                           const double *__restrict__ bandrec,
-                                           const double *__restrict__ bandscal,
-                                           const double *__restrict__ c_sub,
-                                           const double *__restrict__ cldopt,
-                                           const double *__restrict__ aerrec,
-                                           double *__restrict__ partial, int wave, int lane) {
-#pragma clang fp contract(on)
-  const int L = d.L, NB = d.NB, IM = d.n_items;
-  const long long g0 = (long long)wave * kWave, gmax = (long long)d.P * IM;
-  if (g0 >= gmax) return;
-  const int colA = (int)(g0 / IM);
-  const long long glast = (g0 + kWave < gmax ? g0 + kWave : gmax) - 1;
-  const int nseg = (int)(glast / IM) - colA + 1;  // wave-uniform, 1..kMaxSeg
-  const long long g = g0 + lane;
-  const bool inrange = g < gmax;
-  const int col = inrange ? (int)(g / IM) : colA;
-  const int item = inrange ? (int)(g - (long long)col * IM) : 0;
-  const int seg = col - colA;
-  const bool solar = d.isolir == SOCGPU_SOURCE_SOLAR;
-  const double *cs = colscal + (size_t)col * SG_NS;
-  const double fc = d.mcica ? cs[SG_S_FC] : 0.0;
-  const int G = spec->n_g;
-  int gi = 0, isub = 0;
-  double wgt = 0.0;
-  bool active = false;
-  if (inrange) {
-    if (item < G) {
-      if (fc < 1.0) {
-        active = true;
-        gi = item;
-        wgt = spec->g[gi].w * (1.0 - fc);
-      }
-    } else if (fc > 0.0 && item - G < (d.mcica ? spec->n_sub_items[d.mode] : 0)) {
-      const int sI = item - G;
-      active = true;
-      gi = spec->sub_g[d.mode][sI];
-      isub = spec->sub_isub[d.mode][sI];
-      wgt = spec->g[gi].w * (fc * spec->sub_inv_s[d.mode][sI]);
-    }
-  }
-  double *out = partial + (size_t)wave * kMaxSeg * 3 * (L + 1);
-  const SgTerm t = spec->g[gi];
-  const int b = t.band;
-  const double *rec = colrec + (size_t)col * L * SG_NQ;
-  const double *br = bandrec + ((size_t)col * NB + b) * L * SG_NBQ;
-  const double *bs = bandscal + ((size_t)col * NB + b) * SG_NBQ;
-  LaneCtx c;
-  c.solar = solar;
-  c.sec0 = cs[SG_S_SEC0];
-  c.ksc_clear = (solar && l_rayleigh) ? spec->band[b].rayleigh : 0.0;
-  c.ice = d.ice && !MIXED;
-  c.nosc = term_nosc(d.scat, t.iscat);
-  c.aer = GEN && aerrec != nullptr;
-  LaneSrc src;
-  src.aer = c.aer ? aerrec + ((size_t)col * NB + b) * L * 4 : nullptr;
-  src.rec = rec;
-  src.br = br;
-  src.cop = d.mcica ? cldopt + ((size_t)col * NB + b) * L * d.co_stride : nullptr;
-  src.co_stride = d.co_stride;
-  src.ice = d.ice && !MIXED;
-  src.ksc_clear = c.ksc_clear;
-  src.csub = c_sub + (size_t)col * L * SG_MAXSUBCOL + (isub > 0 ? isub - 1 : 0);
-  src.copf = d.mcica ? (const float *)cldopt + ((size_t)col * NB + b) * L * 4 : nullptr;
-  src.csubf = (const float *)c_sub + (size_t)col * L * SG_MAXSUBCOL + (isub > 0 ? isub - 1 : 0);
-  src.gas = t.gas;
-  src.isub = isub;
-  src.fnc = t.fnc;
-  src.term = spec->g + gi;
-  src.spec = spec;
-  src.grec = grec ? grec + (size_t)col * L * SG_NGQ : nullptr;
-  const double alb_diff = bs[2], alb_dir = bs[3];
-
-  constexpr int kNst = RECOMP ? (SG_MAXL + kSeg - 1) / kSeg : SG_MAXL;
-  double st[kNst][RECOMP ? 3 : 4];
-  const double finc = solar ? bs[0] / c.sec0 : -bs[0];  // flux_inc_down, flux_inc_direct
-  double fdir = solar ? finc : 0.0;
-  double rho = 0.0, dn = finc;
-  double vdir[8], o8[8];
-  LayerIn cur, nxt;
-  load_layer<MIXED, GEN>(src, 0, cur);
-  for (int i = 0; i < L; i++) {
-    if (solar) {
-      // direct flux at the top of layer i, summed 8 levels at a time
-      const int m = i & 7;
-      double x = active ? wgt * fdir : 0.0;
-#pragma unroll
-      for (int k = 0; k < 8; k++) if (k == m) vdir[k] = x;
-      if (m == 7) {
-        for (int sg = 0; sg < nseg; sg++) {
-          seg_reduce8(vdir, seg, sg, nseg, o8, lane);
-          if ((lane & 7) == 0) out[(sg * 3 + 2) * (L + 1) + i - 7 + (lane >> 3)] = o8[0];
-        }
-      }
-    }
-    if (i + 1 < L) load_layer<MIXED, GEN>(src, i + 1, nxt);
-    if (active) {
-      if (RECOMP) {
-        if (i % kSeg == 0) {
-          st[i / kSeg][0] = fdir; st[i / kSeg][1] = rho; st[i / kSeg][2] = dn;
-        }
-      }
-      double a, bb;
-      const double rho0 = rho, dn0 = dn;
-      layer_step<MIXED, GEN>(c, t, cur, fdir, rho, dn, a, bb);
-      if (!RECOMP) {
-        st[i][0] = a; st[i][1] = bb; st[i][2] = rho0; st[i][3] = dn0;
-      }
-    }
-    cur = nxt;
-  }
-  if (solar) {
-    // remaining direct-flux levels (the partial block and the surface)
-    const int base = L & ~7;
-    const int m = L & 7;
-    double x = active ? wgt * fdir : 0.0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      if (k == m) vdir[k] = x;
-      else if (k > m) vdir[k] = 0.0;
-    }
-    for (int sg = 0; sg < nseg; sg++) {
-      seg_reduce8(vdir, seg, sg, nseg, o8, lane);
-      if ((lane & 7) == 0 && base + (lane >> 3) <= L) out[(sg * 3 + 2) * (L + 1) + base + (lane >> 3)] = o8[0];
-    }
-  } else {
-    for (int sg = 0; sg < nseg; sg++)
-      for (int i = lane; i <= L; i += kWave) out[(sg * 3 + 2) * (L + 1) + i] = 0.0;
-  }
-  double fu = 0.0, fd = 0.0;
-  if (active) {
-    double sgs = solar ? (alb_dir - alb_diff) * fdir
-                       : (1.0 - alb_diff) * (bs[1] - br[(L - 1) * SG_NBQ + 3]);
-    fu = (alb_diff * dn + sgs) / (1.0 - alb_diff * rho);
-    fd = rho * fu + dn;
-  }
-  if (!RECOMP) {
-    // back-substitution, levels L..0, 4 levels (x up/down) per reduction
-    for (int top = L; top >= 0; top -= 4) {
-      double v[8];
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        const int lev = top - m;
-        if (lev >= 0 && lev < L && active) {
-          fu = st[lev][0] * fu + st[lev][1];
-          fd = st[lev][2] * fu + st[lev][3];
-        }
-        v[2 * m] = lev >= 0 ? wgt * fu : 0.0;
-        v[2 * m + 1] = lev >= 0 ? wgt * fd : 0.0;
-      }
-      for (int sg = 0; sg < nseg; sg++) {
-        seg_reduce8(v, seg, sg, nseg, o8, lane);
-        if ((lane & 7) == 0) {
-          const int j = lane >> 3, lev = top - (j >> 1);
-          if (lev >= 0) out[(sg * 3 + (j & 1)) * (L + 1) + lev] = o8[0];
-        }
-      }
-    }
-  } else {
-    // surface level, then segments bottom-up: recompute the segment's
-    // layers from its checkpoint into registers, back-substitute them
-    {
-      double v[8];
-#pragma unroll
-      for (int m = 0; m < 4; m++) { v[2 * m] = 0.0; v[2 * m + 1] = 0.0; }
-      v[0] = wgt * fu;
-      v[1] = wgt * fd;
-      for (int sg = 0; sg < nseg; sg++) {
-        seg_reduce8(v, seg, sg, nseg, o8, lane);
-        if ((lane & 7) == 0 && (lane >> 3) < 2) out[(sg * 3 + (lane >> 3)) * (L + 1) + L] = o8[0];
-      }
-    }
-    const int nsegL = (L + kSeg - 1) / kSeg;
-    for (int sgi = nsegL - 1; sgi >= 0; sgi--) {
-      const int i0 = sgi * kSeg;
-      double sa[kSeg], sb[kSeg], sr[kSeg], sdn[kSeg];
-      if (active) {
-        double fdir_s = st[sgi][0], rho_s = st[sgi][1], dn_s = st[sgi][2];
-#pragma unroll
-        for (int k = 0; k < kSeg; k++) {
-          const int i = i0 + k;
-          sr[k] = rho_s; sdn[k] = dn_s; sa[k] = 0.0; sb[k] = 0.0;
-          if (i < L) {
-            LayerIn x;
-            load_layer<MIXED, GEN>(src, i, x);
-            layer_step<MIXED, GEN>(c, t, x, fdir_s, rho_s, dn_s, sa[k], sb[k]);
-          }
-        }
-      }
-      double v[8];
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        const int k = kSeg - 1 - m;   // levels i0+3 .. i0
-        const int lev = i0 + k;
-        if (lev < L && active) {
-          fu = sa[k] * fu + sb[k];
-          fd = sr[k] * fu + sdn[k];
-        }
-        v[2 * m] = lev < L ? wgt * fu : 0.0;
-        v[2 * m + 1] = lev < L ? wgt * fd : 0.0;
-      }
-      for (int sg = 0; sg < nseg; sg++) {
-        seg_reduce8(v, seg, sg, nseg, o8, lane);
-        if ((lane & 7) == 0) {
-          const int j = lane >> 3, lev = i0 + kSeg - 1 - (j >> 1);
-          if (lev < L) out[(sg * 3 + (j & 1)) * (L + 1) + lev] = o8[0];
-        }
-      }
-    }
-  }
-}
-
 // Sum of the per-wave partials, the Planck flux added back for the
 // infra-red (adjust_ir_radiance.F90:186-200, weight_band = 1), output in the
-// caller's [level][profile] layout. A column's partials come from the waves
-// its items fall in (packed solve: partial[wave][segment], in wave order) or
-// from its nwpc waves (triple-column solve: partial[col][chunk]).
+// caller's [level][profile] layout. A column's partials come from its waves,
+// partial[col][wave], summed in wave order (the solve writes no direct flux for
+// an infra-red call: it is zero).
 __device__ __forceinline__ void finish_body(const CallDims &d, const double *__restrict__ partial,
                                             const double *__restrict__ bandrec,
                                             const double *__restrict__ bandscal, int col, int lev,
                                             double &su, double &sd, double &sx) {
   const int L = d.L;
   su = 0.0; sd = 0.0; sx = 0.0;
-  if (d.triple) {
-    for (int c = 0; c < d.nwpc; c++) {
-      const double *o = partial + ((size_t)col * d.nwpc + c) * 3 * (L + 1);
-      su += o[lev];
-      sd += o[(L + 1) + lev];
-      sx += o[2 * (L + 1) + lev];
-    }
-  } else {
-    const long long IM = d.n_items;
-    const long long wa = (long long)col * IM / kWave, wb = ((long long)col * IM + IM - 1) / kWave;
-    for (long long w = wa; w <= wb; w++) {
-      const int sg = col - (int)(w * kWave / IM);
-      const double *o = partial + ((size_t)w * kMaxSeg + sg) * 3 * (L + 1);
-      su += o[lev];
-      sd += o[(L + 1) + lev];
-      sx += o[2 * (L + 1) + lev];
-    }
+  const int nw = d.triple ? d.nwpc : d.nw;
+  const bool direct = d.triple || d.isolir == SOCGPU_SOURCE_SOLAR;
+  for (int c = 0; c < nw; c++) {
+    const double *o = partial + ((size_t)col * nw + c) * 3 * (L + 1);
+    su += o[lev];
+    sd += o[(L + 1) + lev];
+    if (direct) sx += o[2 * (L + 1) + lev];
   }
   if (d.isolir == SOCGPU_SOURCE_THERMAL) {
     double bsum = 0.0;
@@ -2257,10 +1719,10 @@ __device__ __forceinline__ void tri_solve_body(const CallDims &d, const SgSpec *
 // W_GEN counts the calls whose spectrum needs the general gas optics (any
 // scaling other than the power law, continua or further gases); a batch with
 // any such call runs the kernels built for it
-// W_PLAIN counts the calls that do not: the solve kernel of each build runs
-// only the calls of its kind, so a call's solve is the one it gets alone.
-enum { W_LEV, W_LAY, W_CG, W_MINOR, W_PREP, W_SOLVE, W_TOVL, W_TSOLVE, W_PTILE, W_CCOL, W_FTILE, W_LONG, W_GEN,
-       W_PLAIN, W_GBAND, kNWork };
+// W_SOLVE..: waves of the solve, by the build that runs them: columns of up to
+// kShortL layers and longer ones, power-law and general gas optics
+enum { W_LEV, W_LAY, W_CG, W_MINOR, W_PREP, W_SOLVE, W_SOLVE_LONG, W_SOLVE_GEN, W_SOLVE_GEN_LONG, W_TOVL, W_TSOLVE,
+       W_PTILE, W_CCOL, W_FTILE, W_LONG, W_GEN, W_GBAND, kNWork };
 
 struct ReqDesc {
   CallDims d;
@@ -2531,27 +1993,7 @@ __global__ __launch_bounds__(64 * kMinorWaves, NCH == 2 ? SG_BAND_OCC : 2) void 
 }
 
 
-template <bool MIXED, bool RECOMP, int OCC, bool GEN>
-__global__ __launch_bounds__(256, OCC) void b_solve_kernel(const BatchHdr *h, const ReqDesc *rq) {
-  const long long tot = h->tot[W_SOLVE];
-  const int lane = threadIdx.x % kWave;
-  const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
-  for (long long w = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w < tot; w += nw) {
-    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W_SOLVE, w));
-    const ReqDesc &q = rq[r];
-    if ((q.d.gen != 0) != GEN) continue;   // the other build's call
-    if (MIXED && GEN)
-      solve_body_items<MIXED, RECOMP, GEN>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
-                                           G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                           G(q.partial),
-                                           (int)(w - q.s[W_SOLVE]), lane);
-    else
-      solve_body<MIXED, RECOMP, GEN>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
-                                     G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                     G(q.partial),
-                                     (int)(w - q.s[W_SOLVE]), lane);
-  }
-}
+#include "solve_rows.h"
 
 // Outputs in tiles of kFinC columns x kFinL levels per block and iteration:
 // partials read along the levels of a column, transposed through LDS,
@@ -3051,13 +2493,16 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
   return 0;
 }
 
-// Lanes per column of the packed solve and its waves: one lane per g-point,
-// or (per_item: the mixed form's calls that need the general gas optics) one
-// lane per clear k-term and per McICA sample.
-static void solve_layout(CallDims &d, const SgSpec &S, bool per_item) {
-  const int items = S.n_g + ((per_item && d.mcica) ? S.n_sub_items[d.mode] : 0);
-  d.n_items = items > kMinItems ? items : kMinItems;
-  d.n_waves = (int)(((long long)d.P * d.n_items + kWave - 1) / kWave);
+// Waves per column of the solve: a round takes 4 g-points, so a wave per
+// round is the finest split. A call of few columns takes it, for the shortest
+// chain; a call of many columns gives each wave several rounds, which saves
+// partial sums, down to kSolveFill waves in all (a few waves per SIMD).
+constexpr long long kSolveFill = 8192;
+static void solve_layout(CallDims &d, const SgSpec &S) {
+  const int rounds = (S.n_g + kRows - 1) / kRows;
+  const long long want = std::max<long long>(1, std::min<long long>(rounds, (kSolveFill + d.P - 1) / d.P));
+  d.rpw = (int)((rounds + want - 1) / want);
+  d.nw = (rounds + d.rpw - 1) / d.rpw;
 }
 
 // Checks one call's arguments and resolves its options (socrates_set_control
@@ -3203,7 +2648,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
     d.gen = 1;
   }
   d.nwpc = (S.n_g + kWave - 1) / kWave;
-  solve_layout(d, S, precision == SOCGPU_MIXED && d.gen);
+  solve_layout(d, S);
   *entry = &e;
   *dout = d;
   return 0;
@@ -3212,7 +2657,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
 // Per-wave partial sums of a request's solve.
 static size_t partial_doubles(const CallDims &d) {
   if (d.triple) return (size_t)d.P * d.nwpc * 3 * (d.L + 1);
-  return (size_t)d.n_waves * kMaxSeg * 3 * (d.L + 1);
+  return (size_t)d.P * d.nw * 3 * (d.L + 1);
 }
 
 // Device workspace of one request, in doubles (8-byte units), and its work
@@ -3236,14 +2681,15 @@ static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]
   w[W_MINOR] = P * d.NB;
   w[W_LONG] = L > 2 * kWave ? P * d.NB : 0;
   w[W_PREP] = P * d.NB * L;
-  w[W_SOLVE] = d.triple ? 0 : d.n_waves;
+  for (int k : {W_SOLVE, W_SOLVE_LONG, W_SOLVE_GEN, W_SOLVE_GEN_LONG}) w[k] = 0;
+  if (!d.triple)
+    w[d.gen ? (L > kShortL ? W_SOLVE_GEN_LONG : W_SOLVE_GEN) : (L > kShortL ? W_SOLVE_LONG : W_SOLVE)] = P * d.nw;
   w[W_TOVL] = d.triple ? P * (L + 1) : 0;
   w[W_TSOLVE] = d.triple ? P * d.nwpc : 0;
   w[W_PTILE] = pack_tiles(d);
   w[W_CCOL] = (d.mcica || d.triple) ? P * ((L + kRangeChunk - 1) / kRangeChunk) : 0;
   w[W_FTILE] = finish_tiles(d);
   w[W_GEN] = d.gen ? 1 : 0;
-  w[W_PLAIN] = d.gen ? 0 : 1;
   w[W_GBAND] = d.ggen ? 1 : 0;
 }
 
@@ -3294,18 +2740,6 @@ static void fill_desc(ReqDesc &q, const CallDims &d, const SpecEntry &e, const S
 // Launches the kernel sequence of a packed batch on stream s. hdr/rq are
 // device copies of the batch header and descriptors; tot is the host copy of
 // the work totals (grid sizes); solve-kernel time between ev_a and ev_b.
-// The solve kernel of a tile, for the power-law-only or the general gas
-// optics.
-using SolveKernel = void (*)(const BatchHdr *, const ReqDesc *);
-static SolveKernel solve_kernel_for(bool mixed, bool recomp, int occ, bool gen) {
-#define SG_SK(M, R, G) (occ == 3 ? b_solve_kernel<M, R, 3, G> : b_solve_kernel<M, R, 4, G>)
-  if (gen) return mixed ? (recomp ? SG_SK(true, true, true) : SG_SK(true, false, true))
-                        : (recomp ? SG_SK(false, true, true) : SG_SK(false, false, true));
-  return mixed ? (recomp ? SG_SK(true, true, false) : SG_SK(true, false, false))
-               : (recomp ? SG_SK(false, true, false) : SG_SK(false, false, false));
-#undef SG_SK
-}
-
 static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long tot[kNWork], int R,
                         int precision, hipStream_t s, const Fork *fk, hipEvent_t ev_a, hipEvent_t ev_b) {
   const int T = 256;
@@ -3344,21 +2778,16 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   if (ev_a) HIPCHK(hipEventRecord(ev_a, s));
   const SocgpuTile &tile = g_tile[precision == SOCGPU_MIXED ? 1 : 0];
   const int wpb = tile.waves_per_block;
-  // general gas optics: the recomputing tile would evaluate the look-up
-  // tables twice per layer; the storing tile is faster there (GA9 files,
-  // 4096 x 90 all-sky: 5.27 ms per SW+LW step against 6.13 ms)
-  if (tot[W_SOLVE] > 0) {
-    // the power-law build for the calls that need no more, the general one
-    // for the others (each skips the other's calls)
-    if (tot[W_PLAIN] > 0) {
-      auto *kern = solve_kernel_for(precision == SOCGPU_MIXED, tile.recompute != 0, tile.waves_per_simd, false);
-      kern<<<blocks(tot[W_SOLVE], wpb), wpb * kWave, 0, s>>>(hdr, rq);
-    }
-    if (gen) {
-      auto *kern = solve_kernel_for(precision == SOCGPU_MIXED, false, tile.waves_per_simd, true);
-      kern<<<blocks(tot[W_SOLVE], wpb), wpb * kWave, 0, s>>>(hdr, rq);
-    }
+#define SG_SOLVE(KMAX, GEN, W)                                                                       \
+  if (tot[W] > 0) {                                                                                 \
+    auto *k = precision == SOCGPU_MIXED ? b_solve_kernel<true, GEN, KMAX, W> : b_solve_kernel<false, GEN, KMAX, W>; \
+    k<<<blocks(tot[W], wpb), wpb * kWave, solve_lds<KMAX>(wpb), s>>>(hdr, rq);                       \
   }
+  SG_SOLVE(6, false, W_SOLVE)
+  SG_SOLVE(12, false, W_SOLVE_LONG)
+  SG_SOLVE(6, true, W_SOLVE_GEN)
+  SG_SOLVE(12, true, W_SOLVE_GEN_LONG)
+#undef SG_SOLVE
   if (tot[W_TSOLVE] > 0) {
     auto *tk = precision == SOCGPU_MIXED ? (gen ? b_tsolve_kernel<true, true> : b_tsolve_kernel<true, false>)
                                          : (gen ? b_tsolve_kernel<false, true> : b_tsolve_kernel<false, false>);
@@ -4235,24 +3664,24 @@ int socgpu_autotune(int n_request, const SocgpuRequest *requests, int precision,
   SocgpuTile win = saved;
   double best_ms = 1e30;
   if (repeats < 1) repeats = 1;
-  for (int rec = 0; rec <= 1; rec++)
-    for (int wpb : {1, 2, 4})
-      for (int occ : {3, 4}) {
-        {
-          std::lock_guard<std::mutex> lk(g_ctx.mu);
-          g_tile[slot] = SocgpuTile{rec, wpb, occ};
-        }
-        double t = 1e30;
-        for (int r = 0; r <= repeats; r++) {  // the first run warms up
-          if (int rc = socgpu_runes_batch(n_request, requests, precision)) {
-            std::lock_guard<std::mutex> lk(g_ctx.mu);
-            g_tile[slot] = saved;
-            return rc;
-          }
-          if (r > 0) t = std::min(t, g_ctx.last_solve_ms);
-        }
-        if (t < best_ms) { best_ms = t; win = SocgpuTile{rec, wpb, occ}; }
+  for (int wpb : {1, 2, 4}) {
+    SocgpuTile tile = saved;
+    tile.waves_per_block = wpb;
+    {
+      std::lock_guard<std::mutex> lk(g_ctx.mu);
+      g_tile[slot] = tile;
+    }
+    double t = 1e30;
+    for (int r = 0; r <= repeats; r++) {  // the first run warms up
+      if (int rc = socgpu_runes_batch(n_request, requests, precision)) {
+        std::lock_guard<std::mutex> lk(g_ctx.mu);
+        g_tile[slot] = saved;
+        return rc;
       }
+      if (r > 0) t = std::min(t, g_ctx.last_solve_ms);
+    }
+    if (t < best_ms) { best_ms = t; win = tile; }
+  }
   std::lock_guard<std::mutex> lk(g_ctx.mu);
   g_tile[slot] = win;
   *best = win;

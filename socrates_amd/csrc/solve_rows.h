@@ -1,0 +1,578 @@
+// The column solve over rows of lanes: included by socgpu.hip, whose layer
+// inputs and coefficients (LaneCtx, LaneSrc, LayerIn, load_layer,
+// layer_coef*) and lane exchanges it uses.
+//
+// A solve is one (column, g-point) clear or McICA profile: the two-stream
+// system of L layers. 16 consecutive lanes (a DPP row) share one solve, each
+// lane taking K = ceil(layers / 16) consecutive layers in registers, so a
+// wave holds 4 solves of one column. The layers' coefficients are independent
+// and are most of the work; the elimination down the column and the
+// back-substitution up it are recurrences, made parallel across the lanes:
+//  - each lane composes its layers into one slab (transmission, reflection
+//    from above and from below, emitted or scattered flux up and down), by the
+//    adding equations;
+//  - a prefix scan of the slabs over the row gives every lane the reflectance
+//    of the atmosphere above it and the diffuse flux that sends down, from
+//    which the lane eliminates its own layers as a single lane would;
+//  - back-substitution is affine in the flux at the lane's bottom, so a suffix
+//    scan gives every lane that flux.
+// Nothing leaves the registers between the sweeps. One lane per solve kept the
+// elimination state of all layers in lane-private memory (20 KB a lane): the
+// solve then moved 4.6 GB of scratch per 4096 x 90 SW + LW step and waited 63 %
+// of its cycles.
+#pragma once
+
+constexpr int kRowLanes = 16;                 // lanes per solve
+constexpr int kRows = kWave / kRowLanes;      // solves per wave
+constexpr int kLowK = 4;                      // layers per lane of a cloudy part held in LDS
+constexpr int kLowQ = 5;                      // doubles per layer there
+#ifndef SG_OCC6
+#define SG_OCC6 2
+#endif
+constexpr int kShortL = 96;                   // layers of the short build (6 per lane)
+
+// v of the lane CTRL selects, 0 where there is none; and with 1 there.
+template <int CTRL>
+__device__ __forceinline__ double dpp_or0(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)lo32(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)hi32(v), CTRL, 0xf, 0xf, true);
+  return mk64((unsigned)lo, (unsigned)hi);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_or1(double v) { return dpp_f64<CTRL, 0xf>(v, 1.0); }
+
+// row_shr:N (from the lane N below), row_shl:N (N above), row_newbcast:N
+constexpr int kShr = 0x110, kShl = 0x100, kBcast = 0x150, kXor1 = 0xB1;
+
+// 1 / x of a denominator in (0, 1]: the hardware estimate and two Newton steps
+// (within an ulp or two).
+__device__ __forceinline__ double rcp_newton(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(y, fma(-x, y, 1.0), y);
+}
+
+// A run of layers seen from outside: transmission (the same both ways),
+// reflection from above and from below, and its own flux up at the top and
+// down at the bottom.
+struct Slab {
+  double T, Rt, Rb, Su, Sd;
+};
+
+// The slab A above the slab B.
+__device__ __forceinline__ Slab slab_add(const Slab &A, const Slab &B) {
+#pragma clang fp contract(on)
+  const double D = rcp_newton(1.0 - A.Rb * B.Rt);
+  const double tb = B.T * D, ta = A.T * D;
+  Slab S;
+  S.Su = A.Su + ta * (B.Su + B.Rt * A.Sd);
+  S.Sd = B.Sd + tb * (A.Sd + A.Rb * B.Su);
+  S.Rt = A.Rt + ta * B.Rt * A.T;
+  S.Rb = B.Rb + tb * A.Rb * B.T;
+  S.T = ta * B.T;
+  return S;
+}
+
+// Only what the slab A above sends on through B: reflection from below and the
+// flux down.
+__device__ __forceinline__ void slab_below(double Rb, double Sd, const Slab &B, double &rb, double &sd) {
+#pragma clang fp contract(on)
+  const double tb = B.T * rcp_newton(1.0 - Rb * B.Rt);
+  rb = B.Rb + tb * Rb * B.T;
+  sd = B.Sd + tb * (Sd + Rb * B.Su);
+}
+
+// One step of the prefix scan of slabs: the slab N lanes below in the row
+// (zeros where there is none: such a lane's slab already starts at the top of
+// the scanned layers, its state is absolute and only Rb and Sd of it are
+// used again).
+template <int N>
+__device__ __forceinline__ void slab_step(Slab &S) {
+  Slab A;
+  A.T = dpp_or0<kShr + N>(S.T);
+  A.Rt = dpp_or0<kShr + N>(S.Rt);
+  A.Rb = dpp_or0<kShr + N>(S.Rb);
+  A.Su = dpp_or0<kShr + N>(S.Su);
+  A.Sd = dpp_or0<kShr + N>(S.Sd);
+  S = slab_add(A, S);
+}
+
+// The scan over a row whose consecutive slabs lie NS lanes apart.
+template <int NS>
+__device__ __forceinline__ void slab_scan(Slab &S) {
+  if (NS == 1) slab_step<1>(S);
+  slab_step<2>(S);
+  slab_step<4>(S);
+  double rb, sd;
+  slab_below(dpp_or0<kShr + 8>(S.Rb), dpp_or0<kShr + 8>(S.Sd), S, rb, sd);
+  S.Rb = rb;
+  S.Sd = sd;
+}
+
+template <int NS>
+__device__ __forceinline__ double product_scan(double p) {
+  if (NS == 1) p = p * dpp_or1<kShr + 1>(p);
+  p = p * dpp_or1<kShr + 2>(p);
+  p = p * dpp_or1<kShr + 4>(p);
+  p = p * dpp_or1<kShr + 8>(p);
+  return p;
+}
+
+// Suffix scan of the affine maps x -> A x + C, the last of the row's maps
+// being absolute (A unused).
+template <int N>
+__device__ __forceinline__ void affine_up_step(double &A, double &C) {
+#pragma clang fp contract(on)
+  const double A1 = dpp_or0<kShl + N>(A), C1 = dpp_or0<kShl + N>(C);
+  C = A * C1 + C;
+  A = A * A1;
+}
+template <int NS>
+__device__ __forceinline__ void affine_up_scan(double A, double &C) {
+#pragma clang fp contract(on)
+  if (NS == 1) affine_up_step<1>(A, C);
+  affine_up_step<2>(A, C);
+  affine_up_step<4>(A, C);
+  C = A * dpp_or0<kShl + 8>(C) + C;
+}
+
+// Four values per lane summed over the wave's 4 rows, lane by lane: row r
+// gets the sum of value row_value(r).
+__device__ __forceinline__ double sum_rows(double v0, double v1, double v2, double v3) {
+  return swap16_sum(swap32_sum(v0, v1), swap32_sum(v2, v3));
+}
+__device__ __forceinline__ int row_value(int row) { return (row & 1) * 2 + (row >> 1); }
+
+// A wave's level sums in LDS: [up, down, direct][lp], each added to by one
+// lane at a time.
+__device__ __forceinline__ void acc_add(double *p, double v) {
+  (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Two-stream coefficients and sources of one layer. in: the layer is one of
+// the solve's (a lane past the last layer carries the identity). f: the direct
+// beam at the layer's top, relative to the lane's; moved to its bottom.
+template <bool MIXED, bool GEN, bool SOLAR>
+__device__ __forceinline__ void row_layer(const LaneCtx &c, const SgTerm &t, const LayerIn &x, bool in, double &f,
+                                          double &T, double &R, double &su, double &sd) {
+#pragma clang fp contract(on)
+  Coef o;
+  if (MIXED) layer_coef_mixed<GEN>(c, t, x, o);
+  else layer_coef<GEN>(c, t, x, o);
+  T = in ? o.T : 1.0;
+  R = in ? o.R : 0.0;
+  if (SOLAR) {
+    const double fnew = f * o.T0 * x.q1;
+    su = in ? o.s1 * f : 0.0;
+    sd = in ? (o.s2 - o.T0) * f + fnew : 0.0;
+    f = in ? fnew : f;
+  } else {
+    su = in ? o.s1 * x.q2 + o.s2 * x.q1 : 0.0;
+    sd = in ? -o.s1 * x.q2 + o.s2 * x.q1 : 0.0;
+  }
+}
+
+// One layer of the elimination: from (rho, dn) at its top to those at its
+// bottom; a, b: fu(top) = a fu(bottom) + b.
+__device__ __forceinline__ void row_elim(double T, double R, double su, double sd, double &rho, double &dn,
+                                         double &a, double &b) {
+#pragma clang fp contract(on)
+  const double bp = rcp_newton(1.0 - R * rho);
+  a = T * bp;
+  b = (R * dn + su) * bp;
+  const double rho_n = R + T * rho * a;
+  dn = T * (rho * b + dn) + sd;
+  rho = rho_n;
+}
+
+// What a lane keeps of its layers between the sweeps.
+template <int KMAX>
+struct RowState {
+  double a[KMAX], b[KMAX], rho[KMAX], dn[KMAX];
+};
+
+// Down the first n layers of the column, all clear: eliminates the lane's K
+// layers; (rho, dn, fdir) become those at the bottom of the lane's layers
+// (lane 15's: at level n). Adds the direct flux at the levels above n, with
+// weight W, to acc.
+template <bool MIXED, bool GEN, bool SOLAR, int KMAX>
+__device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, const LaneSrc &src, int n, int K, int s,
+                                         int row, double finc, double W, RowState<KMAX> &w, double &rho,
+                                         double &dn, double &fdir, double *acc, int lp) {
+#pragma clang fp contract(on)
+  Slab S{1.0, 0.0, 0.0, 0.0, 0.0};
+  double f = 1.0, fr[SOLAR ? KMAX : 1];
+#pragma unroll
+  for (int k = 0; k < KMAX; k++) {
+    if (k < K) {
+      const int i = s * K + k;
+      LayerIn x;
+      load_layer<MIXED, GEN, true>(src, min(i, n - 1), x);
+      if (SOLAR) fr[k] = f;
+      row_layer<MIXED, GEN, SOLAR>(c, t, x, i < n, f, w.a[k], w.b[k], w.rho[k], w.dn[k]);
+      const Slab B{w.a[k], w.b[k], w.b[k], w.rho[k], w.dn[k]};
+      S = k == 0 ? B : slab_add(S, B);
+    }
+  }
+  double F = 1.0;
+  if (SOLAR) {
+    F = finc * dpp_or1<kShr + 1>(product_scan<1>(f));
+    S.Su = S.Su * F;
+    S.Sd = S.Sd * F;
+    const double WF = W * F;
+    const int v = row_value(row);
+#pragma unroll
+    for (int k0 = 0; k0 < KMAX; k0 += 4) {
+      if (k0 < K) {
+        double d[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) d[j] = (k0 + j < KMAX && k0 + j < K) ? WF * fr[k0 + j < KMAX ? k0 + j : 0] : 0.0;
+        const double z = sum_rows(d[0], d[1], d[2], d[3]);
+        const int k = k0 + v, i = s * K + k;
+        if (k < K && i < n) acc_add(acc + 2 * lp + i, z);
+      }
+    }
+  }
+  if (s == 0) S.Sd = S.Sd + S.T * finc;
+  slab_scan<1>(S);
+  rho = dpp_or0<kShr + 1>(S.Rb);
+  dn = dpp_or0<kShr + 1>(S.Sd);
+  if (s == 0) dn = finc;
+#pragma unroll
+  for (int k = 0; k < KMAX; k++) {
+    if (k < K) {
+      const double T = w.a[k], R = w.b[k];
+      double su = w.rho[k], sd = w.dn[k];
+      if (SOLAR) { su = su * F; sd = sd * F; }
+      w.rho[k] = rho;
+      w.dn[k] = dn;
+      row_elim(T, R, su, sd, rho, dn, w.a[k], w.b[k]);
+    }
+  }
+  fdir = SOLAR ? F * f : 0.0;
+}
+
+// Up the same layers: X the (weighted) upward flux at level n, W the weight
+// of the sources; adds the weighted upward and
+// downward fluxes of the levels above n to acc.
+template <int KMAX>
+__device__ __forceinline__ void row_up(int n, int K, int s, int row, double X, double W, const RowState<KMAX> &w,
+                                       double *acc, int lp) {
+#pragma clang fp contract(on)
+  double A = 1.0, C = 0.0;
+#pragma unroll
+  for (int k = KMAX - 1; k >= 0; k--) {
+    if (k < K) {
+      C = w.a[k] * C + w.b[k];
+      A = w.a[k] * A;
+    }
+  }
+  C = C * W;
+  if (s == kRowLanes - 1) C = A * X + C;
+  affine_up_scan<1>(A, C);
+  double x = dpp_or0<kShl + 1>(C);
+  if (s == kRowLanes - 1) x = X;
+  const int v = row_value(row), i0 = s * K;
+#pragma unroll
+  for (int k0 = ((KMAX - 1) / 2) * 2; k0 >= 0; k0 -= 2) {
+    if (k0 < K) {
+      double up0, dw0, up1 = 0.0, dw1 = 0.0;
+      if (k0 + 1 < KMAX && k0 + 1 < K) {
+        x = w.a[k0 + 1] * x + w.b[k0 + 1] * W;
+        up1 = x;
+        dw1 = w.rho[k0 + 1] * x + w.dn[k0 + 1] * W;
+      }
+      x = w.a[k0] * x + w.b[k0] * W;
+      up0 = x;
+      dw0 = w.rho[k0] * x + w.dn[k0] * W;
+      const double z = sum_rows(up0, dw0, up1, dw1);
+      const int k = k0 + (v >> 1), i = i0 + k;
+      if (k < K && i < n) acc_add(acc + (v & 1) * lp + i, z);
+    }
+  }
+}
+
+// The upward flux at the surface (solver_homogen_direct.F90:93-127).
+template <bool SOLAR>
+__device__ __forceinline__ double surface_up(double alb_diff, double alb_dir, double sg_lw, double rho, double dn,
+                                             double fdir) {
+#pragma clang fp contract(on)
+  const double sg = SOLAR ? (alb_dir - alb_diff) * fdir : sg_lw;
+  return (alb_diff * dn + sg) / (1.0 - alb_diff * rho);
+}
+
+// 0, in a way that the compiler does not see: an index it is added to is a new
+// one in each round, so that the records every round reads again (from the
+// caches) are not held in registers across the rounds.
+__device__ __forceinline__ int opaque0() {
+  int z = 0;
+  asm volatile("" : "+s"(z));
+  return z;
+}
+
+// A row's place in its g-point: weights and samples.
+struct RowItem {
+  int n_clear;      // 1 with a clear solve
+  double w_clear;   // its weight
+  double w_sub;     // weight of each McICA sample
+  int n_s, s0;      // samples, the first one's index
+};
+
+// The cloudy part, layers ic..L-1, of each of the row's solves in turn, NS at
+// a time (interleaved lanes: lane s works on solve s % NS, position s / NS),
+// from the state (rho, dn, fdir) at level ic, which all of them share (every
+// layer above ic is clear in every sub-column). Their number per lane varies
+// from column to column, so the layers' state is indexed memory: LDS (low, up
+// to kLowK layers per lane), or for cloud that reaches higher lane-private
+// memory (KPRIV layers per lane). Adds the weighted fluxes of levels ic..L to
+// acc; returns the weighted upward flux at level ic.
+template <bool MIXED, bool GEN, bool SOLAR, int NS, int KPRIV>
+__device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, const LaneSrc &src,
+                                             const SgSpec *__restrict__ spec, int mode, const RowItem &g, int n_it,
+                                             int L, int ic, int s, int row, int lane, double rho_ic, double dn_ic,
+                                             double f_ic, double alb_diff, double alb_dir, double sg_lw, double *acc,
+                                             int lp, double *low) {
+#pragma clang fp contract(on)
+  constexpr int NP = kRowLanes / NS;   // positions
+  const int p = s / NS, q = s % NS, nl = L - ic;
+  const int K = (nl + NP - 1) / NP;
+  const int v = row_value(row);
+  const bool first = p == 0, last = p == NP - 1;
+  const int n_clear = g.n_clear;
+  double *m = low + lane;
+  double priv[KPRIV > 0 ? KPRIV * kLowQ : 1];
+#define SG_LOW(k, j) (*(KPRIV > 0 ? &priv[(k) * kLowQ + (j)] : &m[((k) * kLowQ + (j)) * kWave]))
+  double xsum = 0.0;
+  for (int it = 0; it < n_it; it++) {
+    const int j = it * NS + q, jc = j - n_clear;
+    const bool clr = n_clear && j == 0, act = clr || (jc >= 0 && jc < g.n_s);
+    LaneSrc sj = src;
+    sj.isub = act && !clr ? spec->sub_isub[mode][g.s0 + jc] : 0;
+    sj.csub = src.csub + (sj.isub > 0 ? sj.isub - 1 : 0);
+    sj.csubf = src.csubf + (sj.isub > 0 ? sj.isub - 1 : 0);
+    const double wj = clr ? g.w_clear : (act ? g.w_sub : 0.0);
+    Slab S{1.0, 0.0, 0.0, 0.0, 0.0};
+    double f = 1.0;
+    for (int k = 0; k < K; k++) {
+      const int r = p * K + k;
+      LayerIn x;
+      load_layer<MIXED, GEN>(sj, ic + min(r, nl - 1), x);
+      Slab B;
+      if (SOLAR) SG_LOW(k, 4) = f;
+      row_layer<MIXED, GEN, SOLAR>(c, t, x, r < nl, f, B.T, B.Rt, B.Su, B.Sd);
+      B.Rb = B.Rt;
+      SG_LOW(k, 0) = B.T;
+      SG_LOW(k, 1) = B.Rt;
+      SG_LOW(k, 2) = B.Su;
+      SG_LOW(k, 3) = B.Sd;
+      S = slab_add(S, B);
+    }
+    double F = 1.0;
+    if (SOLAR) {
+      const double e = dpp_or1<kShr + NS>(product_scan<NS>(f));
+      F = f_ic * e;
+      S.Su = S.Su * F;
+      S.Sd = S.Sd * F;
+    }
+    {
+      double rb, sd;
+      slab_below(rho_ic, dn_ic, S, rb, sd);
+      S.Rb = first ? rb : S.Rb;
+      S.Sd = first ? sd : S.Sd;
+    }
+    slab_scan<NS>(S);
+    double rho = dpp_or0<kShr + NS>(S.Rb), dn = dpp_or0<kShr + NS>(S.Sd);
+    if (first) { rho = rho_ic; dn = dn_ic; }
+    double A = 1.0, C = 0.0;   // fu(top of the lane) = A fu(bottom) + C
+    for (int k = 0; k < K; k++) {
+      const double T = SG_LOW(k, 0), R = SG_LOW(k, 1);
+      double su = SG_LOW(k, 2), sd = SG_LOW(k, 3);
+      if (SOLAR) { su = su * F; sd = sd * F; }
+      SG_LOW(k, 2) = rho;
+      SG_LOW(k, 3) = dn;
+      double a, b;
+      row_elim(T, R, su, sd, rho, dn, a, b);
+      SG_LOW(k, 0) = a;
+      SG_LOW(k, 1) = b;
+      C = C + A * b;
+      A = A * a;
+    }
+    const double fdir = SOLAR ? F * f : 0.0;
+    const double fus = surface_up<SOLAR>(alb_diff, alb_dir, sg_lw, rho, dn, fdir);
+    {
+      // level L, from the last position's lanes
+      const double wl = last ? wj : 0.0;
+      double z = sum_rows(wl * fus, wl * (rho * fus + dn), wl * fdir, 0.0);
+      if (NS == 2) z = z + dpp_move<kXor1>(z);
+      if (last && q == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
+    }
+    if (last) C = A * fus + C;
+    affine_up_scan<NS>(A, C);
+    double fu = dpp_or0<kShl + NS>(C);
+    if (last) fu = fus;
+    for (int k = K - 1; k >= 0; k--) {
+      fu = SG_LOW(k, 0) * fu + SG_LOW(k, 1);
+      const double fd = SG_LOW(k, 2) * fu + SG_LOW(k, 3);
+      const double fb = SOLAR ? F * SG_LOW(k, 4) : 0.0;
+      double z = sum_rows(wj * fu, wj * fd, wj * fb, 0.0);
+      if (NS == 2) z = z + dpp_move<kXor1>(z);
+      const int r = p * K + k;
+      if (r < nl && q == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + ic + r, z);
+    }
+    if (first) xsum = xsum + wj * fu;
+  }
+#undef SG_LOW
+  if (NS == 2) xsum = xsum + dpp_move<kXor1>(xsum);
+  return dpp_or0<kBcast + 0>(xsum);
+}
+
+// The solves of one wave: rounds r0..r1-1 of the column's g-points, 4 a round.
+// (mcica_sample.F90:453-930; monochromatic_radiance.F90:429-691;
+// mcica_column.F90:255-622; solver_homogen_direct.F90:93-127.)
+//
+// In a column with McICA cloud every layer above the first cloudy one (ic) is
+// clear in every sample, so a row goes down those layers once per g-point,
+// then through the layers from ic down once per solve (the clear one and each
+// sample), and back up the shared layers once for all of them together: they
+// share fu(i) = a(i) fu(i+1) + b(i), so the weighted sum X(i) obeys X(i) =
+// a(i) X(i+1) + b(i) W with W the sum of the weights. (mcica_column.F90:266-298
+// recomputes those layers for every sample.)
+//
+// Output: partial[wave][up, down, direct][L+1] of this wave's weighted sums
+// (direct: solar calls only).
+template <bool MIXED, bool GEN, bool SOLAR, int KMAX>
+__device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__restrict__ spec, int l_rayleigh,
+                                           const double *__restrict__ colrec, const double *__restrict__ grec,
+                                           const double *__restrict__ colscal, const double *__restrict__ bandrec,
+                                           const double *__restrict__ bandscal, const double *__restrict__ c_sub,
+                                           const double *__restrict__ cldopt, const double *__restrict__ aerrec,
+                                           double *__restrict__ partial, int wave, int lane, double *acc, int lp,
+                                           double *low) {
+#pragma clang fp contract(on)
+  const int L = d.L, NB = d.NB, G = spec->n_g;
+  const int col = wave / d.nw, part = wave - col * d.nw;
+  const int s = lane % kRowLanes, row = lane / kRowLanes;
+  const double *cs = colscal + (size_t)col * SG_NS;
+  const double fc = d.mcica ? cs[SG_S_FC] : 0.0;
+  const bool cloudy = d.mcica && fc > 0.0;
+  const int ic = cloudy ? min(max((int)cs[SG_S_CT], 0), L) : L;
+  for (int i = lane; i < 3 * lp; i += kWave) acc[i] = 0.0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  const int n_round = (G + kRows - 1) / kRows;
+  const int r1 = min(n_round, (part + 1) * d.rpw);
+  for (int rd = part * d.rpw; rd < r1; rd++) {
+    const int item = rd * kRows + row;
+    const bool act = item < G;
+    const int gi = act ? item : 0;
+    const SgTerm t = spec->g[gi];
+    const int b = t.band;
+    RowItem g;
+    g.n_s = (act && cloudy) ? spec->g_n_sub[d.mode][gi] : 0;
+    g.s0 = g.n_s > 0 ? spec->g_sub0[d.mode][gi] : 0;
+    g.n_clear = act && fc < 1.0;
+    g.w_clear = g.n_clear ? t.w * (1.0 - fc) : 0.0;
+    g.w_sub = g.n_s > 0 ? t.w * (fc * spec->sub_inv_s[d.mode][g.s0]) : 0.0;
+    const double *br = bandrec + ((size_t)col * NB + b) * L * SG_NBQ;
+    const double *bs = bandscal + ((size_t)col * NB + b) * SG_NBQ;
+    LaneCtx c;
+    c.solar = SOLAR;
+    c.sec0 = cs[SG_S_SEC0];
+    c.ksc_clear = (SOLAR && l_rayleigh) ? spec->band[b].rayleigh : 0.0;
+    c.ice = d.ice && !MIXED;
+    c.nosc = SOLAR ? 0 : term_nosc(d.scat, t.iscat);
+    c.aer = GEN && aerrec != nullptr;
+    LaneSrc src;
+    src.aer = c.aer ? aerrec + ((size_t)col * NB + b) * L * 4 : nullptr;
+    src.rec = colrec + ((size_t)col * L * SG_NQ + opaque0());
+    src.br = br;
+    src.cop = d.mcica ? cldopt + ((size_t)col * NB + b) * L * d.co_stride : nullptr;
+    src.co_stride = d.co_stride;
+    src.ice = d.ice && !MIXED;
+    src.ksc_clear = c.ksc_clear;
+    src.copf = d.mcica ? (const float *)cldopt + ((size_t)col * NB + b) * L * 4 : nullptr;
+    src.csub = c_sub + (size_t)col * L * SG_MAXSUBCOL;
+    src.csubf = (const float *)c_sub + (size_t)col * L * SG_MAXSUBCOL;
+    src.gas = t.gas;
+    src.isub = 0;
+    src.fnc = t.fnc;
+    src.term = spec->g + gi;
+    src.spec = spec;
+    src.grec = grec ? grec + (size_t)col * L * SG_NGQ : nullptr;
+    const double alb_diff = bs[2], alb_dir = bs[3];
+    const double finc = SOLAR ? bs[0] / c.sec0 : -bs[0];   // flux_inc_down, flux_inc_direct
+    const double sg_lw = SOLAR ? 0.0 : (1.0 - alb_diff) * (bs[1] - br[(L - 1) * SG_NBQ + 3]);
+    // the row's solves, and the most any row of the wave has
+    const int n_clear = g.n_clear;
+    int n_solve = n_clear + g.n_s;
+    n_solve = max(n_solve, __shfl_xor(n_solve, 16, kWave));
+    n_solve = __builtin_amdgcn_readfirstlane(max(n_solve, __shfl_xor(n_solve, 32, kWave)));
+    const int nl = L - ic;
+    const int K = (ic + kRowLanes - 1) / kRowLanes;
+    RowState<KMAX> w;
+    double rho, dn, fdir;
+    const double W = g.w_clear + g.n_s * g.w_sub;
+    row_down<MIXED, GEN, SOLAR, KMAX>(c, t, src, ic, K, s, row, finc, W, w, rho, dn, fdir, acc, lp);
+    rho = dpp_or0<kBcast + 15>(rho);
+    dn = dpp_or0<kBcast + 15>(dn);
+    if (SOLAR) fdir = dpp_or0<kBcast + 15>(fdir);
+    double X;
+    if (nl == 0) {
+      // no cloud: the surface ends the shared part
+      const double fus = surface_up<SOLAR>(alb_diff, alb_dir, sg_lw, rho, dn, fdir);
+      X = W * fus;
+      const double z = sum_rows(X, W * (rho * fus + dn), W * fdir, 0.0);
+      const int v = row_value(row);
+      if (s == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
+    } else if (nl <= 8 * kLowK) {
+      // two solves side by side where the cloudy layers fit 8 lanes of the row
+      X = row_cloudy<MIXED, GEN, SOLAR, 2, 0>(c, t, src, spec, d.mode, g, (n_solve + 1) / 2, L, ic, s, row, lane,
+                                              rho, dn, fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+    } else if (nl <= 16 * kLowK) {
+      X = row_cloudy<MIXED, GEN, SOLAR, 1, 0>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, row, lane, rho, dn,
+                                              fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+    } else {
+      X = row_cloudy<MIXED, GEN, SOLAR, 1, KMAX>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, row, lane, rho, dn,
+                                                 fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+    }
+    row_up<KMAX>(ic, K, s, row, X, W, w, acc, lp);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  double *out = partial + (size_t)wave * 3 * (L + 1);
+  for (int i = lane; i <= L; i += kWave) {
+    out[i] = acc[i];
+    out[(L + 1) + i] = acc[lp + i];
+    if (SOLAR) out[2 * (L + 1) + i] = acc[2 * lp + i];
+  }
+}
+
+// Waves (64 threads each) of the calls of one build: W the work space. lds:
+// per wave the level sums and the cloudy part's layers.
+template <bool MIXED, bool GEN, int KMAX, int W>
+__global__ __launch_bounds__(256, KMAX == 6 ? SG_OCC6 : 2) void b_solve_kernel(const BatchHdr *h, const ReqDesc *rq) {
+  extern __shared__ double lds[];
+  constexpr int lp = KMAX * kRowLanes + 1;
+  constexpr int per = 3 * lp + kLowK * kLowQ * kWave;
+  const long long tot = h->tot[W];
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  double *acc = lds + wv * per, *low = acc + 3 * lp;
+  const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
+  for (long long w0 = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w0 < tot; w0 += nw) {
+    const int w = __builtin_amdgcn_readfirstlane((int)w0);
+    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W, w));
+    const ReqDesc &q = rq[r];
+    const int wave = w - (int)q.s[W];
+    if (q.d.isolir == SOCGPU_SOURCE_SOLAR)
+      solve_rows<MIXED, GEN, true, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+                                         G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
+                                         G(q.partial), wave, lane, acc, lp, low);
+    else
+      solve_rows<MIXED, GEN, false, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+                                          G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
+                                          G(q.partial), wave, lane, acc, lp, low);
+  }
+}
+
+template <int KMAX>
+constexpr int solve_lds(int waves) {
+  return waves * (3 * (KMAX * kRowLanes + 1) + kLowK * kLowQ * kWave) * 8;
+}
