@@ -370,16 +370,13 @@ int socgpu_serve_replay(SocgpuServer *server, int n_pool, const SocgpuRequest *p
 
 /* Launch shape of the column-solve kernel, per precision form (no reference
  * counterpart; socgpu_autotune picks it):
- *   recompute        0: keep each layer's elimination state in lane-private
- *                       memory between the two sweeps (64 B per lane and
- *                       layer of memory traffic); 1: keep a checkpoint every
- *                       4 layers and recompute each segment in registers on
- *                       the way up (twice the arithmetic, a sixth of the
- *                       traffic). Results are bit-identical either way.
- *   waves_per_block  1, 2 or 4 waves (64 items each: k-terms and McICA
- *                    samples of consecutive columns) per block.
- *   waves_per_simd   3 or 4: the register budget the kernel is compiled for
- *                    (168 or 128 registers per lane). */
+ *   recompute        0 or 1, kept for callers: the solve holds every layer's
+ *                       elimination state in registers and has nothing to
+ *                       recompute.
+ *   waves_per_block  1, 2 or 4 waves (4 solves of one column each) per block.
+ *   waves_per_simd   3 or 4, kept for callers: the register budget follows
+ *                       from the number of layers.
+ * Results are bit-identical for every tile. */
 typedef struct SocgpuTile {
   int recompute;
   int waves_per_block;
@@ -387,10 +384,9 @@ typedef struct SocgpuTile {
 } SocgpuTile;
 
 int socgpu_set_tile(int precision, const SocgpuTile *tile);
-/* Autotuner: times every tile (recompute 0/1 x waves_per_block 1/2/4 x
- * waves_per_simd 3/4) on the given batch with HIP events around the solve
- * kernel (best of `repeats` runs after a warm-up), keeps the fastest for the
- * precision form and returns it. */
+/* Autotuner: times every launch shape (waves_per_block 1/2/4) on the given
+ * batch with HIP events around the solve kernel (best of `repeats` runs after a
+ * warm-up), keeps the fastest for the precision form and returns it. */
 int socgpu_autotune(int n_request, const SocgpuRequest *requests,
                     int precision, int repeats, SocgpuTile *best);
 int socgpu_get_tile(int precision, SocgpuTile *tile);

@@ -54,14 +54,17 @@ struct Coef {
 // lambda = sec(theta_0), infra-red quadratic source for tau near 2^-13), and
 // a contracted product there moves fluxes by up to 1e-4 W m-2; unfused, the
 // device differs from the reference only by its exp.
+// ISO: g is zero (clear air without aerosols); its terms, which are zero, are
+// left out, to the same bits.
+template <bool ISO = false>
 SG_HD void two_coeff(bool solar, double tau, double om, double g, double sec0, Coef &c) {
 #pragma clang fp contract(off)
   double sum, diff;
   if (solar) {
-    sum = 2.0 - 1.5 * om * g - 0.5 * om;
+    sum = ISO ? 2.0 - 0.5 * om : 2.0 - 1.5 * om * g - 0.5 * om;
     diff = 2.0 * (1.0 - om);
   } else {
-    sum = kElsasser - 1.5 * om * g;
+    sum = ISO ? kElsasser : kElsasser - 1.5 * om * g;
     diff = kElsasser * (1.0 - om);
   }
   double lambda = sqrt(sum * diff);
@@ -73,10 +76,15 @@ SG_HD void two_coeff(bool solar, double tau, double om, double g, double sec0, C
       diff *= 1.0 + tolp;
       lambda *= 1.0 + tolp;
     }
-    double ksi0 = 1.5 * g / sec0;
     double factor = 0.5 * om * sec0 / ((lambda - sec0) * (lambda + sec0));
-    gup = factor * (sum - sec0 - ksi0 * (diff - sec0));
-    gdn = factor * (sum + sec0 + ksi0 * (diff + sec0));
+    if (ISO) {
+      gup = factor * (sum - sec0);
+      gdn = factor * (sum + sec0);
+    } else {
+      double ksi0 = 1.5 * g / sec0;
+      gup = factor * (sum - sec0 - ksi0 * (diff - sec0));
+      gdn = factor * (sum + sec0 + ksi0 * (diff + sec0));
+    }
   }
   const double sqe = 1.4901161193847656e-08;  // sqrt(DBL_EPSILON)
   const double tol = 1.220703125e-04;         // sqrt(sqrt(DBL_EPSILON))
@@ -98,6 +106,22 @@ SG_HD void two_coeff(bool solar, double tau, double om, double g, double sec0, C
                          : -2.0 + diff * tau;
     c.s2 = -(1.0 + c.R + c.T + q) / (sum * tau + sqe);
   }
+}
+
+// The infra-red two_coeff of a layer that scatters nothing (om = 0, no
+// aerosols), in the FP64 form: lambda = sqrt(1.66 * 1.66) = 1.66 and gamma = 0,
+// so T = exp(-1.66 tau), R = 0, and the quadratic term q of two_coeff is -2 s1
+// (the same numerator and denominator), all to the same bits. nosc: the term is
+// solved without scattering (two_coeff_fast_lw), which differs in the order of
+// the thin layer's sum only.
+SG_HD void two_coeff_absorb(double tau, bool nosc, double &T, double &s1, double &s2) {
+#pragma clang fp contract(off)
+  const double sqe = 1.4901161193847656e-08, tol = 1.220703125e-04;
+  const double x = kElsasser * tau, den = x + sqe;
+  T = exp(-x);
+  s1 = (1.0 - T + sqe) / den;
+  const double thin = nosc ? 1.0 + T - 2.0 + x : 1.0 + T + (-2.0 + x);
+  s2 = -(tau > tol ? 1.0 + T - 2.0 * s1 : thin) / den;
 }
 
 // Horner evaluation of the band Planck polynomial (planck_flux_band_mod.F90:33-49)

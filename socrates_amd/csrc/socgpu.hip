@@ -1,16 +1,16 @@
 // socgpu: the SOCRATES two-stream flux path on MI355X (gfx950).
 //
-// One radiation call (socgpu_runes) runs five kernels on the library stream:
+// One radiation call (socgpu_runes) runs these kernels on the library stream:
 //   pack      (col,layer) lanes: caller arrays -> per-column layer records
 //   cldrange  (col,layer) lanes: cloud top/base over the call (cloud_gen)
 //   cloudgen  one wave per column, one lane per McICA sub-column
-//   prep      (col,band) lanes: grey extinction, minor-gas equivalent
-//             extinction, solar direct-beam adjustment, Planck terms
-//   solve     one wave per column, one lane per (k-term, sub-column) item:
-//             gas optics, single scattering, two-stream coefficients,
-//             sources and the column solve; g-point-weighted band sums by
-//             wavefront shuffles, one partial per wave
-//   finish    (col,level) lanes: sum of partials, Planck, heating rates
+//   band      one wave per (col,band): minor-gas equivalent extinction, solar
+//             direct-beam adjustment, Planck terms, grey and cloud optics
+//   solve     16 lanes per (col,g-point), over the layers: gas optics, single
+//             scattering, two-stream coefficients, sources and the column
+//             solve; g-point-weighted sums, one partial per wave
+//   finish    (col,level) lanes: sum of partials, Planck
+//   heating   (col,layer) lanes: heating rates
 // The spectral tables live on the device from registration on.
 #include <hip/hip_runtime.h>
 
@@ -56,12 +56,6 @@ static int fail(int code, const char *fmt, ...) {
 
 // ---------------------------------------------------------------- kernels
 constexpr int kWave = 64;
-
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, kWave);
-  return x;
-}
 
 // Cross-lane exchanges of doubles without the LDS: gfx950's
 // v_permlane32_swap / v_permlane16_swap (swap the upper 32 lanes of one
@@ -115,34 +109,7 @@ __device__ __forceinline__ double sum8(double x) {
 
 __device__ __forceinline__ double lane_below(double v) { return dpp_move<0x138>(v); }
 
-// Butterfly reduce-scatter of 16 values per lane over the 64 lanes of a
-// wave: afterwards lanes 4j..4j+3 (j = 0..15) hold the wave total of value j
-// in v[0]. Each step halves the values a lane carries, summing them with
-// the matching values of its partner lane: 15 exchanges instead of the 96
-// of sixteen separate all-reductions.
-__device__ __forceinline__ void reduce16(double (&v)[16], int lane) {
-#pragma unroll
-  for (int k = 0; k < 8; k++) v[k] = swap32_sum(v[k], v[k + 8]);
-#pragma unroll
-  for (int k = 0; k < 4; k++) v[k] = swap16_sum(v[k], v[k + 4]);
-  {
-    const bool hi = lane & 8;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-      const double keep = hi ? v[k + 2] : v[k], give = hi ? v[k] : v[k + 2];
-      v[k] = keep + dpp_move<0x140>(give);  // row_mirror: a partner in the other 8 lanes
-    }
-  }
-  {
-    const bool hi = lane & 4;
-    const double keep = hi ? v[1] : v[0], give = hi ? v[0] : v[1];
-    v[0] = keep + dpp_move<0x141>(give);    // row_half_mirror: the other quad
-  }
-  v[0] = v[0] + dpp_move<0x4E>(v[0]);
-  v[0] = v[0] + dpp_move<0xB1>(v[0]);
-}
-
-// Same for 8 values per lane: lanes 8j..8j+7 (j = 0..7) hold the total of
+// Butterfly reduce-scatter of 8 values per lane over the 64 lanes of a wave: lanes 8j..8j+7 (j = 0..7) hold the total of
 // value j.
 __device__ __forceinline__ void reduce8(double (&v)[8], int lane) {
 #pragma unroll
@@ -970,7 +937,7 @@ struct LaneCtx {
 // that the loads of layer i+1 are in flight while layer i is computed.
 struct LayerIn {
   double lnp, lnt, mmr, mass, frac1;  // column record (wave-uniform but mmr)
-  double kx;                          // the term's k_abs, for scalings other than the power law
+  double kx;                          // the term's k_abs (general gas optics)
   double kgt, q1, q2;                 // band record: grey extinction, adjust or Planck terms
   double ksa, pfa, fwa;               // clear-air scattering and its moment products
                                       // (Rayleigh only: ksc_clear, 0, 0)
@@ -984,11 +951,13 @@ struct LayerIn {
 
 struct LaneSrc {
   const double *rec, *br, *csub, *cop;
+  const double *hot, *mmr;    // in LDS: the column's ln p, ln T and mass, hp apart, and
+  int hp;                     // the mixing ratio of the term's gas
   const float *csubf, *copf;  // FP32 forms (mixed form)
   double ksc_clear;           // clear-air scattering (Rayleigh)
   const double *aer;          // the lane's aerosol record (column, band), or null
   int co_stride, ice;         // doubles per layer of cop; ice optics beside the droplets'
-  int gas, isub;
+  int isub;
   int fnc;                    // the term's scaling function
   const SgTerm *term;         // the term (device table), for fnc other than the power law
   const SgSpec *spec;
@@ -1000,17 +969,19 @@ struct LaneSrc {
 // the lane knows to be clear (above the column's first cloudy layer, or its
 // clear solve): no cloud fraction, scaling or cloud optics are read, so a
 // prefetch of the next layer issues its loads and waits for none of them.
-template <bool MIXED, bool GEN, bool CLR = false>
+template <bool MIXED, bool GEN, bool CLR = false, bool GAS = false>
 __device__ __forceinline__ void load_layer(const LaneSrc &s, int i, LayerIn &x) {
   const double *r = s.rec + i * SG_NQ;
-  x.lnp = r[SG_Q_LNP];
-  x.lnt = r[SG_Q_LNT];
-  x.mmr = r[SG_Q_MMR + s.gas];
-  x.mass = r[SG_Q_MASS];
-  x.kx = (!GEN || s.fnc == SG_FNC_POWER_LAW)
-             ? 0.0
-             : k_scaled(*s.term, s.spec, x.lnp, r[SG_Q_P], r[SG_Q_T], s.grec ? s.grec + i * SG_NGQ : nullptr,
-                        x.mmr);
+  x.lnp = s.hot[i];
+  x.lnt = s.hot[s.hp + i];
+  x.mass = s.hot[2 * s.hp + i];
+  x.mmr = s.mmr[i];
+  if (GEN && !CLR)
+    x.kx = s.fnc != SG_FNC_POWER_LAW
+               ? k_scaled(*s.term, s.spec, x.lnp, r[SG_Q_P], r[SG_Q_T], s.grec ? s.grec + i * SG_NGQ : nullptr, x.mmr)
+               : (MIXED ? (double)k_term_f32(*s.term, (float)x.lnp, (float)x.lnt, (float)x.mmr)
+                        : k_term(*s.term, x.lnp, x.lnt, x.mmr));
+  if (GAS) return;
   const double *q = s.br + i * SG_NBQ;
   x.kgt = q[0];
   x.q1 = q[1];
@@ -1047,14 +1018,15 @@ __device__ __forceinline__ void load_layer(const LaneSrc &s, int i, LayerIn &x) 
   }
 }
 
-// x.co: the layer's cloudy totals of the lane's sub-column (load_layer).
-template <bool GEN>
+// x.co: the layer's cloudy totals of the lane's sub-column (load_layer). CLR:
+// the layer is known to be clear.
+template <bool GEN, bool CLR = false>
 __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, const LayerIn &x,
                                            Coef &o) {
 #pragma clang fp contract(off)
-  double kgas = (!GEN || t.fnc == SG_FNC_POWER_LAW) ? k_term(t, x.lnp, x.lnt, x.mmr) : x.kx;
+  double kgas = GEN ? x.kx : k_term(t, x.lnp, x.lnt, x.mmr);
   const double kgt = x.kgt, csub = x.cv;
-  const bool cloudy = csub * x.frac1 > 0.0;
+  const bool cloudy = !CLR && csub * x.frac1 > 0.0;
   double tau, om, pf = 0.0, frac1 = 1.0;
   if (cloudy) {
     // the sub-column's cloudy totals (mcica_sample.F90:614-640): each
@@ -1070,7 +1042,7 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
       fw = fw + x.ci[3] * cs;
     }
     frac1 = x.frac1;
-    if (c.nosc) {
+    if (GEN && c.nosc) {
       // single_scattering.F90:132-158, mcica_column.F90:509-522
       const double kt = kg + kgas;
       two_coeff_fast_lw((c.nosc == SOCGPU_SCATTER_NONE ? kt - ks : kt) * x.mass, o);
@@ -1086,7 +1058,7 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
     om = om * (1.0 - fw) / (1.0 - om * fw);
   } else {
     double ktot = kgt + kgas;
-    if (c.nosc) {
+    if (GEN && c.nosc) {
       two_coeff_fast_lw((c.nosc == SOCGPU_SCATTER_NONE ? ktot - x.ksa : ktot) * x.mass, o);
       return;
     }
@@ -1108,6 +1080,10 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
       om = om * (1.0 - fw) / (1.0 - om * fw);
     }
   }
+  if (CLR && !(GEN && c.aer)) {
+    two_coeff<true>(c.solar, tau, om, 0.0, c.sec0, o);
+    return;
+  }
   // (one evaluation for the lanes of both kinds: the lanes of a wave differ)
   two_coeff(c.solar, tau, om, pf, c.sec0, o);
   if (cloudy) { o.T *= frac1; o.R *= frac1; o.T0 *= frac1; o.s1 *= frac1; o.s2 *= frac1; }
@@ -1119,13 +1095,11 @@ __device__ __forceinline__ void layer_coef(const LaneCtx &c, const SgTerm &t, co
 // accuracy; the reference's clamp omega <= 1 - 32 eps(FP64) is kept as
 // 1 - omega >= 32 eps(FP64). No FP64 fallback: two_coeff_f32 has no
 // resonance singularity.
-template <bool GEN>
+template <bool GEN, bool CLR = false>
 __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm &t, const LayerIn &x,
                                                 Coef &o) {
 #pragma clang fp contract(on)
-  const float kgas =
-      (!GEN || t.fnc == SG_FNC_POWER_LAW) ? k_term_f32(t, (float)x.lnp, (float)x.lnt, (float)x.mmr)
-                                          : (float)x.kx;
+  const float kgas = GEN ? (float)x.kx : k_term_f32(t, (float)x.lnp, (float)x.lnt, (float)x.mmr);
   const double csub = x.cv;
   const double *co = x.co;
   const float frac1 = (float)x.frac1;
@@ -1133,7 +1107,7 @@ __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm 
   const float mass = (float)x.mass;
   const float omc_min = (float)(32.0 * kEps);
   float tau, om, omc, g;
-  bool cloudy = csub * frac1 > 0.0;
+  const bool cloudy = !CLR && csub * frac1 > 0.0;
   if (cloudy) {
     // absorption kext - kscat formed in FP64 by the prep kernel (relative
     // accuracy ~1e-10 even for weakly absorbing droplets), kept in FP32
@@ -1147,7 +1121,7 @@ __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm 
     fw = SG_FDIV(fw, fmaxf(ks, (float)kEps));
     float ktot = (float)x.ksa + kag + kgas + kext * cs;
     float kab = kag + kgas + kabs * cs;
-    if (c.nosc) {
+    if (GEN && c.nosc) {
       // without scattering: the optical depth of absorption or of
       // extinction, no albedo (single_scattering.F90:132-158)
       CoefF f;
@@ -1166,7 +1140,7 @@ __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm 
     g = pf;
   } else {
     float ktot = (float)x.ksa + kag + kgas;
-    if (c.nosc) {
+    if (GEN && c.nosc) {
       CoefF f;
       two_coeff_f32(false, (c.nosc == SOCGPU_SCATTER_NONE ? kag + kgas : ktot) * mass, 0.0f, 1.0f, 0.0f, 1.0f,
                     f);
@@ -1719,10 +1693,11 @@ __device__ __forceinline__ void tri_solve_body(const CallDims &d, const SgSpec *
 // W_GEN counts the calls whose spectrum needs the general gas optics (any
 // scaling other than the power law, continua or further gases); a batch with
 // any such call runs the kernels built for it
-// W_SOLVE..: waves of the solve, by the build that runs them: columns of up to
-// kShortL layers and longer ones, power-law and general gas optics
-enum { W_LEV, W_LAY, W_CG, W_MINOR, W_PREP, W_SOLVE, W_SOLVE_LONG, W_SOLVE_GEN, W_SOLVE_GEN_LONG, W_TOVL, W_TSOLVE,
-       W_PTILE, W_CCOL, W_FTILE, W_LONG, W_GEN, W_GBAND, kNWork };
+// W_SOLVE + 3 i + opt: waves of the solve, by the build that runs them (i = 0
+// for calls of up to kShortL layers, 1 up to kLongL; opt: kOptPlain, kOptGen,
+// kOptAer); W_SOLVE_ANY: calls of more layers
+enum { W_LEV, W_LAY, W_CG, W_MINOR, W_PREP, W_SOLVE, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE, W_PTILE, W_CCOL,
+       W_FTILE, W_LONG, W_GEN, W_GBAND, kNWork };
 
 struct ReqDesc {
   CallDims d;
@@ -2493,14 +2468,19 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
   return 0;
 }
 
-// Waves per column of the solve: a round takes 4 g-points, so a wave per
-// round is the finest split. A call of few columns takes it, for the shortest
-// chain; a call of many columns gives each wave several rounds, which saves
-// partial sums, down to kSolveFill waves in all (a few waves per SIMD).
-constexpr long long kSolveFill = 8192;
+// Waves per column of the solve, each taking some rounds of 4 g-points. A wave
+// first brings its column into LDS and at its end writes its partial sums, so it
+// should have several rounds; the chip holds 2048 waves of this kernel (two per
+// SIMD), so a call should have about as many. From 16 columns a wave has 3
+// rounds at least (10 000 columns in 216 calls of about 46, mixed: 2.66 ms per
+// batch with one round per wave, 2.45 ms with three); a call of fewer columns
+// takes a wave per round, the shortest chain (4096 x 90 SW + LW, FP64: 1.20 ms
+// per step with 8192 waves per call, 1.18 ms with 2048 to 4096).
+constexpr long long kSolveWaves = 2048;
 static void solve_layout(CallDims &d, const SgSpec &S) {
   const int rounds = (S.n_g + kRows - 1) / kRows;
-  const long long want = std::max<long long>(1, std::min<long long>(rounds, (kSolveFill + d.P - 1) / d.P));
+  const long long most = d.P < 16 ? rounds : (rounds + 2) / 3;
+  const long long want = std::max<long long>(1, std::min<long long>(most, (kSolveWaves + d.P - 1) / d.P));
   d.rpw = (int)((rounds + want - 1) / want);
   d.nw = (rounds + d.rpw - 1) / d.rpw;
 }
@@ -2623,6 +2603,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
   }
   d.ir_lin = !solar && a->l_ir_source_linear;
   d.no_cont = a->l_no_continuum;
+  d.ggen = d.gen;
   // treatment of scattering (socrates_set_control.F90:247-277, 312-318,
   // 368-370; solve_band_k_eqv_scl.F90:1053-1058)
   d.scat = a->i_scatter_method > 0 ? a->i_scatter_method : SOCGPU_SCATTER_FULL;
@@ -2630,6 +2611,8 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
   d.grey1 = d.scat != SOCGPU_SCATTER_FULL;
   for (int g = 0; g < S.n_g; g++) {
     const int m = d.scat == SOCGPU_SCATTER_HYBRID ? (S.g[g].iscat > 0 ? S.g[g].iscat : SOCGPU_SCATTER_FULL) : d.scat;
+    // (the power-law solve build has full scattering only)
+    if (term_nosc(d.scat, S.g[g].iscat)) d.gen = 1;
     if (term_nosc(d.scat, S.g[g].iscat) && solar)
       return fail(SOCGPU_EUNSUPPORTED, "scattering can be ignored in the infra-red only (k-term %d)", g + 1);
     if (term_nosc(d.scat, S.g[g].iscat) && d.triple)
@@ -2639,8 +2622,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
   }
   // modal aerosols (socrates_set_control.F90:378-384: on when modes are
   // given; socrates_set_aer.F90:299-309): the general solve build carries
-  // them; the band kernel's build follows the gas optics alone
-  d.ggen = d.gen;
+  // them; the band kernel's build follows the gas optics alone (d.ggen)
   if (a->n_aer_mode > 0) {
     if (!a->aer_mix_ratio || !a->aer_absorption || !a->aer_scattering || !a->aer_asymmetry)
       return fail(SOCGPU_EINVAL, "aerosol modes need aer_mix_ratio, aer_absorption, aer_scattering and aer_asymmetry");
@@ -2681,9 +2663,11 @@ static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]
   w[W_MINOR] = P * d.NB;
   w[W_LONG] = L > 2 * kWave ? P * d.NB : 0;
   w[W_PREP] = P * d.NB * L;
-  for (int k : {W_SOLVE, W_SOLVE_LONG, W_SOLVE_GEN, W_SOLVE_GEN_LONG}) w[k] = 0;
-  if (!d.triple)
-    w[d.gen ? (L > kShortL ? W_SOLVE_GEN_LONG : W_SOLVE_GEN) : (L > kShortL ? W_SOLVE_LONG : W_SOLVE)] = P * d.nw;
+  for (int k = W_SOLVE; k <= W_SOLVE_ANY; k++) w[k] = 0;
+  if (!d.triple) {
+    const int opt = d.n_aer > 0 ? kOptAer : (d.gen ? kOptGen : kOptPlain);
+    w[L > kLongL ? (int)W_SOLVE_ANY : W_SOLVE + 3 * (L > kShortL) + opt] = P * d.nw;
+  }
   w[W_TOVL] = d.triple ? P * (L + 1) : 0;
   w[W_TSOLVE] = d.triple ? P * d.nwpc : 0;
   w[W_PTILE] = pack_tiles(d);
@@ -2778,15 +2762,18 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   if (ev_a) HIPCHK(hipEventRecord(ev_a, s));
   const SocgpuTile &tile = g_tile[precision == SOCGPU_MIXED ? 1 : 0];
   const int wpb = tile.waves_per_block;
-#define SG_SOLVE(KMAX, GEN, W)                                                                       \
-  if (tot[W] > 0) {                                                                                 \
-    auto *k = precision == SOCGPU_MIXED ? b_solve_kernel<true, GEN, KMAX, W> : b_solve_kernel<false, GEN, KMAX, W>; \
-    k<<<blocks(tot[W], wpb), wpb * kWave, solve_lds<KMAX>(wpb), s>>>(hdr, rq);                       \
+#define SG_SOLVE(KMAX, OPT, W)                                                                               \
+  if (tot[W] > 0) {                                                                                         \
+    auto *k = precision == SOCGPU_MIXED ? b_solve_kernel<true, OPT, KMAX, W> : b_solve_kernel<false, OPT, KMAX, W>; \
+    k<<<blocks(tot[W], wpb), wpb * kWave, wpb * solve_lds_doubles<KMAX>() * 8, s>>>(hdr, rq);                \
   }
-  SG_SOLVE(6, false, W_SOLVE)
-  SG_SOLVE(12, false, W_SOLVE_LONG)
-  SG_SOLVE(6, true, W_SOLVE_GEN)
-  SG_SOLVE(12, true, W_SOLVE_GEN_LONG)
+  SG_SOLVE(6, kOptPlain, W_SOLVE + kOptPlain)
+  SG_SOLVE(6, kOptGen, W_SOLVE + kOptGen)
+  SG_SOLVE(6, kOptAer, W_SOLVE + kOptAer)
+  SG_SOLVE(9, kOptPlain, W_SOLVE + 3 + kOptPlain)
+  SG_SOLVE(9, kOptGen, W_SOLVE + 3 + kOptGen)
+  SG_SOLVE(9, kOptAer, W_SOLVE + 3 + kOptAer)
+  SG_SOLVE(12, kOptAny, W_SOLVE_ANY)
 #undef SG_SOLVE
   if (tot[W_TSOLVE] > 0) {
     auto *tk = precision == SOCGPU_MIXED ? (gen ? b_tsolve_kernel<true, true> : b_tsolve_kernel<true, false>)

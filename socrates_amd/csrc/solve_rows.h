@@ -26,10 +26,13 @@ constexpr int kRowLanes = 16;                 // lanes per solve
 constexpr int kRows = kWave / kRowLanes;      // solves per wave
 constexpr int kLowK = 4;                      // layers per lane of a cloudy part held in LDS
 constexpr int kLowQ = 5;                      // doubles per layer there
-#ifndef SG_OCC6
-#define SG_OCC6 2
-#endif
-constexpr int kShortL = 96;                   // layers of the short build (6 per lane)
+constexpr int kHotQ = 7;                      // column record slots a wave keeps in LDS
+// Builds of the kernel by the call's layers, 6 or 9 per lane (a lane's state is
+// in registers; 9 cost the short calls 72 of them), and its optics: power-law
+// gases without aerosols; any gas scaling and treatment of scattering; that with
+// aerosols. Calls of more layers than kLongL are few: one build for all optics.
+constexpr int kShortL = 6 * kRowLanes, kLongL = 9 * kRowLanes;
+enum { kOptPlain, kOptGen, kOptAer, kOptAny };
 
 // v of the lane CTRL selects, 0 where there is none; and with 1 there.
 template <int CTRL>
@@ -136,6 +139,22 @@ __device__ __forceinline__ void affine_up_scan(double A, double &C) {
   C = A * dpp_or0<kShl + 8>(C) + C;
 }
 
+// The same down the row, the first of its maps being absolute.
+template <int N>
+__device__ __forceinline__ void affine_down_step(double &A, double &C) {
+#pragma clang fp contract(on)
+  const double A1 = dpp_or0<kShr + N>(A), C1 = dpp_or0<kShr + N>(C);
+  C = A * C1 + C;
+  A = A * A1;
+}
+__device__ __forceinline__ void affine_down_scan(double A, double &C) {
+#pragma clang fp contract(on)
+  affine_down_step<1>(A, C);
+  affine_down_step<2>(A, C);
+  affine_down_step<4>(A, C);
+  C = A * dpp_or0<kShr + 8>(C) + C;
+}
+
 // Four values per lane summed over the wave's 4 rows, lane by lane: row r
 // gets the sum of value row_value(r).
 __device__ __forceinline__ double sum_rows(double v0, double v1, double v2, double v3) {
@@ -152,13 +171,13 @@ __device__ __forceinline__ void acc_add(double *p, double v) {
 // Two-stream coefficients and sources of one layer. in: the layer is one of
 // the solve's (a lane past the last layer carries the identity). f: the direct
 // beam at the layer's top, relative to the lane's; moved to its bottom.
-template <bool MIXED, bool GEN, bool SOLAR>
+template <bool MIXED, bool GEN, bool SOLAR, bool CLR>
 __device__ __forceinline__ void row_layer(const LaneCtx &c, const SgTerm &t, const LayerIn &x, bool in, double &f,
                                           double &T, double &R, double &su, double &sd) {
 #pragma clang fp contract(on)
   Coef o;
-  if (MIXED) layer_coef_mixed<GEN>(c, t, x, o);
-  else layer_coef<GEN>(c, t, x, o);
+  if (MIXED) layer_coef_mixed<GEN, CLR>(c, t, x, o);
+  else layer_coef<GEN, CLR>(c, t, x, o);
   T = in ? o.T : 1.0;
   R = in ? o.R : 0.0;
   if (SOLAR) {
@@ -185,31 +204,62 @@ __device__ __forceinline__ void row_elim(double T, double R, double su, double s
   rho = rho_n;
 }
 
-// What a lane keeps of its layers between the sweeps.
-template <int KMAX>
-struct RowState {
-  double a[KMAX], b[KMAX], rho[KMAX], dn[KMAX];
+// The layers of a run of n that lane s of its row takes: K on the first lanes,
+// K - 1 on the others, from layer i0.
+struct RowMap {
+  int K, i0;
+  bool full;
+  __device__ __forceinline__ bool has(int k) const { return k + 1 < K || full; }
 };
+__device__ __forceinline__ RowMap row_map(int n, int s) {
+  const int K = (n + kRowLanes - 1) / kRowLanes, rem = n - kRowLanes * (K - 1);
+  return RowMap{K, s * (K - 1) + min(s, rem), s < rem};
+}
+
+// What a lane keeps of its layers between the sweeps. ABS: layers that do not
+// scatter, whose reflection (and so rho) is zero.
+template <int KMAX, bool ABS>
+struct RowState {
+  double a[KMAX], b[KMAX], dn[KMAX], rho[ABS ? 1 : KMAX];
+};
+
+// General gas optics: the term's absorption in each of the lane's layers,
+// ahead of the unrolled layer code (which would hold every scaling K times).
+template <bool MIXED>
+__device__ __forceinline__ void row_gas(const SgTerm &t, const LaneSrc &src, int n, const RowMap &mp, double *low,
+                                        int lane) {
+  for (int k = 0; k < mp.K; k++) {
+    const int i = min(mp.i0 + k, n - 1);
+    LayerIn x;
+    load_layer<MIXED, true, false, true>(src, i, x);
+    low[k * kWave + lane] = x.kx;
+  }
+}
 
 // Down the first n layers of the column, all clear: eliminates the lane's K
 // layers; (rho, dn, fdir) become those at the bottom of the lane's layers
 // (lane 15's: at level n). Adds the direct flux at the levels above n, with
 // weight W, to acc.
 template <bool MIXED, bool GEN, bool SOLAR, int KMAX>
-__device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, const LaneSrc &src, int n, int K, int s,
-                                         int row, double finc, double W, RowState<KMAX> &w, double &rho,
-                                         double &dn, double &fdir, double *acc, int lp) {
+__device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, const LaneSrc &src, int n,
+                                         const RowMap &mp, int s, int row, double finc, double W,
+                                         RowState<KMAX, false> &w, double &rho, double &dn, double &fdir, double *acc,
+                                         int lp, double *low, int lane) {
 #pragma clang fp contract(on)
   Slab S{1.0, 0.0, 0.0, 0.0, 0.0};
   double f = 1.0, fr[SOLAR ? KMAX : 1];
+  if (GEN) row_gas<MIXED>(t, src, n, mp, low, lane);
+  // each layer's inputs are loaded while the one before is computed
+  LayerIn x, nx;
+  load_layer<MIXED, GEN, true>(src, max(min(mp.i0, n - 1), 0), nx);
 #pragma unroll
   for (int k = 0; k < KMAX; k++) {
-    if (k < K) {
-      const int i = s * K + k;
-      LayerIn x;
-      load_layer<MIXED, GEN, true>(src, min(i, n - 1), x);
+    if (k < mp.K) {
+      x = nx;
+      if (GEN) x.kx = low[k * kWave + lane];
+      if (k + 1 < KMAX) load_layer<MIXED, GEN, true>(src, min(mp.i0 + k + 1, n - 1), nx);
       if (SOLAR) fr[k] = f;
-      row_layer<MIXED, GEN, SOLAR>(c, t, x, i < n, f, w.a[k], w.b[k], w.rho[k], w.dn[k]);
+      row_layer<MIXED, GEN, SOLAR, true>(c, t, x, mp.has(k), f, w.a[k], w.b[k], w.rho[k], w.dn[k]);
       const Slab B{w.a[k], w.b[k], w.b[k], w.rho[k], w.dn[k]};
       S = k == 0 ? B : slab_add(S, B);
     }
@@ -223,13 +273,14 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
     const int v = row_value(row);
 #pragma unroll
     for (int k0 = 0; k0 < KMAX; k0 += 4) {
-      if (k0 < K) {
+      if (k0 < mp.K) {
         double d[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = (k0 + j < KMAX && k0 + j < K) ? WF * fr[k0 + j < KMAX ? k0 + j : 0] : 0.0;
+        for (int j = 0; j < 4; j++)
+          d[j] = (k0 + j < KMAX && k0 + j < mp.K) ? WF * fr[k0 + j < KMAX ? k0 + j : 0] : 0.0;
         const double z = sum_rows(d[0], d[1], d[2], d[3]);
-        const int k = k0 + v, i = s * K + k;
-        if (k < K && i < n) acc_add(acc + 2 * lp + i, z);
+        const int k = k0 + v;
+        if (k < mp.K && mp.has(k)) acc_add(acc + 2 * lp + mp.i0 + k, z);
       }
     }
   }
@@ -240,7 +291,7 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
   if (s == 0) dn = finc;
 #pragma unroll
   for (int k = 0; k < KMAX; k++) {
-    if (k < K) {
+    if (k < mp.K) {
       const double T = w.a[k], R = w.b[k];
       double su = w.rho[k], sd = w.dn[k];
       if (SOLAR) { su = su * F; sd = sd * F; }
@@ -252,17 +303,58 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
   fdir = SOLAR ? F * f : 0.0;
 }
 
+// row_down of infra-red layers that do not scatter, FP64 form: the flux goes
+// down them by one affine recurrence, and fu(top) = T fu(bottom) + su.
+template <bool GEN, int KMAX>
+__device__ __forceinline__ void row_down_absorb(const LaneCtx &c, const SgTerm &t, const LaneSrc &src, int n,
+                                                const RowMap &mp, int s, double finc, RowState<KMAX, true> &w,
+                                                double &dn, double *low, int lane) {
+#pragma clang fp contract(on)
+  if (GEN) row_gas<false>(t, src, n, mp, low, lane);
+  LayerIn x, nx;
+  load_layer<false, GEN, true>(src, max(min(mp.i0, n - 1), 0), nx);
+  double A = 1.0, C = 0.0;
+#pragma unroll
+  for (int k = 0; k < KMAX; k++) {
+    if (k < mp.K) {
+      x = nx;
+      if (k + 1 < KMAX) load_layer<false, GEN, true>(src, min(mp.i0 + k + 1, n - 1), nx);
+      const double kgas = GEN ? low[k * kWave + lane] : k_term(t, x.lnp, x.lnt, x.mmr);
+      double T, s1, s2;
+      two_coeff_absorb((x.kgt + kgas) * x.mass, GEN && c.nosc, T, s1, s2);
+      const bool in = mp.has(k);
+      w.a[k] = in ? T : 1.0;
+      w.b[k] = in ? s1 * x.q2 + s2 * x.q1 : 0.0;
+      w.dn[k] = in ? -s1 * x.q2 + s2 * x.q1 : 0.0;
+      C = w.a[k] * C + w.dn[k];
+      A = w.a[k] * A;
+    }
+  }
+  if (s == 0) C = A * finc + C;
+  affine_down_scan(A, C);
+  dn = dpp_or0<kShr + 1>(C);
+  if (s == 0) dn = finc;
+#pragma unroll
+  for (int k = 0; k < KMAX; k++) {
+    if (k < mp.K) {
+      const double sd = w.dn[k];
+      w.dn[k] = dn;
+      dn = w.a[k] * dn + sd;
+    }
+  }
+}
+
 // Up the same layers: X the (weighted) upward flux at level n, W the weight
-// of the sources; adds the weighted upward and
-// downward fluxes of the levels above n to acc.
-template <int KMAX>
-__device__ __forceinline__ void row_up(int n, int K, int s, int row, double X, double W, const RowState<KMAX> &w,
-                                       double *acc, int lp) {
+// of the sources; adds the weighted upward and downward fluxes of the levels
+// above n to acc.
+template <int KMAX, bool ABS>
+__device__ __forceinline__ void row_up(const RowMap &mp, int s, int row, double X, double W,
+                                       const RowState<KMAX, ABS> &w, double *acc, int lp) {
 #pragma clang fp contract(on)
   double A = 1.0, C = 0.0;
 #pragma unroll
   for (int k = KMAX - 1; k >= 0; k--) {
-    if (k < K) {
+    if (k < mp.K) {
       C = w.a[k] * C + w.b[k];
       A = w.a[k] * A;
     }
@@ -272,22 +364,23 @@ __device__ __forceinline__ void row_up(int n, int K, int s, int row, double X, d
   affine_up_scan<1>(A, C);
   double x = dpp_or0<kShl + 1>(C);
   if (s == kRowLanes - 1) x = X;
-  const int v = row_value(row), i0 = s * K;
+  const int v = row_value(row);
 #pragma unroll
   for (int k0 = ((KMAX - 1) / 2) * 2; k0 >= 0; k0 -= 2) {
-    if (k0 < K) {
-      double up0, dw0, up1 = 0.0, dw1 = 0.0;
-      if (k0 + 1 < KMAX && k0 + 1 < K) {
-        x = w.a[k0 + 1] * x + w.b[k0 + 1] * W;
-        up1 = x;
-        dw1 = w.rho[k0 + 1] * x + w.dn[k0 + 1] * W;
+    if (k0 < mp.K) {
+      double up[2] = {0.0, 0.0}, dw[2] = {0.0, 0.0};
+#pragma unroll
+      for (int j = 1; j >= 0; j--) {
+        const int k = k0 + j;
+        if (k < KMAX && k < mp.K) {
+          x = w.a[k < KMAX ? k : 0] * x + w.b[k < KMAX ? k : 0] * W;
+          up[j] = x;
+          dw[j] = ABS ? w.dn[k < KMAX ? k : 0] * W : w.rho[ABS ? 0 : (k < KMAX ? k : 0)] * x + w.dn[k < KMAX ? k : 0] * W;
+        }
       }
-      x = w.a[k0] * x + w.b[k0] * W;
-      up0 = x;
-      dw0 = w.rho[k0] * x + w.dn[k0] * W;
-      const double z = sum_rows(up0, dw0, up1, dw1);
-      const int k = k0 + (v >> 1), i = i0 + k;
-      if (k < K && i < n) acc_add(acc + (v & 1) * lp + i, z);
+      const double z = sum_rows(up[0], dw[0], up[1], dw[1]);
+      const int k = k0 + (v >> 1);
+      if (k < mp.K && mp.has(k)) acc_add(acc + (v & 1) * lp + mp.i0 + k, z);
     }
   }
 }
@@ -299,15 +392,6 @@ __device__ __forceinline__ double surface_up(double alb_diff, double alb_dir, do
 #pragma clang fp contract(on)
   const double sg = SOLAR ? (alb_dir - alb_diff) * fdir : sg_lw;
   return (alb_diff * dn + sg) / (1.0 - alb_diff * rho);
-}
-
-// 0, in a way that the compiler does not see: an index it is added to is a new
-// one in each round, so that the records every round reads again (from the
-// caches) are not held in registers across the rounds.
-__device__ __forceinline__ int opaque0() {
-  int z = 0;
-  asm volatile("" : "+s"(z));
-  return z;
 }
 
 // A row's place in its g-point: weights and samples.
@@ -359,7 +443,7 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
       load_layer<MIXED, GEN>(sj, ic + min(r, nl - 1), x);
       Slab B;
       if (SOLAR) SG_LOW(k, 4) = f;
-      row_layer<MIXED, GEN, SOLAR>(c, t, x, r < nl, f, B.T, B.Rt, B.Su, B.Sd);
+      row_layer<MIXED, GEN, SOLAR, false>(c, t, x, r < nl, f, B.T, B.Rt, B.Su, B.Sd);
       B.Rb = B.Rt;
       SG_LOW(k, 0) = B.T;
       SG_LOW(k, 1) = B.Rt;
@@ -440,15 +524,16 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
 //
 // Output: partial[wave][up, down, direct][L+1] of this wave's weighted sums
 // (direct: solar calls only).
-template <bool MIXED, bool GEN, bool SOLAR, int KMAX>
+template <bool MIXED, int OPT, bool SOLAR, int KMAX>
 __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__restrict__ spec, int l_rayleigh,
                                            const double *__restrict__ colrec, const double *__restrict__ grec,
                                            const double *__restrict__ colscal, const double *__restrict__ bandrec,
                                            const double *__restrict__ bandscal, const double *__restrict__ c_sub,
                                            const double *__restrict__ cldopt, const double *__restrict__ aerrec,
                                            double *__restrict__ partial, int wave, int lane, double *acc, int lp,
-                                           double *low) {
+                                           double *low, double *hot) {
 #pragma clang fp contract(on)
+  constexpr bool GEN = OPT != kOptPlain;
   const int L = d.L, NB = d.NB, G = spec->n_g;
   const int col = wave / d.nw, part = wave - col * d.nw;
   const int s = lane % kRowLanes, row = lane / kRowLanes;
@@ -457,6 +542,13 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
   const bool cloudy = d.mcica && fc > 0.0;
   const int ic = cloudy ? min(max((int)cs[SG_S_CT], 0), L) : L;
   for (int i = lane; i < 3 * lp; i += kWave) acc[i] = 0.0;
+  // the column's ln p, ln T, mass and mixing ratios, read by every round
+  static_assert(SG_Q_LNP == 0 && SG_Q_LNT == 1 && SG_Q_MASS == 2 && SG_Q_MMR == 3, "the record's first kHotQ slots");
+  for (int i = lane; i < L; i += kWave) {
+    const double *r = colrec + ((size_t)col * L + i) * SG_NQ;
+#pragma unroll
+    for (int j = 0; j < kHotQ; j++) hot[j * lp + i] = r[j];
+  }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   const int n_round = (G + kRows - 1) / kRows;
   const int r1 = min(n_round, (part + 1) * d.rpw);
@@ -479,11 +571,11 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
     c.sec0 = cs[SG_S_SEC0];
     c.ksc_clear = (SOLAR && l_rayleigh) ? spec->band[b].rayleigh : 0.0;
     c.ice = d.ice && !MIXED;
-    c.nosc = SOLAR ? 0 : term_nosc(d.scat, t.iscat);
-    c.aer = GEN && aerrec != nullptr;
+    c.nosc = GEN && !SOLAR ? term_nosc(d.scat, t.iscat) : 0;
+    c.aer = OPT == kOptAer || (OPT == kOptAny && aerrec != nullptr);
     LaneSrc src;
     src.aer = c.aer ? aerrec + ((size_t)col * NB + b) * L * 4 : nullptr;
-    src.rec = colrec + ((size_t)col * L * SG_NQ + opaque0());
+    src.rec = colrec + (size_t)col * L * SG_NQ;
     src.br = br;
     src.cop = d.mcica ? cldopt + ((size_t)col * NB + b) * L * d.co_stride : nullptr;
     src.co_stride = d.co_stride;
@@ -492,7 +584,9 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
     src.copf = d.mcica ? (const float *)cldopt + ((size_t)col * NB + b) * L * 4 : nullptr;
     src.csub = c_sub + (size_t)col * L * SG_MAXSUBCOL;
     src.csubf = (const float *)c_sub + (size_t)col * L * SG_MAXSUBCOL;
-    src.gas = t.gas;
+    src.hot = hot;
+    src.hp = lp;
+    src.mmr = hot + (3 + t.gas) * lp;
     src.isub = 0;
     src.fnc = t.fnc;
     src.term = spec->g + gi;
@@ -507,34 +601,41 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
     n_solve = max(n_solve, __shfl_xor(n_solve, 16, kWave));
     n_solve = __builtin_amdgcn_readfirstlane(max(n_solve, __shfl_xor(n_solve, 32, kWave)));
     const int nl = L - ic;
-    const int K = (ic + kRowLanes - 1) / kRowLanes;
-    RowState<KMAX> w;
-    double rho, dn, fdir;
+    const RowMap mp = row_map(ic, s);
     const double W = g.w_clear + g.n_s * g.w_sub;
-    row_down<MIXED, GEN, SOLAR, KMAX>(c, t, src, ic, K, s, row, finc, W, w, rho, dn, fdir, acc, lp);
-    rho = dpp_or0<kBcast + 15>(rho);
-    dn = dpp_or0<kBcast + 15>(dn);
-    if (SOLAR) fdir = dpp_or0<kBcast + 15>(fdir);
-    double X;
-    if (nl == 0) {
-      // no cloud: the surface ends the shared part
-      const double fus = surface_up<SOLAR>(alb_diff, alb_dir, sg_lw, rho, dn, fdir);
-      X = W * fus;
-      const double z = sum_rows(X, W * (rho * fus + dn), W * fdir, 0.0);
-      const int v = row_value(row);
-      if (s == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
-    } else if (nl <= 8 * kLowK) {
+    // the layers from ic down: the surface, or the cloudy part first
+    const auto below = [&](double rho, double dn, double fdir) -> double {
+      if (nl == 0) {
+        const double fus = surface_up<SOLAR>(alb_diff, alb_dir, sg_lw, rho, dn, fdir);
+        const double X = W * fus;
+        const double z = sum_rows(X, W * (rho * fus + dn), W * fdir, 0.0);
+        const int v = row_value(row);
+        if (s == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
+        return X;
+      }
       // two solves side by side where the cloudy layers fit 8 lanes of the row
-      X = row_cloudy<MIXED, GEN, SOLAR, 2, 0>(c, t, src, spec, d.mode, g, (n_solve + 1) / 2, L, ic, s, row, lane,
-                                              rho, dn, fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
-    } else if (nl <= 16 * kLowK) {
-      X = row_cloudy<MIXED, GEN, SOLAR, 1, 0>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, row, lane, rho, dn,
-                                              fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+      if (nl <= 8 * kLowK)
+        return row_cloudy<MIXED, GEN, SOLAR, 2, 0>(c, t, src, spec, d.mode, g, (n_solve + 1) / 2, L, ic, s, row, lane,
+                                                   rho, dn, fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+      return row_cloudy<MIXED, GEN, SOLAR, 1, KMAX>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, row, lane, rho, dn,
+                                                    fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+    };
+    double rho, dn, fdir;
+    if (!MIXED && !SOLAR && !c.aer) {
+      // infra-red clear air without aerosols does not scatter
+      RowState<KMAX, true> w;
+      row_down_absorb<GEN, KMAX>(c, t, src, ic, mp, s, finc, w, dn, low, lane);
+      const double X = below(0.0, dpp_or0<kBcast + 15>(dn), 0.0);
+      row_up<KMAX, true>(mp, s, row, X, W, w, acc, lp);
     } else {
-      X = row_cloudy<MIXED, GEN, SOLAR, 1, KMAX>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, row, lane, rho, dn,
-                                                 fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+      RowState<KMAX, false> w;
+      row_down<MIXED, GEN, SOLAR, KMAX>(c, t, src, ic, mp, s, row, finc, W, w, rho, dn, fdir, acc, lp, low, lane);
+      rho = dpp_or0<kBcast + 15>(rho);
+      dn = dpp_or0<kBcast + 15>(dn);
+      if (SOLAR) fdir = dpp_or0<kBcast + 15>(fdir);
+      const double X = below(rho, dn, fdir);
+      row_up<KMAX, false>(mp, s, row, X, W, w, acc, lp);
     }
-    row_up<KMAX>(ic, K, s, row, X, W, w, acc, lp);
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   double *out = partial + (size_t)wave * 3 * (L + 1);
@@ -545,16 +646,20 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
   }
 }
 
-// Waves (64 threads each) of the calls of one build: W the work space. lds:
-// per wave the level sums and the cloudy part's layers.
-template <bool MIXED, bool GEN, int KMAX, int W>
-__global__ __launch_bounds__(256, KMAX == 6 ? SG_OCC6 : 2) void b_solve_kernel(const BatchHdr *h, const ReqDesc *rq) {
+// LDS of one wave: the cloudy part's layers, the level sums and the column.
+template <int KMAX>
+__host__ __device__ constexpr int solve_lds_doubles() {
+  return kLowK * kLowQ * kWave + (3 + kHotQ) * (KMAX * kRowLanes + 1);
+}
+
+// Waves (64 threads each) of the calls of one build: W the work space.
+template <bool MIXED, int OPT, int KMAX, int W>
+__global__ __launch_bounds__(256, KMAX <= 9 ? 2 : 1) void b_solve_kernel(const BatchHdr *h, const ReqDesc *rq) {
   extern __shared__ double lds[];
   constexpr int lp = KMAX * kRowLanes + 1;
-  constexpr int per = 3 * lp + kLowK * kLowQ * kWave;
   const long long tot = h->tot[W];
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
-  double *acc = lds + wv * per, *low = acc + 3 * lp;
+  double *low = lds + wv * solve_lds_doubles<KMAX>(), *acc = low + kLowK * kLowQ * kWave, *hot = acc + 3 * lp;
   const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
   for (long long w0 = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w0 < tot; w0 += nw) {
     const int w = __builtin_amdgcn_readfirstlane((int)w0);
@@ -562,17 +667,12 @@ __global__ __launch_bounds__(256, KMAX == 6 ? SG_OCC6 : 2) void b_solve_kernel(c
     const ReqDesc &q = rq[r];
     const int wave = w - (int)q.s[W];
     if (q.d.isolir == SOCGPU_SOURCE_SOLAR)
-      solve_rows<MIXED, GEN, true, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+      solve_rows<MIXED, OPT, true, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
                                          G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                         G(q.partial), wave, lane, acc, lp, low);
+                                         G(q.partial), wave, lane, acc, lp, low, hot);
     else
-      solve_rows<MIXED, GEN, false, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+      solve_rows<MIXED, OPT, false, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
                                           G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                          G(q.partial), wave, lane, acc, lp, low);
+                                          G(q.partial), wave, lane, acc, lp, low, hot);
   }
-}
-
-template <int KMAX>
-constexpr int solve_lds(int waves) {
-  return waves * (3 * (KMAX * kRowLanes + 1) + kLowK * kLowQ * kWave) * 8;
 }
