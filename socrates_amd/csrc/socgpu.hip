@@ -1174,32 +1174,6 @@ __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm 
   if (cloudy) { o.T *= frac1; o.R *= frac1; o.T0 *= frac1; o.s1 *= frac1; o.s2 *= frac1; }
 }
 
-// The elimination update of one layer: with the layer's transmission and
-// reflection (o.T, o.R) and its upward and downward sources (su, sd), the
-// reflectance of the atmosphere above (rho) and the diffuse flux it sends
-// down (dn) move to the layer's bottom; returns the back-substitution pair
-// fu(top) = a fu(bottom) + bb. The mixed form takes 1 / (1 - R rho) from the
-// hardware reciprocal estimate and two Newton steps (a few ulp of FP64).
-template <bool MIXED>
-__device__ __forceinline__ void elim_step(const Coef &o, double su, double sd, double &rho, double &dn,
-                                          double &a, double &bb) {
-#pragma clang fp contract(on)
-  double bp;
-  if (MIXED) {
-    const double x = 1.0 - o.R * rho;
-    bp = __builtin_amdgcn_rcp(x);
-    bp = fma(bp, fma(-x, bp, 1.0), bp);
-    bp = fma(bp, fma(-x, bp, 1.0), bp);
-  } else {
-    bp = 1.0 / (1.0 - o.R * rho);
-  }
-  a = o.T * bp;
-  bb = (o.R * dn + su) * bp;
-  double rho_n = o.R + o.T * rho * a;
-  dn = o.T * (rho * bb + dn) + sd;
-  rho = rho_n;
-}
-
 // Sum of the per-wave partials, the Planck flux added back for the
 // infra-red (adjust_ir_radiance.F90:186-200, weight_band = 1), output in the
 // caller's [level][profile] layout. A column's partials come from its waves,
@@ -2044,88 +2018,7 @@ __global__ void b_heating_kernel(const BatchHdr *h, const ReqDesc *rq) {
   }
 }
 
-// Kernel-level two-stream solve on prescribed optical properties, one lane
-// per (term, profile) (profile fastest, so every per-layer read and
-// per-level write is coalesced), with the packed solve's per-layer
-// functions (two_coeff or two_coeff_f32 with coef_from_f32, elim_step):
-// two_coeff, the infra-red (ir_source.F90:
-// 93-120) or solar (solar_source.F90:104-162) sources, the surface source
-// (column_solver.F90:160-185) and the column solve (solver_homogen_direct.F90
-// :93-127 as a top-down elimination and bottom-up back-substitution).
-// Arrays [term][layer][profile] (optical properties, outputs [term][level]
-// [profile]) and [layer][profile] / [profile] for the rest.
-struct TwoStreamArgs {
-  int P, L, G, isolir, l_scale_solar, l_quad;
-  const double *tau, *omega, *asym, *sec0, *finc_down, *finc_dir, *alb_diff, *alb_dir;
-  const double *dpl, *dpl2, *dsurf, *adjust;
-  double *fdir, *fup, *fdown;
-};
-
-template <bool MIXED>
-__global__ __launch_bounds__(256) void two_stream_kernel(TwoStreamArgs a) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= a.P * a.G) return;
-  const int P = a.P, L = a.L;
-  const int l = idx % P, g = idx / P;
-  const bool solar = a.isolir == SOCGPU_SOURCE_SOLAR;
-  const double sec0 = solar ? a.sec0[l] : 1.0;
-  const size_t t0 = (size_t)g * L * P + l;
-  const size_t o0 = (size_t)g * (L + 1) * P + l;
-  double st[SG_MAXL][4];
-  double fd = solar ? a.finc_dir[l] : 0.0;
-  if (solar && a.fdir) a.fdir[o0] = fd;
-  double rho = 0.0, dn = a.finc_down[l];
-  for (int i = 0; i < L; i++) {
-    const size_t k = t0 + (size_t)i * P;
-    const size_t kl = (size_t)i * P + l;
-    const double tau = a.tau[k], om = a.omega[k], asym = a.asym[k];
-    Coef o;
-    if (MIXED) {
-      CoefF f;
-      two_coeff_f32(solar, (float)tau, (float)om, (float)fmax(1.0 - om, 32.0 * kEps), (float)asym,
-                    (float)sec0, f);
-      coef_from_f32(f, o);
-    } else {
-      two_coeff(solar, tau, om, asym, sec0, o);
-    }
-    double su, sd;
-    if (solar) {
-      if (a.l_scale_solar) {
-        double fnew = fd * o.T0 * a.adjust[kl];
-        su = o.s1 * fd;
-        sd = (o.s2 - o.T0) * fd + fnew;
-        fd = fnew;
-      } else {
-        su = o.s1 * fd;
-        sd = o.s2 * fd;
-        fd = fd * o.T0;
-      }
-      if (a.fdir) a.fdir[o0 + (size_t)(i + 1) * P] = fd;
-    } else if (a.l_quad) {
-      su = o.s1 * a.dpl[kl] + o.s2 * a.dpl2[kl];
-      sd = -o.s1 * a.dpl[kl] + o.s2 * a.dpl2[kl];
-    } else {
-      su = o.s1 * a.dpl[kl];
-      sd = -su;
-    }
-    double aa, bb;
-    const double rho0 = rho, dn0 = dn;
-    elim_step<MIXED>(o, su, sd, rho, dn, aa, bb);
-    st[i][0] = aa; st[i][1] = bb; st[i][2] = rho0; st[i][3] = dn0;
-  }
-  const double ad = a.alb_diff[l];
-  const double sg = solar ? (a.alb_dir[l] - ad) * fd : (1.0 - ad) * a.dsurf[l];
-  double fu = (ad * dn + sg) / (1.0 - ad * rho);
-  double fdn = rho * fu + dn;
-  a.fup[o0 + (size_t)L * P] = fu;
-  a.fdown[o0 + (size_t)L * P] = fdn;
-  for (int i = L - 1; i >= 0; i--) {
-    fu = st[i][0] * fu + st[i][1];
-    fdn = st[i][2] * fu + st[i][3];
-    a.fup[o0 + (size_t)i * P] = fu;
-    a.fdown[o0 + (size_t)i * P] = fdn;
-  }
-}
+#include "two_stream_split.h"
 
 // ---------------------------------------------------------------- host side
 // Device and pinned host buffers grow by at least half their size when they
@@ -3758,10 +3651,10 @@ int socgpu_two_stream(int n_profile, int n_layer, int n_term, int isolir, int l_
     a.fup = ob; a.fdown = ob + nout; a.fdir = flux_direct ? ob + 2 * nout : nullptr;
   }
   if (!solar) a.fdir = nullptr;
-  const int threads = 256, blocks = (int)(((size_t)P * G + threads - 1) / threads);
   HIPCHK(hipEventRecord(g_ctx.ev1, s));
-  if (precision == SOCGPU_MIXED) two_stream_kernel<true><<<blocks, threads, 0, s>>>(a);
-  else two_stream_kernel<false><<<blocks, threads, 0, s>>>(a);
+  const bool mixed = precision == SOCGPU_MIXED;
+  if (solar) mixed ? two_stream_launch<true, true>(a, s) : two_stream_launch<false, true>(a, s);
+  else mixed ? two_stream_launch<true, false>(a, s) : two_stream_launch<false, false>(a, s);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(g_ctx.ev2, s));
   if (!l_on_device) {

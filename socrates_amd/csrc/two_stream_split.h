@@ -1,0 +1,165 @@
+// The kernel-level two-stream solve on prescribed optical properties: included
+// by socgpu.hip after solve_rows.h, whose slab composition it uses.
+#pragma once
+
+// Arrays [term][layer][profile] (optical properties, outputs [term][level]
+// [profile]) and [layer][profile] / [profile] for the rest.
+struct TwoStreamArgs {
+  int P, L, G, isolir, l_scale_solar, l_quad;
+  const double *tau, *omega, *asym, *sec0, *finc_down, *finc_dir, *alb_diff, *alb_dir;
+  const double *dpl, *dpl2, *dsurf, *adjust;
+  double *fdir, *fup, *fdown;
+};
+
+// One lane per (term, profile), profile fastest, so every per-layer read and
+// per-level write is coalesced; the layers of 64 such solves are split over the
+// kTsWaves waves of a block, at most KMAX consecutive ones each, whose state
+// stays in registers. Each wave composes its layers into one slab; the slabs
+// pass through LDS, every wave eliminates down those above its own to find the
+// state at its top, and after the local elimination the affine maps of the
+// waves below pass the upward flux back the same way. With the whole column in
+// one lane the elimination state went through lane-private memory (64 B a layer
+// beside the 48 B the solve has to move) and a small call was one chain of all
+// its layers.
+// (two_coeff, ir_source.F90:93-120, solar_source.F90:104-162, the surface source
+// of column_solver.F90:160-185, solver_homogen_direct.F90:93-127.)
+constexpr int kTsWaves = 16;
+
+template <bool MIXED, bool SOLAR, int KMAX>
+__global__ __launch_bounds__(kTsWaves *kWave) void two_stream_kernel(TwoStreamArgs a) {
+#pragma clang fp contract(on)
+  constexpr int kQ = 6;
+  __shared__ double sh[kTsWaves][kQ][kWave];
+  const int lane = threadIdx.x % kWave;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int P = a.P, L = a.L;
+  const long long n = (long long)P * a.G, idx = (long long)blockIdx.x * kWave + lane;
+  const bool act = idx < n;
+  // lanes past the last solve repeat it and store nothing
+  const long long id = act ? idx : n - 1;
+  const int g = (int)(id / P), l = (int)(id - (long long)g * P);
+  const int K = (L + kTsWaves - 1) / kTsWaves, i0 = wv * K, nk = max(0, min(K, L - i0));
+  const int n_wave = (L + K - 1) / K;   // waves with layers
+  const double sec0 = SOLAR ? a.sec0[l] : 1.0;
+  const size_t t0 = (size_t)g * L * P + l, o0 = (size_t)g * (L + 1) * P + l;
+  const double finc_down = a.finc_down[l], finc_dir = SOLAR ? a.finc_dir[l] : 0.0;
+
+  double w0[KMAX], w1[KMAX], w2[KMAX], w3[KMAX], wf[SOLAR ? KMAX : 1];
+  Slab S{1.0, 0.0, 0.0, 0.0, 0.0};
+  double f = 1.0;   // the direct beam relative to the wave's top
+#pragma unroll
+  for (int k = 0; k < KMAX; k++) {
+    if (k < nk) {
+      const size_t kk = t0 + (size_t)(i0 + k) * P, kl = (size_t)(i0 + k) * P + l;
+      const double tau = a.tau[kk], om = a.omega[kk], asym = a.asym[kk];
+      Coef o;
+      if (MIXED) {
+        CoefF c;
+        two_coeff_f32(SOLAR, (float)tau, (float)om, (float)fmax(1.0 - om, 32.0 * kEps), (float)asym, (float)sec0, c);
+        coef_from_f32(c, o);
+      } else {
+        two_coeff(SOLAR, tau, om, asym, sec0, o);
+      }
+      double su, sd;
+      if (SOLAR) {
+        wf[k] = f;
+        su = o.s1 * f;
+        if (a.l_scale_solar) {
+          const double fnew = f * o.T0 * a.adjust[kl];
+          sd = (o.s2 - o.T0) * f + fnew;
+          f = fnew;
+        } else {
+          sd = o.s2 * f;
+          f = f * o.T0;
+        }
+      } else if (a.l_quad) {
+        su = o.s1 * a.dpl[kl] + o.s2 * a.dpl2[kl];
+        sd = -o.s1 * a.dpl[kl] + o.s2 * a.dpl2[kl];
+      } else {
+        su = o.s1 * a.dpl[kl];
+        sd = -su;
+      }
+      w0[k] = o.T;
+      w1[k] = o.R;
+      w2[k] = su;
+      w3[k] = sd;
+      const Slab B{o.T, o.R, o.R, su, sd};
+      S = k == 0 ? B : slab_add(S, B);
+    }
+  }
+  sh[wv][0][lane] = S.T;
+  sh[wv][1][lane] = S.Rt;
+  sh[wv][2][lane] = S.Rb;
+  sh[wv][3][lane] = S.Su;
+  sh[wv][4][lane] = S.Sd;
+  if (SOLAR) sh[wv][5][lane] = f;
+  __syncthreads();
+  // down the slabs above
+  double rho = 0.0, dn = finc_down, F = finc_dir;
+  for (int u = 0; u < wv && u < n_wave; u++) {
+    Slab B{sh[u][0][lane], sh[u][1][lane], sh[u][2][lane], sh[u][3][lane], sh[u][4][lane]};
+    if (SOLAR) { B.Su = B.Su * F; B.Sd = B.Sd * F; }
+    double rb, sd;
+    slab_below(rho, dn, B, rb, sd);
+    rho = rb;
+    dn = sd;
+    if (SOLAR) F = F * sh[u][5][lane];
+  }
+  __syncthreads();
+  double A = 1.0, C = 0.0;   // fu(top of the wave) = A fu(bottom) + C
+#pragma unroll
+  for (int k = 0; k < KMAX; k++) {
+    if (k < nk) {
+      const double T = w0[k], R = w1[k];
+      double su = w2[k], sd = w3[k];
+      if (SOLAR) {
+        su = su * F;
+        sd = sd * F;
+        if (act && a.fdir) a.fdir[o0 + (size_t)(i0 + k) * P] = wf[k] * F;
+      }
+      w2[k] = rho;
+      w3[k] = dn;
+      row_elim(T, R, su, sd, rho, dn, w0[k], w1[k]);
+      C = C + A * w1[k];
+      A = A * w0[k];
+    }
+  }
+  const bool bottom = wv == n_wave - 1;
+  sh[wv][0][lane] = A;
+  sh[wv][1][lane] = C;
+  if (bottom) {
+    const double ad = a.alb_diff[l], fd = F * f;
+    const double sg = SOLAR ? (a.alb_dir[l] - ad) * fd : (1.0 - ad) * a.dsurf[l];
+    const double fu = (ad * dn + sg) / (1.0 - ad * rho);
+    sh[wv][2][lane] = fu;
+    if (act) {
+      a.fup[o0 + (size_t)L * P] = fu;
+      a.fdown[o0 + (size_t)L * P] = rho * fu + dn;
+      if (SOLAR && a.fdir) a.fdir[o0 + (size_t)L * P] = fd;
+    }
+  }
+  __syncthreads();
+  // up from the surface through the waves below
+  double fu = sh[n_wave - 1][2][lane];
+  for (int u = n_wave - 1; u > wv; u--) fu = sh[u][0][lane] * fu + sh[u][1][lane];
+#pragma unroll
+  for (int k = KMAX - 1; k >= 0; k--) {
+    if (k < nk) {
+      fu = w0[k] * fu + w1[k];
+      if (act) {
+        a.fup[o0 + (size_t)(i0 + k) * P] = fu;
+        a.fdown[o0 + (size_t)(i0 + k) * P] = w2[k] * fu + w3[k];
+      }
+    }
+  }
+}
+
+template <bool MIXED, bool SOLAR>
+static void two_stream_launch(const TwoStreamArgs &a, hipStream_t s) {
+  const long long n = (long long)a.P * a.G;
+  const int blocks = (int)((n + kWave - 1) / kWave), T = kTsWaves * kWave;
+  if (a.L <= 3 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 3><<<blocks, T, 0, s>>>(a);
+  else if (a.L <= 6 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 6><<<blocks, T, 0, s>>>(a);
+  else if (a.L <= 9 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 9><<<blocks, T, 0, s>>>(a);
+  else two_stream_kernel<MIXED, SOLAR, 12><<<blocks, T, 0, s>>>(a);
+}

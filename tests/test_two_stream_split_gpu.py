@@ -1,0 +1,26 @@
+"""The kernel-level two-stream solve's split of a column over 16 waves (3, 6, 9
+or 12 layers each by build) at the sizes where it changes, with solve counts
+that do not fill the last wave, against the oracle with the tolerance of
+test_two_stream_gpu (1e-10 relative, 1e-9 W m-2 or 1e-11 of the column's scale,
+plus the oracle's own spread in the infra-red)."""
+import numpy as np
+import pytest
+
+from socrates_amd import runes as R
+from socrates_amd import synth
+from test_two_stream_gpu import _check, _oracle_terms, _spread
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("isolir", [1, 2])
+@pytest.mark.parametrize("shape", [(1, 2, 1), (13, 16, 7), (64, 17, 1), (13, 48, 5), (13, 49, 5), (3, 96, 3),
+                                   (3, 97, 22), (5, 144, 2), (5, 145, 2), (7, 192, 3)])
+def test_split_sizes_match_oracle(isolir, shape):
+    P, L, G = shape
+    tsc = synth.make_two_stream_case(P, L, isolir, seed=70 + L + isolir, n_term=G, omc_range=(-3.0, 0.0))
+    ref = _oracle_terms(tsc)
+    gpu = R.two_stream_case(tsc, "fp64")
+    _check(gpu, ref, _spread(tsc, ref) if isolir == 2 else None, "fp64 isolir=%d %s" % (isolir, shape))
+    if isolir == 1:
+        assert np.abs(np.asarray(gpu["flux_direct"]) - ref[2]).max() <= 1e-10 * np.abs(ref[2]).max()
