@@ -35,6 +35,40 @@ SG_HD T *G(T *p) {
 #endif
 }
 
+// A value of the device tables at an address that is the same for the whole
+// wave, read through the constant address space: a scalar load. (Read through a
+// global pointer after the kernel has stored anything it becomes a vector load
+// of one address, since the compiler cannot tell that the tables never change.)
+template <class T>
+SG_HD T U(const T &x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const __attribute__((address_space(4))) T *)(unsigned long long)&x;
+#else
+  return x;
+#endif
+}
+
+// The same for a struct of 4-byte words' multiple (a call's descriptor).
+template <class T>
+SG_HD T U_struct(const T &x) {
+  static_assert(sizeof(T) % 4 == 0, "copied in words");
+  struct Words { unsigned w[sizeof(T) / 4]; } v;
+  const unsigned *p = (const unsigned *)&x;
+#pragma unroll
+  for (unsigned j = 0; j < sizeof(T) / 4; j++) v.w[j] = U(p[j]);
+  return __builtin_bit_cast(T, v);
+}
+
+// A k-term of the tables, the same for the whole wave.
+SG_HD SgTerm U_term(const SgTerm &t) {
+  SgTerm o;
+  o.k = U(t.k); o.w = U(t.w); o.a = U(t.a); o.b = U(t.b); o.c = U(t.c);
+  o.lnpref = U(t.lnpref); o.lntref = U(t.lntref); o.tinv = U(t.tinv);
+  o.band = U(t.band); o.gas = U(t.gas); o.n_sub = 0; o.sub0 = 0;
+  o.fnc = U(t.fnc); o.lut = U(t.lut); o.iscat = U(t.iscat);
+  return o;
+}
+
 constexpr double kElsasser = 1.66;       // diffusivity_factor.F90: elsasser_factor
 constexpr double kDiffMinor = 1.66;      // diffusivity_factor_minor
 constexpr double kEps = DBL_EPSILON;
@@ -124,12 +158,27 @@ SG_HD void two_coeff_absorb(double tau, bool nosc, double &T, double &s1, double
   s2 = -(tau > tol ? 1.0 + T - 2.0 * s1 : thin) / den;
 }
 
-// Horner evaluation of the band Planck polynomial (planck_flux_band_mod.F90:33-49)
-SG_HD double planck_band(const SgBand &b, int n_deg, double t_ref, double temp) {
+// The band's Planck polynomial (planck_flux_band_mod.F90:33-49, Horner) for a
+// whole wave: its coefficients by scalar loads, once.
+struct PlanckBand {
+  double c[SG_NPL], t_ref;
+  int n_deg;
+};
+SG_HD PlanckBand planck_coef(const SgSpec *spec, const SgBand &b) {
+  PlanckBand p;
+  p.n_deg = U(spec->n_deg);
+  p.t_ref = U(spec->t_ref_planck);
+  for (int j = 0; j < SG_NPL; j++) p.c[j] = U(b.planck[j]);
+  return p;
+}
+SG_HD double planck_band(const PlanckBand &b, double temp) {
 #pragma clang fp contract(off)
-  double x = temp / t_ref;
-  double v = b.planck[n_deg];
-  for (int j = n_deg - 1; j >= 0; j--) v = v * x + b.planck[j];
+  const double x = temp / b.t_ref;
+  double v = b.c[SG_NPL - 1];
+  for (int j = SG_NPL - 2; j >= 0; j--) {
+    if (j == b.n_deg) v = b.c[j];
+    else if (j < b.n_deg) v = v * x + b.c[j];
+  }
   return v;
 }
 
@@ -160,8 +209,8 @@ SG_HD double k_scaled(const SgTerm &t, const SgSpec *spec, double lnp, double p,
 #pragma clang fp contract(off)
   if (t.fnc == SG_FNC_LOOKUP) {
     const int idx = (int)g[SG_G_IDX];
-    const int jp = idx & 255, jt = (idx >> 8) & 255, jtt = idx >> 16, nt = spec->n_tmp;
-    const double *kl = G(spec->klut) + (size_t)t.lut * spec->n_pre * nt;
+    const int jp = idx & 255, jt = (idx >> 8) & 255, jtt = idx >> 16, nt = U(spec->n_tmp);
+    const double *kl = G(U(spec->klut)) + (size_t)t.lut * U(spec->n_pre) * nt;
     const double ke = fmax(0.0, g[SG_G_F00] * kl[jp * nt + jt] + g[SG_G_F10] * kl[(jp + 1) * nt + jtt] +
                                     g[SG_G_F01] * kl[jp * nt + jt + 1] +
                                     g[SG_G_F11] * kl[(jp + 1) * nt + jtt + 1]);
@@ -172,7 +221,7 @@ SG_HD double k_scaled(const SgTerm &t, const SgSpec *spec, double lnp, double p,
     const double x = tk * t.tinv - 1.0;
     s = exp(t.a * (lnp - t.lnpref)) * (1.0 + x * t.b + t.c * x * x);
   } else {  // SG_FNC_WENYI
-    const double *gk4 = G(spec->wenyi), *gk250b = gk4 + 3640, *plg = gk250b + 14, *ttb = plg + 26;
+    const double *gk4 = G(U(spec->wenyi)), *gk250b = gk4 + 3640, *plg = gk250b + 14, *ttb = plg + 26;
     const double cgp = fmax(-5.5, log(p / 100.0));
     int jp = (int)((5.5 + cgp) * 2.0) + 1;
     jp = jp < 1 ? 1 : (jp > 26 ? 26 : jp);
@@ -201,19 +250,20 @@ SG_HD double continuum_k(const SgBand &B, double p, double tk, double rho, doubl
 #pragma clang fp contract(off)
   const double mol_weight_air = 28.966e-03, repsilon = 18.0153 / 28.966;
   double kg = 0.0;
-  for (int j = 0; j < B.n_cont; j++) {
-    const double *sc = B.cont_s[j];
-    const double pwk = pow(p / B.cont_pref[j], sc[0]);
+  const int n = U(B.n_cont);
+  for (int j = 0; j < n; j++) {
+    const double s0 = U(B.cont_s[j][0]), s1 = U(B.cont_s[j][1]), tref = U(B.cont_tref[j]);
+    const double pwk = pow(p / U(B.cont_pref[j]), s0);
     double amount;
-    if (B.cont_fnc[j] == SG_FNC_POWER_LAW) {
-      amount = pwk * pow(tk / B.cont_tref[j], sc[1]);
+    if (U(B.cont_fnc[j]) == SG_FNC_POWER_LAW) {
+      amount = pwk * pow(tk / tref, s1);
     } else {
-      const double x = tk / B.cont_tref[j] - 1.0;
-      amount = pwk * (1.0 + sc[1] * x + sc[2] * (x * x));
+      const double x = tk / tref - 1.0;
+      amount = pwk * (1.0 + s1 * x + U(B.cont_s[j][2]) * (x * x));
     }
-    if (B.cont_type[j] == 1) amount = amount * (rho * h2o / (repsilon * mol_weight_air)) * h2o;
+    if (U(B.cont_type[j]) == 1) amount = amount * (rho * h2o / (repsilon * mol_weight_air)) * h2o;
     else amount = amount * rho * h2o * (1.0 - h2o) / mol_weight_air;
-    kg = kg + B.cont_k[j] * amount;
+    kg = kg + U(B.cont_k[j]) * amount;
   }
   return kg;
 }
@@ -280,11 +330,14 @@ SG_HD void slingo(const double *cp, double mmr, double re, double &kext, double 
   fwd = kscat * (g * g);
 }
 
-// Droplet optics by the type's scheme (5 Pade-2, 1 Slingo-Schrecker).
+// Droplet optics by the type's scheme (5 Pade-2, 1 Slingo-Schrecker); type and
+// band are the same for the whole wave.
 SG_HD void drop_optics(const SgDrop &dr, int b, double mmr, double re, double &kext, double &kscat,
                        double &phf, double &fwd) {
-  if (dr.scheme == 5) pade2(dr.parm[b], mmr, re, kext, kscat, phf, fwd);
-  else slingo(dr.parm[b], mmr, re, kext, kscat, phf, fwd);
+  double cp[SG_NDPARM];
+  for (int j = 0; j < SG_NDPARM; j++) cp[j] = U(dr.parm[b][j]);
+  if (U(dr.scheme) == 5) pade2(cp, mmr, re, kext, kscat, phf, fwd);
+  else slingo(cp, mmr, re, kext, kscat, phf, fwd);
 }
 
 // Ice optics of the two-stream case of opt_prop_ice_cloud.F90:227-256 (one
@@ -296,8 +349,10 @@ SG_HD void drop_optics(const SgDrop &dr, int b, double mmr, double re, double &k
 SG_HD void ice_optics(const SgDrop &ic, int b, double iwc, double de, double t, double &kext,
                       double &kscat, double &phf, double &fwd) {
 #pragma clang fp contract(off)
-  const double *cp = ic.parm[b];
-  if (ic.scheme == 12) {
+  double cp[SG_NDPARM];
+  for (int j = 0; j < SG_NDPARM; j++) cp[j] = U(ic.parm[b][j]);
+  const int scheme = U(ic.scheme);
+  if (scheme == 12) {
     double x = cp[3] / de;
     kext = iwc * ((cp[2] * x + cp[1]) * x + cp[0]);
     x = de / cp[8];
@@ -306,7 +361,7 @@ SG_HD void ice_optics(const SgDrop &ic, int b, double iwc, double de, double t, 
     const double g = cp[9] + x * (cp[10] + x * (cp[11] + x * cp[12]));
     phf = kscat * g;
     fwd = phf * g;
-  } else if (ic.scheme == 19) {
+  } else if (scheme == 19) {
     double x = fmin(iwc + 1.0e-12, 1.0e-01);
     kext = cp[0] * x / (t * t * t * t);
     x = fmin(iwc + 1.0e-12, 1.0e-03 - kEps);

@@ -92,13 +92,6 @@ __device__ __forceinline__ double dpp_move(double v) {
   return mk64((unsigned)lo, (unsigned)hi);
 }
 
-// The value of lane 63 in every lane, and the value of the lane below
-// (wave_shr:1; lane 0 gets 0).
-__device__ __forceinline__ double lane63(double v) {
-  return mk64((unsigned)__builtin_amdgcn_readlane((int)lo32(v), 63),
-              (unsigned)__builtin_amdgcn_readlane((int)hi32(v), 63));
-}
-
 // Sum over each group of 8 lanes, in every lane of the group.
 __device__ __forceinline__ double sum8(double x) {
   x = x + dpp_move<0x141>(x);  // row_half_mirror
@@ -106,8 +99,6 @@ __device__ __forceinline__ double sum8(double x) {
   x = x + dpp_move<0xB1>(x);   // quad_perm [1, 0, 3, 2]
   return x;
 }
-
-__device__ __forceinline__ double lane_below(double v) { return dpp_move<0x138>(v); }
 
 // Butterfly reduce-scatter of 8 values per lane over the 64 lanes of a wave: lanes 8j..8j+7 (j = 0..7) hold the total of
 // value j.
@@ -511,7 +502,6 @@ __device__ __forceinline__ void cloudgen_body(const CallDims &d, const double *_
   }
 }
 
-// Wave-wide inclusive scans over the 64 lanes (lane order = scan order).
 // A double moved across lanes by DPP (both 32-bit halves with the same
 // control): row_shr:n (CTRL 0x110 + n) within rows of 16, row_bcast:15
 // (0x142) and row_bcast:31 (0x143) across rows. Lanes with no source lane,
@@ -522,398 +512,6 @@ __device__ __forceinline__ double dpp_f64(double v, double id) {
   const int lo = __builtin_amdgcn_update_dpp((int)ib, (int)vb, CTRL, ROWMASK, 0xf, false);
   const int hi = __builtin_amdgcn_update_dpp((int)(ib >> 32), (int)(vb >> 32), CTRL, ROWMASK, 0xf, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// Inclusive product scan over the 64 lanes (lane j ends with x_0 ... x_j):
-// shifts by 1, 2, 4 and 8 within each row of 16, then the last lane of row 0
-// (and of row 2) into rows 1 (and 3), then lane 31 into rows 2 and 3. DPP
-// moves are register operations, unlike the LDS-routed shuffles.
-__device__ __forceinline__ double scan_mul(double x, int lane) {
-  (void)lane;
-  x = x * dpp_f64<0x111, 0xf>(x, 1.0);
-  x = x * dpp_f64<0x112, 0xf>(x, 1.0);
-  x = x * dpp_f64<0x114, 0xf>(x, 1.0);
-  x = x * dpp_f64<0x118, 0xf>(x, 1.0);
-  x = x * dpp_f64<0x142, 0xa>(x, 1.0);
-  x = x * dpp_f64<0x143, 0xc>(x, 1.0);
-  return x;
-}
-
-// One step of the affine scan: the maps of lower lanes (A0, C0; identity
-// (1, 0) where there is none) applied before the lane's own.
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ void affine_step(double &A, double &C) {
-  const double A0 = dpp_f64<CTRL, ROWMASK>(A, 1.0), C0 = dpp_f64<CTRL, ROWMASK>(C, 0.0);
-  C = A * C0 + C;
-  A = A * A0;
-}
-
-// Composition of affine maps F -> A F + C in lane order: lane j ends with
-// the map of lanes 0..j applied in turn (the steps of scan_mul).
-__device__ __forceinline__ void scan_affine(double &A, double &C, int lane) {
-  (void)lane;
-  affine_step<0x111, 0xf>(A, C);
-  affine_step<0x112, 0xf>(A, C);
-  affine_step<0x114, 0xf>(A, C);
-  affine_step<0x118, 0xf>(A, C);
-  affine_step<0x142, 0xa>(A, C);
-  affine_step<0x143, 0xc>(A, C);
-}
-
-// One wave per (column, band), lanes over layers (64 at a time, at most
-// NCH chunks, with carries between them): the equivalent extinction of the
-// band's minor gases (solve_band_k_eqv_scl.F90:572-1047), then the band's
-// per-layer records (prep_layer). The band's gases and their k-terms in
-// turn:
-//  - solar: each term's direct-beam transmission down the column (a wave
-//    product scan, :654-739); k_eqv = sum_k k T_k(surface) / sum_k
-//    T_k(surface) per gas (:826-846), and adjust_solar_ke from the per-layer
-//    ratios of the summed transmissions (:848-891);
-//  - infra-red: each term's non-scattering fluxes (monochromatic_gas_flux.F90:
-//    115-196, diffusivity 1.66) as two affine recurrences solved by wave
-//    scans; k_eqv = sum k |F| / sum |F| over the layer's two levels
-//    (:995-1019);
-//  - where the weighting flux vanishes, the smallest k of the gas's terms.
-// Per lane, the layer records and (infra-red) the band's Planck fluxes at
-// the layer's levels are read or evaluated once for all terms and for the
-// records. The scans associate the products differently from the
-// reference's left-to-right sweeps (relative differences of order 1e-16).
-// NCH: chunks of 64 layers the lane arrays hold (kernels for NCH = 2 and 3
-// each take the calls with that many chunks, so a call of at most 128
-// layers runs with the smaller register footprint).
-constexpr int kMinorWaves = 4;
-constexpr int kKeqMaxChunks = (SG_MAXL + kWave - 1) / kWave;
-
-template <int kKeqChunks, bool GEN>
-__device__ __forceinline__ void band_body(const CallDims &d, const SgSpec *__restrict__ spec,
-                                          int l_rayleigh, const double *__restrict__ colrec,
-                                          const double *__restrict__ grec, const double *__restrict__ wm,
-                                          const double *const *gfield, const double *__restrict__ tlev,
-                                          const double *__restrict__ colscal,
-                                          double *__restrict__ bandrec,
-                                          double *__restrict__ bandscal,
-                                          double *__restrict__ cldopt, const int *__restrict__ krange,
-                                          const AerIn &ae, int wave, int lane) {
-  const int L = d.L, NB = d.NB;
-  if (wave >= d.P * NB) return;
-  const int col = wave / NB, b = wave % NB;
-  const SgBand &B = spec->band[b];
-  const double *rec = colrec + (size_t)col * L * SG_NQ;
-  const int nch = (L + kWave - 1) / kWave;
-  const bool solar = d.isolir == SOCGPU_SOURCE_SOLAR;
-  double lnp[kKeqChunks], lnt[kKeqChunks], mass[kKeqChunks], b0[kKeqChunks], b1[kKeqChunks];
-  double keq[kKeqChunks], adj[kKeqChunks], kgrey[kKeqChunks];
-  const double *tl = tlev + (size_t)col * (L + 1);
-#pragma unroll
-  for (int c = 0; c < kKeqChunks; c++) {
-    const int i = c * kWave + lane;
-    lnp[c] = 0.0; lnt[c] = 0.0; mass[c] = 0.0; b0[c] = 0.0; b1[c] = 0.0;
-    keq[c] = 0.0; adj[c] = 1.0; kgrey[c] = 0.0;
-    if (c < nch && i < L) {
-      const double *r = rec + (size_t)i * SG_NQ;
-      lnp[c] = r[SG_Q_LNP]; lnt[c] = r[SG_Q_LNT]; mass[c] = r[SG_Q_MASS];
-      if (!solar) {
-        b0[c] = planck_band(B, spec->n_deg, spec->t_ref_planck, tl[i]);
-        b1[c] = planck_band(B, spec->n_deg, spec->t_ref_planck, tl[i + 1]);
-      }
-    }
-  }
-  const double sec0 = colscal[(size_t)col * SG_NS + SG_S_SEC0];
-  const double alb = bandscal[((size_t)col * d.NB + b) * SG_NBQ + 2];
-  double b_top = 0.0, b_bot = 0.0, bg = 0.0;
-  if (!solar) {
-    b_top = planck_band(B, spec->n_deg, spec->t_ref_planck, tl[0]);
-    b_bot = planck_band(B, spec->n_deg, spec->t_ref_planck, tl[L]);
-    bg = colscal[(size_t)col * SG_NS + SG_S_LFG] != 0.0
-             ? bandscal[((size_t)col * d.NB + b) * SG_NBQ + 1]
-             : planck_band(B, spec->n_deg, spec->t_ref_planck, colscal[(size_t)col * SG_NS + SG_S_TGROUND]);
-  }
-  const double sqe = 1.4901161193847656e-08;
-  int t0 = B.minor0;
-  for (int j = 0; j < B.n_minor_gas; j++) {
-    const int nk = B.minor_nk[j];
-    const int gas = spec->minor[t0].gas;
-    double mmr[kKeqChunks], num[kKeqChunks], den[kKeqChunks], kmin[kKeqChunks];
-#pragma unroll
-    for (int c = 0; c < kKeqChunks; c++) {
-      const int i = c * kWave + lane;
-      // further gases (general gas optics): the call's field, clamped at
-      // 0, else its well-mixed ratio (socrates_set_atm.F90:535-622)
-      const double *fld = (GEN && gas >= SG_GAS_WM0) ? G(gfield[gas - SG_GAS_WM0]) : nullptr;
-      mmr[c] = (c < nch && i < L) ? ((!GEN || gas < SG_GAS_WM0) ? rec[(size_t)i * SG_NQ + SG_Q_MMR + gas]
-                                     : fld ? fmax(fld[(size_t)i * d.P + col], 0.0)
-                                           : wm[gas - SG_GAS_WM0])
-                                  : 0.0;
-      num[c] = 0.0; den[c] = 0.0; kmin[c] = DBL_MAX;
-    }
-    double sflux = 0.0;
-    for (int q = 0; q < nk; q++) {
-      const SgTerm &t = spec->minor[t0 + q];
-      double kk[kKeqChunks];
-#pragma unroll
-      for (int c = 0; c < kKeqChunks; c++) {
-        const int i = c * kWave + lane;
-        if (c < nch && i < L) {
-          if (!GEN || t.fnc == SG_FNC_POWER_LAW) kk[c] = k_term(t, lnp[c], lnt[c], mmr[c]);
-          else {
-            const double *r = rec + (size_t)i * SG_NQ;
-            kk[c] = k_scaled(t, spec, lnp[c], r[SG_Q_P], r[SG_Q_T],
-                             grec ? grec + ((size_t)col * L + i) * SG_NGQ : nullptr, mmr[c]);
-          }
-        } else {
-          kk[c] = 0.0;
-        }
-        kmin[c] = fmin(kmin[c], kk[c]);
-      }
-      if (d.grey1 && nk == 1) {
-        // a single k-term with l_grey_single: its absorption joins the grey
-        // extinction as it is (solve_band_k_eqv_scl.F90:941-951)
-#pragma unroll
-        for (int c = 0; c < kKeqChunks; c++) kgrey[c] = kgrey[c] + kk[c];
-        continue;
-      }
-      if (solar) {
-        // direct-beam transmission: f = w prod exp(-k m sec0) down to the
-        // bottom of each layer; den accumulates f (summed over terms, fg)
-        double fdt = t.w, f[kKeqChunks];
-#pragma unroll
-        for (int c = 0; c < kKeqChunks; c++) {
-          f[c] = 0.0;
-          if (c < nch) {
-            const int i = c * kWave + lane;
-            const double x = i < L ? exp(-kk[c] * mass[c] * sec0) : 1.0;
-            f[c] = fdt * scan_mul(x, lane);
-            fdt = lane63(f[c]);
-          }
-        }
-        // lanes below layer L-1 carry the identity, so fdt is now the
-        // transmission to the surface (the value at layer L-1)
-        const double fs = fdt;
-#pragma unroll
-        for (int c = 0; c < kKeqChunks; c++) {
-          num[c] = num[c] + kk[c] * fs;
-          den[c] = den[c] + f[c];
-        }
-        sflux = sflux + fs;
-      } else {
-        // downward differential flux F at the top of each layer
-        double F = -b_top, tr[kKeqChunks], su[kKeqChunks], fdl[kKeqChunks];
-#pragma unroll
-        for (int c = 0; c < kKeqChunks; c++) {
-          tr[c] = 1.0; su[c] = 0.0; fdl[c] = 0.0;
-          if (c < nch) {
-            const int i = c * kWave + lane;
-            double A = 1.0, C = 0.0;
-            if (i < L) {
-              const double tau = kk[c] * mass[c];
-              tr[c] = exp(-kDiffMinor * tau);
-              su[c] = (1.0 - tr[c] + sqe) * (b1[c] - b0[c]) / (kDiffMinor * tau + sqe);
-              A = tr[c];
-              C = -su[c];
-            }
-            scan_affine(A, C, lane);
-            const double below = A * F + C;
-            double above = lane_below(below);
-            if (lane == 0) above = F;
-            fdl[c] = above;
-            F = lane63(below);
-          }
-        }
-        // lanes below layer L-1 carry the identity, so F is the downward
-        // flux at the surface
-        double U = (bg - b_bot) + alb * F;   // upward flux at the surface
-#pragma unroll
-        for (int cc = kKeqChunks - 1; cc >= 0; cc--) {
-          if (cc < nch) {
-            // bottom-up over this chunk: lane with layer i = cc*64 + lane,
-            // scanned in reverse lane order
-            const int rl = kWave - 1 - lane;     // reverse position
-            const int i = cc * kWave + rl;
-            double A = 1.0, C = 0.0;
-            const double trr = __shfl(tr[cc], rl, kWave), sur = __shfl(su[cc], rl, kWave);
-            if (i < L) { A = trr; C = sur; }
-            scan_affine(A, C, lane);
-            const double above = A * U + C;                  // F up at the top of layer i
-            double belowu = lane_below(above);                // at its bottom
-            if (lane == 0) belowu = U;
-            // back to natural lane order: lane l holds layer cc*64 + l
-            const double bl = __shfl(belowu, rl, kWave);
-            const int il = cc * kWave + lane;
-            if (il < L) {
-              const double a = t.w * fabs(fdl[cc]), bb = t.w * fabs(bl);
-              num[cc] = num[cc] + (kk[cc] * a + kk[cc] * bb);
-              den[cc] = den[cc] + (a + bb);
-            }
-            U = lane63(above);
-          }
-        }
-      }
-    }
-    // this gas's equivalent extinction and (solar) direct-beam adjustment
-    if (!(d.grey1 && nk == 1)) {
-#pragma unroll
-    for (int c = 0; c < kKeqChunks; c++) {
-      if (c < nch) {
-        const int i = c * kWave + lane;
-        double kq;
-        if (solar) {
-          kq = sflux > 0.0 ? num[c] / sflux : kmin[c];
-          // flux_gas at the top of layer i: the summed transmission one layer
-          // up (1 above the first layer)
-          double fgp = lane_below(den[c]);
-          const double carry = lane63(den[c > 0 ? c - 1 : 0]);
-          if (lane == 0) fgp = c > 0 ? carry : 1.0;
-          if (i == 0) fgp = 1.0;
-          if (i < L && fgp > 0.0) adj[c] = adj[c] * den[c] / fgp;
-        } else {
-          kq = den[c] > 0.0 ? num[c] / den[c] : kmin[c];
-        }
-        if (i < L) keq[c] = keq[c] + kq;
-      }
-    }
-    }
-    t0 += nk;
-  }
-#pragma unroll
-  for (int c = 0; c < kKeqChunks; c++) {
-    const int i = c * kWave + lane;
-    if (c < nch && i < L)
-      prep_layer(d, spec, l_rayleigh, colrec, grec, colscal, bandrec, bandscal, cldopt, krange, ae, col, b, i,
-                 keq[c], kgrey[c], adj[c], b0[c], b1[c], GEN);
-  }
-}
-
-// Per (column, band, layer), given the layer's equivalent extinction and
-// direct-beam adjustment product: the grey extinction (Rayleigh,
-// grey_opt_prop.F90:476-541, 816-835, plus k_eqv), the solar direct-beam
-// adjustment with the exponential of the equivalent optical depth
-// (solve_band_k_eqv_scl.F90:848-891), the Planck source terms
-// (diff_planck_source_mod.F90:100-134) and the cloud optics.
-// bandrec[col][band][layer][4].
-__device__ __forceinline__ void prep_layer(const CallDims &d, const SgSpec *__restrict__ spec,
-                                           int l_rayleigh, const double *__restrict__ colrec,
-                                           const double *__restrict__ grec,
-                                           const double *__restrict__ colscal,
-                                           double *__restrict__ bandrec,
-                                           double *__restrict__ bandscal,
-                                           double *__restrict__ cldopt, const int *__restrict__ krange,
-                                           const AerIn &ae, int col, int b, int i, double keq, double kgrey,
-                                           double adjust, double b0, double b1, bool gen) {
-  const int NB = d.NB, L = d.L;
-  const SgBand &B = spec->band[b];
-  const double *rec = colrec + (size_t)col * L * SG_NQ;
-  const double *r = rec + i * SG_NQ;
-  if (d.mcica) {
-    // droplet optics of the layer's in-cloud water at unit condensate
-    // scaling (they depend on the band, not on the k-term; the solve scales
-    // them by each sub-column's c_sub)
-    // (written only where the layer has cloud: the solve reads them only
-    // for cloudy layers of a sub-column)
-    if (r[SG_Q_FRAC1] > 0.0) {
-      double *co = cldopt + (((size_t)col * NB + b) * L + i) * d.co_stride;
-      double kext, kscat, phf, fwd;
-      drop_optics(spec->drop[d.drop], b, r[SG_Q_LWC], r[SG_Q_RE], kext, kscat, phf, fwd);
-      double ie = 0.0, is = 0.0, ip = 0.0, iff = 0.0;
-      if (d.ice) ice_optics(spec->ice[d.ice_t], b, r[SG_Q_IWC], r[SG_Q_DE], r[SG_Q_T], ie, is, ip, iff);
-      if (d.f32) {
-        // mixed form: droplets and ice together, (kext, kext - kscat, phf,
-        // fwd) in FP32, the absorption formed here in FP64
-        float4 *cf = (float4 *)((float *)cldopt + (((size_t)col * NB + b) * L + i) * 4);
-        kext = kext + ie; kscat = kscat + is; phf = phf + ip; fwd = fwd + iff;
-        *cf = make_float4((float)kext, (float)(kext - kscat), (float)phf, (float)fwd);
-      } else {
-        co[0] = kext; co[1] = kscat; co[2] = phf; co[3] = fwd;
-        if (d.ice) { co[4] = ie; co[5] = is; co[6] = ip; co[7] = iff; }
-      }
-    }
-  }
-  double *br = bandrec + (((size_t)col * NB + b) * L + i) * SG_NBQ;
-  double *bs = bandscal + ((size_t)col * NB + b) * SG_NBQ;
-  const bool solar = d.isolir == SOCGPU_SOURCE_SOLAR;
-  const double sec0 = colscal[(size_t)col * SG_NS + SG_S_SEC0];
-  const double ray = (solar && l_rayleigh) ? B.rayleigh : 0.0;
-  // clear-air grey extinction: continua, then Rayleigh scattering
-  // (grey_opt_prop.F90:801-835), then the equivalent extinction
-  const double kcont = (gen && B.n_cont > 0 && !d.no_cont) ? continuum_k(B, r[SG_Q_P], r[SG_Q_T],
-                                                  grec[((size_t)col * L + i) * SG_NGQ + SG_G_RHO],
-                                                  r[SG_Q_MMR + SG_GAS_H2O])
-                                    : 0.0;
-  // modal aerosols: their absorption precedes the continua in the clear-air
-  // extinction, their scattering follows Rayleigh's (the sums over the
-  // modes are formed by the pack kernel, aer_sums)
-  double kaer = 0.0, ksc = ray, pfa = 0.0, fwa = 0.0;
-  if (d.n_aer > 0) {
-    const double *ar = ae.rec + (((size_t)col * NB + b) * L + i) * 4;
-    ksc = ar[0]; pfa = ar[1]; fwa = ar[2]; kaer = ar[3];
-  }
-  br[0] = ((kaer + kcont) + ksc) + keq + kgrey;
-  const double ksc_clr = ksc;
-  if (d.triple) {
-    // grey optics of each cloud type (grey_opt_prop.F90:975-1000,
-    // 1185-1230: Rayleigh, then the type's droplets and its ice component
-    // (zero without ice), at layers from the call's cloud top where the
-    // column has cloud), the equivalent extinction (solve_band_k_eqv_scl.F90:
-    // 1038-1045), moments normalised by the scattering (grey_opt_prop.F90:
-    // 1474-1500) and the delta-rescaled phase function (rescale_phase_fnc.F90)
-    const int nct = krange[0] < L ? krange[0] : L;
-    double *co = cldopt + (((size_t)col * NB + b) * L + i) * 8;
-    for (int k = 0; k < 2; k++) {
-      // every type starts from the clear-air totals (aerosols included)
-      double kgt = (kaer + kcont) + ksc_clr, ksc = ksc_clr, phf = pfa, fwd = fwa;
-      if (i + 1 >= nct && r[SG_Q_WCLD] > 0.0) {
-        const SgDrop &dr = spec->drop[k == 0 ? d.drop : d.drop2];
-        const double mmr = r[k == 0 ? SG_Q_LWC : SG_Q_LWC2], re = r[k == 0 ? SG_Q_RE : SG_Q_RE2];
-        double ct, cs, cp, cf;
-        drop_optics(dr, b, mmr, re, ct, cs, cp, cf);
-        kgt = kgt + ct;
-        ksc = ksc + cs;
-        phf = phf + cp;
-        fwd = fwd + cf;
-        // the type's ice component
-        ct = 0.0; cs = 0.0; cp = 0.0; cf = 0.0;
-        if (d.ice)
-          ice_optics(spec->ice[k == 0 ? d.ice_t : d.ice_t2], b, r[k == 0 ? SG_Q_IWC : SG_Q_IWC2],
-                     r[k == 0 ? SG_Q_DE : SG_Q_DE2], r[SG_Q_T], ct, cs, cp, cf);
-        kgt = kgt + ct;
-        ksc = ksc + cs;
-        phf = phf + cp;
-        fwd = fwd + cf;
-      }
-      kgt = kgt + keq + kgrey;
-      if (ksc > kTiny) {
-        const double inv = 1.0 / ksc;
-        fwd = fwd * inv;
-        phf = phf * inv;
-      }
-      phf = (phf - fwd) / (1.0 - fwd);
-      co[4 * k + 0] = kgt;
-      co[4 * k + 1] = ksc;
-      co[4 * k + 2] = phf;
-      co[4 * k + 3] = fwd;
-    }
-  }
-  if (solar) {
-    const double temp_max = 36.043653389117154;  // log(1/DBL_EPSILON)
-    br[1] = adjust * exp(fmin(keq * r[SG_Q_MASS] * sec0, temp_max));
-    br[2] = 0.0;
-    br[3] = 0.0;
-    if (i == 0) { bs[0] = colscal[(size_t)col * SG_NS + SG_S_SOL] * B.solar_flux; bs[1] = 0.0; }
-  } else {
-    // b0, b1: the band's Planck fluxes at the top and bottom of the layer
-    double bt = planck_band(B, spec->n_deg, spec->t_ref_planck, r[SG_Q_T]);
-    // diff_2 (diff_planck_source_mod.F90:112-121); zero for a linear source,
-    // whose sources (ir_source.F90:52-59) are the quadratic ones without it
-    br[1] = d.ir_lin ? 0.0 : 2.0 * (b1 + b0 - 2.0 * bt);
-    br[2] = b1 - b0;                     // diff
-    br[3] = b1;                          // planck at the bottom of the layer
-    if (i == 0) {
-      bs[0] = b0;
-      // (the given surface emission was stored by the pack kernel)
-      if (colscal[(size_t)col * SG_NS + SG_S_LFG] == 0.0)
-        bs[1] = planck_band(B, spec->n_deg, spec->t_ref_planck,
-                            colscal[(size_t)col * SG_NS + SG_S_TGROUND]);
-    }
-  }
 }
 
 // Optical properties of one layer for one lane: clear sky (gas + grey
@@ -1661,17 +1259,15 @@ __device__ __forceinline__ void tri_solve_body(const CallDims &d, const SgSpec *
 // every kernel loops over the concatenated work of all requests and finds
 // the request of a work item by binary search over per-request starts. A
 // request's results are those of the same call made alone.
-// W_MINOR: waves of the per-(column, band) kernel; W_LONG counts those of
-// calls with more than 128 layers (it only decides whether their kernel is
-// launched).
-// W_GEN counts the calls whose spectrum needs the general gas optics (any
-// scaling other than the power law, continua or further gases); a batch with
-// any such call runs the kernels built for it
+// W_BAND + 2 i + gen: blocks (4 columns) of the band kernel by the build that
+// runs them, i = 0, 1, 2 for calls of up to kShortL layers, up to kLongL and
+// more; gen: the spectrum needs the general gas optics.
+// W_GEN counts the calls that need the general build of the triple-column solve.
 // W_SOLVE + 3 i + opt: waves of the solve, by the build that runs them (i = 0
 // for calls of up to kShortL layers, 1 up to kLongL; opt: kOptPlain, kOptGen,
 // kOptAer); W_SOLVE_ANY: calls of more layers
-enum { W_LEV, W_LAY, W_CG, W_MINOR, W_PREP, W_SOLVE, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE, W_PTILE, W_CCOL,
-       W_FTILE, W_LONG, W_GEN, W_GBAND, kNWork };
+enum { W_LAY, W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE, W_PTILE, W_CCOL, W_FTILE,
+       W_GEN, kNWork };
 
 struct ReqDesc {
   CallDims d;
@@ -1917,32 +1513,8 @@ __global__ __launch_bounds__(64 * kCgWaves) void b_cloudgen_kernel(const BatchHd
   }
 }
 
-// waves per SIMD the band kernel is built for (calls of up to 128 layers)
-#ifndef SG_BAND_OCC
-#define SG_BAND_OCC 3
-#endif
-
-template <int NCH, bool GEN>
-__global__ __launch_bounds__(64 * kMinorWaves, NCH == 2 ? SG_BAND_OCC : 2) void b_band_kernel(const BatchHdr *h, const ReqDesc *rq) {
-  const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const long long tot = h->tot[W_MINOR];
-  for (long long w = blockIdx.x * (long long)kMinorWaves + wv; w < tot; w += (long long)gridDim.x * kMinorWaves) {
-    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W_MINOR, w));
-    const ReqDesc &q = rq[r];
-    const int nch = (q.d.L + kWave - 1) / kWave;
-    if ((NCH == 2 && nch <= 2) || (NCH > 2 && nch > 2))
-    {
-      const AerIn ae{G(q.a.aer_mix_ratio), G(q.a.aer_absorption), G(q.a.aer_scattering), G(q.a.aer_asymmetry),
-                     G(q.aerrec)};
-      band_body<NCH, GEN>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), q.a.gas_mix_ratio, q.a.gas_field,
-                          G(q.tlev), G(q.colscal), G(q.bandrec), G(q.bandscal), G(q.cldopt), G(q.krange), ae,
-                          (int)(w - q.s[W_MINOR]), lane);
-    }
-  }
-}
-
-
 #include "solve_rows.h"
+#include "band_rows.h"
 
 // Outputs in tiles of kFinC columns x kFinL levels per block and iteration:
 // partials read along the levels of a column, transposed through LDS,
@@ -2550,12 +2122,10 @@ static size_t request_ws_doubles(const CallDims &d, const SgSpec &S) {
 
 static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]) {
   const long long P = d.P, L = d.L;
-  w[W_LEV] = P * (L + 1);
   w[W_LAY] = P * L;
   w[W_CG] = d.mcica ? P : 0;
-  w[W_MINOR] = P * d.NB;
-  w[W_LONG] = L > 2 * kWave ? P * d.NB : 0;
-  w[W_PREP] = P * d.NB * L;
+  for (int k = 0; k < 6; k++) w[W_BAND + k] = 0;
+  w[W_BAND + 2 * ((L > kShortL) + (L > kLongL)) + (d.ggen ? 1 : 0)] = band_quads(d);
   for (int k = W_SOLVE; k <= W_SOLVE_ANY; k++) w[k] = 0;
   if (!d.triple) {
     const int opt = d.n_aer > 0 ? kOptAer : (d.gen ? kOptGen : kOptPlain);
@@ -2567,7 +2137,6 @@ static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]
   w[W_CCOL] = (d.mcica || d.triple) ? P * ((L + kRangeChunk - 1) / kRangeChunk) : 0;
   w[W_FTILE] = finish_tiles(d);
   w[W_GEN] = d.gen ? 1 : 0;
-  w[W_GBAND] = d.ggen ? 1 : 0;
 }
 
 // Lays out the workspace of request r at *cursor (doubles, 32-byte aligned)
@@ -2639,17 +2208,20 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   } else if (tot[W_CG] > 0) {
     b_cloudgen_kernel<<<blocks(tot[W_CG], kCgWaves), 64 * kCgWaves, 0, s>>>(hdr, rq);
   }
-  {
-    // calls of up to 128 layers, then the longer ones (each kernel skips the
-    // other's waves)
-    const bool gband = tot[W_GBAND] > 0;
-    auto *bk = gband ? b_band_kernel<2, true> : b_band_kernel<2, false>;
-    bk<<<blocks(tot[W_MINOR], kMinorWaves), 64 * kMinorWaves, 0, s>>>(hdr, rq);
-    if (tot[W_LONG] > 0) {
-      auto *bl = gband ? b_band_kernel<kKeqMaxChunks, true> : b_band_kernel<kKeqMaxChunks, false>;
-      bl<<<blocks(tot[W_MINOR], kMinorWaves), 64 * kMinorWaves, 0, s>>>(hdr, rq);
-    }
+#define SG_BAND(KMAX, GEN, W)                                                                                  \
+  if (tot[W] > 0) {                                                                                           \
+    const bool few = tot[W] <= kBandFew;                                                                      \
+    const int n = few ? kBandFewWaves : kBandWaves;                                                           \
+    b_band_kernel<KMAX, GEN, W><<<dim3(blocks(tot[W], 1), few ? kBandFewBlocks : 1), kWave * n,                \
+                                  band_lds_doubles(KMAX, n) * 8, s>>>(hdr, rq);                                \
   }
+  SG_BAND(6, false, W_BAND)
+  SG_BAND(6, true, W_BAND + 1)
+  SG_BAND(9, false, W_BAND + 2)
+  SG_BAND(9, true, W_BAND + 3)
+  SG_BAND(12, false, W_BAND + 4)
+  SG_BAND(12, true, W_BAND + 5)
+#undef SG_BAND
   if (tot[W_TOVL] > 0) b_overlap_kernel<<<blocks(tot[W_TOVL], T), T, 0, s>>>(hdr, rq);
   if (fork) HIPCHK(hipStreamWaitEvent(s, fk->j, 0));
   if (ev_a) HIPCHK(hipEventRecord(ev_a, s));
