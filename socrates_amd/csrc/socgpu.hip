@@ -119,7 +119,7 @@ struct CallDims {
   int P, L, NB, isolir;
   int mcica, mode;   // McICA on, sampling table (0 single, 1 optimal)
   int drop;          // droplet type index (0-based; the stratiform type)
-  int nwpc;          // waves per column of the triple-column solve
+  int n_g;           // major k-terms
   int nw, rpw;       // waves per column of the solve, and rounds of g-points per wave
   int n_gen, n_fill, ipph, ioverlap;
   int triple, drop2; // triple-column representation; convective droplet type
@@ -783,7 +783,7 @@ __device__ __forceinline__ void finish_body(const CallDims &d, const double *__r
                                             double &su, double &sd, double &sx) {
   const int L = d.L;
   su = 0.0; sd = 0.0; sx = 0.0;
-  const int nw = d.triple ? d.nwpc : d.nw;
+  const int nw = d.triple ? 1 : d.nw;
   const bool direct = d.triple || d.isolir == SOCGPU_SOURCE_SOLAR;
   for (int c = 0; c < nw; c++) {
     const double *o = partial + ((size_t)col * nw + c) * 3 * (L + 1);
@@ -887,372 +887,6 @@ __device__ __forceinline__ void overlap_body(const CallDims &d, const double *__
     for (int a = 0; a < 3; a++) o[9 + 3 * a + b] = lo[b] > tol ? ao[a][b] / lo[b] : (a == b ? 1.0 : 0.0);
 }
 
-// Two-stream coefficients of one region of one layer for one lane: single
-// scattering and delta-rescaling (single_scattering_all.F90,
-// rescale_tau_omega.F90:73-80) of the region's grey optics kg (extinction,
-// with the equivalent extinction), ks (scattering), g (rescaled asymmetry),
-// fw (forward scattering) plus the lane's gas absorption kgas, then
-// two_coeff (FP64) or two_coeff_f32 (mixed form, with the absorption formed
-// in FP64 before rounding, as in layer_coef_mixed).
-template <bool MIXED>
-__device__ __forceinline__ void region_coef(const LaneCtx &c, double kgas, double mass, double kg, double ks,
-                                            double g, double fw, Coef &o) {
-#pragma clang fp contract(on)
-  if (!MIXED) {
-    double ktot = kg + kgas;
-    double tau = ktot * mass;
-    double om = fmin(ks / (ktot + kTiny), 1.0 - 32.0 * kEps);
-    tau = tau * (1.0 - om * fw);
-    om = om * (1.0 - fw) / (1.0 - om * fw);
-    two_coeff(c.solar, tau, om, g, c.sec0, o);
-  } else {
-    const float ktot = (float)(kg + kgas);
-    const float kab = (float)((kg - ks) + kgas);
-    const float omc_min = (float)(32.0 * kEps);
-    float tau = ktot * (float)mass;
-    float omc = ktot > 0.0f ? fmaxf(SG_FDIV(kab, ktot), omc_min) : 1.0f;
-    float om = 1.0f - omc;
-    const float sc = 1.0f - om * (float)fw;
-    tau = tau * sc;
-    omc = SG_FDIV(omc, sc);
-    om = 1.0f - omc;
-    CoefF f;
-    two_coeff_f32(c.solar, tau, om, omc, (float)g, (float)c.sec0, f);
-    coef_from_f32(f, o);
-  }
-}
-
-// Region coefficients weighted as two_coeff_region.F90:200-445 forms them:
-// the type's coefficients times its fraction, summed from zero, times the
-// reciprocal of the region fraction (the same fraction here); zero where
-// the type is absent.
-__device__ __forceinline__ void region_mix(double f, Coef &o) {
-  if (f > kTiny) {
-    const double inv = 1.0 / f;
-    o.T = (0.0 + f * o.T) * inv;
-    o.R = (0.0 + f * o.R) * inv;
-    o.T0 = (0.0 + f * o.T0) * inv;
-    o.s1 = (0.0 + f * o.s1) * inv;
-    o.s2 = (0.0 + f * o.s2) * inv;
-  } else {
-    o.T = 0.0; o.R = 0.0; o.T0 = 0.0; o.s1 = 0.0; o.s2 = 0.0;
-  }
-}
-
-template <bool MIXED, bool GEN>
-__device__ __forceinline__ double lane_kgas(const SgTerm &t, const SgSpec *spec, const double *r,
-                                            const double *g) {
-  if (GEN && t.fnc != SG_FNC_POWER_LAW) {
-    const double k = k_scaled(t, spec, r[SG_Q_LNP], r[SG_Q_P], r[SG_Q_T], g, r[SG_Q_MMR + t.gas]);
-    return MIXED ? (double)(float)k : k;
-  }
-  if (MIXED) return (double)k_term_f32(t, (float)r[SG_Q_LNP], (float)r[SG_Q_LNT], (float)r[SG_Q_MMR + t.gas]);
-  return k_term(t, r[SG_Q_LNP], r[SG_Q_LNT], r[SG_Q_MMR + t.gas]);
-}
-
-// Coefficients of the three regions of layer i (0-based) for one lane; the
-// cloud regions only from the cloud top (1-based nct) down.
-template <bool MIXED>
-__device__ __forceinline__ void tri_layer_coef(const LaneCtx &c, double kgas, const double *r,
-                                               const double *bq, const double *co, const double *ar,
-                                               bool cloud_rows, Coef (&o)[3]) {
-  const double mass = r[SG_Q_MASS];
-  if (c.aer) {
-    // clear region with aerosols: moments over the scattering, the phase
-    // function delta-rescaled (grey_opt_prop.F90:1360-1440,
-    // rescale_phase_fnc.F90:116-124)
-    double ks = ar[0], pf = ar[1], fw = ar[2];
-    {
-#pragma clang fp contract(off)
-      if (ks > kTiny) {
-        const double inv = 1.0 / ks;
-        fw = fw * inv;
-        pf = pf * inv;
-      }
-      pf = (pf - fw) / (1.0 - fw);
-    }
-    region_coef<MIXED>(c, kgas, mass, bq[0], ks, pf, fw, o[0]);
-  } else {
-    region_coef<MIXED>(c, kgas, mass, bq[0], c.ksc_clear, 0.0, 0.0, o[0]);
-  }
-  if (cloud_rows) {
-    const double f1 = r[SG_Q_FRAC1], f2 = r[SG_Q_FRAC2];
-    if (f1 > kTiny) region_coef<MIXED>(c, kgas, mass, co[0], co[1], co[2], co[3], o[1]);
-    region_mix(f1, o[1]);
-    if (f2 > kTiny) region_coef<MIXED>(c, kgas, mass, co[4], co[5], co[6], co[7], o[2]);
-    region_mix(f2, o[2]);
-  }
-}
-
-// The triple-column solve of one column for one lane per major k-term
-// (triple_column.F90:255-569): region coefficients (two_coeff_region), the
-// direct beam carried through the overlap (triple_solar_source.F90:180-412)
-// or the area-weighted infra-red sources (triple_column.F90:298-349), the
-// surface sources, and solver_triple_hogan (solver_triple_hogan.F90:
-// 207-411): an upward elimination of the region albedos and sources coupled
-// through the overlap coefficients, then a downward substitution. Three
-// sweeps over the layers: down (solar only; the direct flux entering each
-// region of each layer, kept in tws), up (coefficients, sources and the
-// elimination; per layer and region the substitution pair fu = c1 fd + c2,
-// fd' = e1 fd + e2 kept in tws) and down again (fluxes). tws holds kTriQ
-// doubles per layer and lane, lane-interleaved: [wave][layer][q][64].
-// Output: partial[col][chunk][3][L+1] of this wave's k-term-weighted sums.
-constexpr int kTriQ = 12;
-
-template <bool MIXED, bool GEN>
-__device__ __forceinline__ void tri_solve_body(const CallDims &d, const SgSpec *__restrict__ spec,
-                                               int l_rayleigh, const double *__restrict__ colrec,
-                                               const double *__restrict__ grec,
-                                               const double *__restrict__ colscal,
-                                               const double *__restrict__ bandrec,
-                                               const double *__restrict__ bandscal,
-                                               const double *__restrict__ cldopt,
-                                               const double *__restrict__ ovl,
-                                               const int *__restrict__ krange, double *__restrict__ tws,
-                                               const double *__restrict__ aerrec,
-                                               double *__restrict__ partial, int wave, int lane) {
-  const int L = d.L, NB = d.NB;
-  const int col = wave / d.nwpc, chunk = wave % d.nwpc;
-  if (col >= d.P) return;
-  const bool solar = d.isolir == SOCGPU_SOURCE_SOLAR;
-  const int item = chunk * kWave + lane;
-  const bool active = item < spec->n_g;
-  const int gi = active ? item : 0;
-  const double wgt = active ? spec->g[gi].w : 0.0;
-  const SgTerm t = spec->g[gi];
-  const int b = t.band;
-  const int nct = krange[0] < L ? krange[0] : L;  // 1-based cloud top of the call
-  const double *cs = colscal + (size_t)col * SG_NS;
-  const double *rec = colrec + (size_t)col * L * SG_NQ;
-  const double *br = bandrec + ((size_t)col * NB + b) * L * SG_NBQ;
-  const double *bs = bandscal + ((size_t)col * NB + b) * SG_NBQ;
-  const double *cop = cldopt + ((size_t)col * NB + b) * L * 8;
-  const double *ov = ovl + (size_t)col * (L + 1) * kOv;
-  double *ws = tws + (size_t)wave * L * kTriQ * kWave + lane;
-  double *out = partial + ((size_t)col * d.nwpc + chunk) * 3 * (L + 1);
-  LaneCtx c;
-  c.solar = solar;
-  c.sec0 = cs[SG_S_SEC0];
-  c.ksc_clear = (solar && l_rayleigh) ? spec->band[b].rayleigh : 0.0;
-  c.ice = false;
-  c.nosc = 0;
-  c.aer = GEN && aerrec != nullptr;
-  const double *ab = c.aer ? aerrec + ((size_t)col * NB + b) * L * 4 : nullptr;
-  const double alb_diff = bs[2], alb_dir = bs[3];
-  const double finc = solar ? bs[0] / c.sec0 : -bs[0];  // flux_inc_down (= flux_inc_direct)
-#define TWS(i, q) ws[((size_t)(i) * kTriQ + (q)) * kWave]
-  // lanes past the last k-term neither store nor load the workspace (their
-  // results carry weight 0; zeros keep them finite)
-#define TWL(i, q) (active ? TWS(i, q) : 0.0)
-
-  // --- sweep 1 (solar): direct flux entering each region of each layer
-  double base0 = finc, base1 = 0.0, base2 = 0.0;  // direct flux leaving the layer above, per region
-  if (solar) {
-    double vdir[8];
-    for (int i = 0; i < L; i++) {
-      {  // direct flux at level i, summed 8 levels at a time
-        const int m = i & 7;
-        const double x = wgt * (base0 + base1 + base2);
-#pragma unroll
-        for (int k = 0; k < 8; k++) if (k == m) vdir[k] = x;
-        if (m == 7) {
-          reduce8(vdir, lane);
-          if ((lane & 7) == 0) out[2 * (L + 1) + i - 7 + (lane >> 3)] = vdir[0];
-        }
-      }
-      const double *r = rec + (size_t)i * SG_NQ;
-      const double *bq = br + (size_t)i * SG_NBQ;
-      const double adj = bq[1];
-      const double kgas = lane_kgas<MIXED, GEN>(t, spec, r, grec ? grec + ((size_t)col * L + i) * SG_NGQ : nullptr);
-      Coef o[3];
-      const bool cloud_rows = i + 1 >= nct;
-      tri_layer_coef<MIXED>(c, kgas, r, bq, cop + (size_t)i * 8, ab ? ab + (size_t)i * 4 : nullptr, cloud_rows, o);
-      double top0, top1 = 0.0, top2 = 0.0;
-      if (!cloud_rows) {
-        top0 = base0;
-        base0 = top0 * o[0].T0 * adj;
-      } else {
-        const double *v = ov + (size_t)i * kOv;  // interface at the top of layer i+1
-        top0 = v[0] * base0 + v[1] * base1 + v[2] * base2;
-        top1 = v[3] * base0 + v[4] * base1 + v[5] * base2;
-        top2 = v[6] * base0 + v[7] * base1 + v[8] * base2;
-        base0 = top0 * o[0].T0 * adj;
-        base1 = top1 * o[1].T0 * adj;
-        base2 = top2 * o[2].T0 * adj;
-      }
-      if (active) TWS(i, 0) = top0;
-      if (active) TWS(i, 1) = top1;
-      if (active) TWS(i, 2) = top2;
-    }
-    {  // remaining direct-flux levels (the partial block and the surface)
-      const int bl = L & ~7, m = L & 7;
-      const double x = wgt * (base0 + base1 + base2);
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        if (k == m) vdir[k] = x;
-        else if (k > m) vdir[k] = 0.0;
-      }
-      reduce8(vdir, lane);
-      if ((lane & 7) == 0 && bl + (lane >> 3) <= L) out[2 * (L + 1) + bl + (lane >> 3)] = vdir[0];
-    }
-  } else {
-    for (int i = lane; i <= L; i += kWave) out[2 * (L + 1) + i] = 0.0;
-  }
-
-  // --- sweep 2: upward elimination (solver_triple_hogan.F90:207-312)
-  double a0 = alb_diff, a1 = alb_diff, a2 = alb_diff, g0, g1, g2;
-  if (solar) {
-    g0 = (alb_dir - alb_diff) * base0;
-    g1 = (alb_dir - alb_diff) * base1;
-    g2 = (alb_dir - alb_diff) * base2;
-  } else {
-    const double dps = bs[1] - br[(size_t)(L - 1) * SG_NBQ + 3];
-    const double *u = ov + (size_t)L * kOv + 9;
-    g0 = u[0] * (1.0 - alb_diff) * dps;
-    g1 = u[3] * (1.0 - alb_diff) * dps;
-    g2 = u[6] * (1.0 - alb_diff) * dps;
-  }
-  for (int i = L - 1; i >= 0; i--) {
-    const double *r = rec + (size_t)i * SG_NQ;
-    const double *bq = br + (size_t)i * SG_NBQ;
-    const double kgas = lane_kgas<MIXED, GEN>(t, spec, r, grec ? grec + ((size_t)col * L + i) * SG_NGQ : nullptr);
-    const bool cloud_rows = i + 1 >= nct;
-    Coef o[3];
-    tri_layer_coef<MIXED>(c, kgas, r, bq, cop + (size_t)i * 8, ab ? ab + (size_t)i * 4 : nullptr, cloud_rows, o);
-    double su[3], sd[3];
-    const int nreg = cloud_rows ? 3 : 1;
-    if (solar) {
-      const double adj = bq[1];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        if (k < nreg) {
-          const double top = TWL(i, k);
-          const double base = top * o[k].T0 * adj;
-          su[k] = o[k].s1 * top;
-          sd[k] = (o[k].s2 - o[k].T0) * top + base;
-        }
-      }
-    } else {
-      const double dpl2 = bq[1], dpl = bq[2];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        if (k < nreg) {
-          su[k] = o[k].s1 * dpl + o[k].s2 * dpl2;
-          sd[k] = -o[k].s1 * dpl + o[k].s2 * dpl2;
-        }
-      }
-      if (cloud_rows) {
-        const double w = r[SG_Q_WCLD], wf = 1.0 - w;
-        const double w1 = w * r[SG_Q_FRAC1], w2 = w * r[SG_Q_FRAC2];
-        sd[0] = wf * sd[0]; su[0] = wf * su[0];
-        sd[1] = w1 * sd[1]; su[1] = w1 * su[1];
-        sd[2] = w2 * sd[2]; su[2] = w2 * su[2];
-      }
-    }
-    if (cloud_rows) {
-      const double *vb = ov + (size_t)(i + 1) * kOv;  // interface at the bottom of layer i+1
-      const double th[3] = {a0 * vb[0] + a1 * vb[3] + a2 * vb[6], a0 * vb[1] + a1 * vb[4] + a2 * vb[7],
-                            a0 * vb[2] + a1 * vb[5] + a2 * vb[8]};
-      const double gg[3] = {g0, g1, g2};
-      double lsrc[3], aa[3];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const double T = o[k].T, R = o[k].R;
-        const double binv = 1.0 / (1.0 - th[k] * R);
-        const double gam = th[k] * T;
-        const double h = gg[k] + th[k] * sd[k];
-        lsrc[k] = su[k] + h * T * binv;
-        aa[k] = R + th[k] * T * T * binv;
-        const double c1 = gam * binv, c2 = h * binv;
-        if (active) TWS(i, 4 * k + 0) = c1;
-        if (active) TWS(i, 4 * k + 1) = c2;
-        if (active) TWS(i, 4 * k + 2) = T + R * c1;
-        if (active) TWS(i, 4 * k + 3) = R * c2 + sd[k];
-      }
-      const double *ut = ov + (size_t)i * kOv + 9;    // interface at the top of layer i+1
-      a0 = aa[0]; a1 = aa[1]; a2 = aa[2];
-      g0 = ut[0] * lsrc[0] + ut[1] * lsrc[1] + ut[2] * lsrc[2];
-      g1 = ut[3] * lsrc[0] + ut[4] * lsrc[1] + ut[5] * lsrc[2];
-      g2 = ut[6] * lsrc[0] + ut[7] * lsrc[1] + ut[8] * lsrc[2];
-    } else {
-      double th = a0;
-      if (i + 1 == nct - 1 && nct < L) {
-        const double *vb = ov + (size_t)(i + 1) * kOv;
-        th = a0 * vb[0] + a1 * vb[3] + a2 * vb[6];
-      }
-      const double T = o[0].T, R = o[0].R;
-      const double binv = 1.0 / (1.0 - th * R);
-      const double gam = th * T;
-      const double h = g0 + th * sd[0];
-      const double lam = T * binv;
-      a0 = R + lam * gam;
-      g0 = su[0] + lam * h;
-      const double c1 = gam * binv, c2 = h * binv;
-      if (active) TWS(i, 0) = c1;
-      if (active) TWS(i, 1) = c2;
-      if (active) TWS(i, 2) = T + R * c1;
-      if (active) TWS(i, 3) = R * c2 + sd[0];
-    }
-  }
-
-  // --- sweep 3: downward substitution, up and down fluxes at every level,
-  // summed over the wave 4 levels at a time
-  double v[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) v[k] = 0.0;
-  auto put = [&](int lev, double fu, double fd) {
-    const int m = lev & 3;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      if (k == m) { v[2 * k] = wgt * fu; v[2 * k + 1] = wgt * fd; }
-      else if (k > m && lev == L) { v[2 * k] = 0.0; v[2 * k + 1] = 0.0; }
-    }
-    if (m == 3 || lev == L) {
-      reduce8(v, lane);
-      if ((lane & 7) == 0) {
-        const int j = lane >> 3, lv = (lev & ~3) + (j >> 1);
-        if (lv <= L) out[(j & 1) * (L + 1) + lv] = v[0];
-      }
-    }
-  };
-  double fdt = finc;
-  {
-    const double up0 = nct > 1 ? a0 * finc + g0 : g0 + finc * (ov[0] * a0 + ov[3] * a1 + ov[6] * a2);
-    put(0, up0, finc);
-  }
-  double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-  for (int i = 0; i < L; i++) {
-    double fu, fd;
-    if (i + 1 < nct) {
-      fu = TWL(i, 0) * fdt + TWL(i, 1);
-      fdt = TWL(i, 2) * fdt + TWL(i, 3);
-      fd = fdt;
-    } else {
-      const double *vt = ov + (size_t)i * kOv;
-      if (i + 1 == nct) {
-        d0 = vt[0] * fdt; d1 = vt[3] * fdt; d2 = vt[6] * fdt;
-      } else {
-        const double x0 = d0, x1 = d1, x2 = d2;
-        d0 = vt[0] * x0 + vt[1] * x1 + vt[2] * x2;
-        d1 = vt[3] * x0 + vt[4] * x1 + vt[5] * x2;
-        d2 = vt[6] * x0 + vt[7] * x1 + vt[8] * x2;
-      }
-      const double u0 = TWL(i, 0) * d0 + TWL(i, 1);
-      const double u1 = TWL(i, 4) * d1 + TWL(i, 5);
-      const double u2 = TWL(i, 8) * d2 + TWL(i, 9);
-      d0 = TWL(i, 2) * d0 + TWL(i, 3);
-      d1 = TWL(i, 6) * d1 + TWL(i, 7);
-      d2 = TWL(i, 10) * d2 + TWL(i, 11);
-      fu = u0 + u1 + u2;
-      fd = d0 + d1 + d2;
-      fdt = fd;
-    }
-    put(i + 1, fu, fd);
-  }
-#undef TWS
-#undef TWL
-}
-
 // ------------------------------------------------------------ batches
 // A batch is a list of radiation calls ("requests"), each with its own
 // spectrum, source, shape and options, packed into one launch sequence:
@@ -1266,8 +900,11 @@ __device__ __forceinline__ void tri_solve_body(const CallDims &d, const SgSpec *
 // W_SOLVE + 3 i + opt: waves of the solve, by the build that runs them (i = 0
 // for calls of up to kShortL layers, 1 up to kLongL; opt: kOptPlain, kOptGen,
 // kOptAer); W_SOLVE_ANY: calls of more layers
-enum { W_LAY, W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE, W_PTILE, W_CCOL, W_FTILE,
-       W_GEN, kNWork };
+// W_TSOLVE + 2 i + odd: columns of the triple-column solve, i = 0 and 1 as there,
+// 2 for calls of more layers (they differ in the LDS a block takes); odd: blocks
+// of three waves instead of two (an odd number of waves' k-terms)
+enum { W_LAY, W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE,
+       W_PTILE = W_TSOLVE + 6, W_CCOL, W_FTILE, W_GEN, kNWork };
 
 struct ReqDesc {
   CallDims d;
@@ -1515,6 +1152,7 @@ __global__ __launch_bounds__(64 * kCgWaves) void b_cloudgen_kernel(const BatchHd
 
 #include "solve_rows.h"
 #include "band_rows.h"
+#include "tri_rows.h"
 
 // Outputs in tiles of kFinC columns x kFinL levels per block and iteration:
 // partials read along the levels of a column, transposed through LDS,
@@ -1563,20 +1201,6 @@ __global__ void b_overlap_kernel(const BatchHdr *h, const ReqDesc *rq) {
     const ReqDesc &q = rq[find_req(h, rq, W_TOVL, g)];
     overlap_body(q.d, G(q.colrec), G(q.krange), q.a.cloud_vertical_decorr, q.a.conv_vertical_decorr, G(q.ovl),
                  (int)(g - q.s[W_TOVL]));
-  }
-}
-
-template <bool MIXED, bool GEN>
-__global__ __launch_bounds__(256) void b_tsolve_kernel(const BatchHdr *h, const ReqDesc *rq) {
-  const long long tot = h->tot[W_TSOLVE];
-  const int lane = threadIdx.x % kWave;
-  const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
-  for (long long w = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w < tot; w += nw) {
-    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W_TSOLVE, w));
-    const ReqDesc &q = rq[r];
-    tri_solve_body<MIXED, GEN>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal), G(q.bandrec),
-                               G(q.bandscal), G(q.cldopt), G(q.ovl), G(q.krange), G(q.tws), G(q.aerrec),
-                               G(q.partial), (int)(w - q.s[W_TSOLVE]), lane);
   }
 }
 
@@ -2094,7 +1718,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
     d.n_aer = a->n_aer_mode;
     d.gen = 1;
   }
-  d.nwpc = (S.n_g + kWave - 1) / kWave;
+  d.n_g = S.n_g;
   solve_layout(d, S);
   *entry = &e;
   *dout = d;
@@ -2103,7 +1727,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
 
 // Per-wave partial sums of a request's solve.
 static size_t partial_doubles(const CallDims &d) {
-  if (d.triple) return (size_t)d.P * d.nwpc * 3 * (d.L + 1);
+  if (d.triple) return (size_t)d.P * 3 * (d.L + 1);
   return (size_t)d.P * d.nw * 3 * (d.L + 1);
 }
 
@@ -2115,7 +1739,7 @@ static size_t request_ws_doubles(const CallDims &d, const SgSpec &S) {
              partial_doubles(d) + 2;
   if (d.gx) n += P * L * SG_NGQ;
   if (d.mcica) n += P * L * SG_MAXSUBCOL + P * NB * L * d.co_stride;
-  if (d.triple) n += P * NB * L * 8 + P * (L + 1) * kOv + P * d.nwpc * L * kTriQ * kWave;
+  if (d.triple) n += P * NB * L * 8 + P * (L + 1) * kOv + P * L * kTriQ * tri_row(d.n_g);
   if (d.n_aer) n += P * NB * L * 4;
   return n;
 }
@@ -2132,7 +1756,8 @@ static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]
     w[L > kLongL ? (int)W_SOLVE_ANY : W_SOLVE + 3 * (L > kShortL) + opt] = P * d.nw;
   }
   w[W_TOVL] = d.triple ? P * (L + 1) : 0;
-  w[W_TSOLVE] = d.triple ? P * d.nwpc : 0;
+  for (int k = 0; k < 6; k++) w[W_TSOLVE + k] = 0;
+  if (d.triple) w[W_TSOLVE + 2 * ((L > kShortL) + (L > kLongL)) + tri_chunks(d.n_g) % 2] = P;
   w[W_PTILE] = pack_tiles(d);
   w[W_CCOL] = (d.mcica || d.triple) ? P * ((L + kRangeChunk - 1) / kRangeChunk) : 0;
   w[W_FTILE] = finish_tiles(d);
@@ -2160,7 +1785,7 @@ static void place_request(ReqDesc &q, const SgSpec &S, double *base, size_t *cur
   q.csub = d.mcica ? take(P * L * SG_MAXSUBCOL) : nullptr;
   q.cldopt = d.mcica ? take(P * NB * L * d.co_stride) : (d.triple ? take(P * NB * L * 8) : nullptr);
   q.ovl = d.triple ? take(P * (L + 1) * kOv) : nullptr;
-  q.tws = d.triple ? take((size_t)P * d.nwpc * L * kTriQ * kWave) : nullptr;
+  q.tws = d.triple ? take(P * L * kTriQ * tri_row(d.n_g)) : nullptr;
   q.aerrec = d.n_aer ? take(P * NB * L * 4) : nullptr;
 }
 
@@ -2240,10 +1865,13 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   SG_SOLVE(9, kOptAer, W_SOLVE + 3 + kOptAer)
   SG_SOLVE(12, kOptAny, W_SOLVE_ANY)
 #undef SG_SOLVE
-  if (tot[W_TSOLVE] > 0) {
-    auto *tk = precision == SOCGPU_MIXED ? (gen ? b_tsolve_kernel<true, true> : b_tsolve_kernel<true, false>)
-                                         : (gen ? b_tsolve_kernel<false, true> : b_tsolve_kernel<false, false>);
-    tk<<<blocks(tot[W_TSOLVE], 4), 4 * kWave, 0, s>>>(hdr, rq);
+  for (int w = W_TSOLVE; w < W_TSOLVE + 6; w++) {
+    if (tot[w] == 0) continue;
+    const int i = (w - W_TSOLVE) / 2, lmax = i == 0 ? kShortL : (i == 1 ? kLongL : SG_MAXL);
+    const int n = (w - W_TSOLVE) % 2 ? kTriWaves : kTriWaves - 1;
+    auto *k = precision == SOCGPU_MIXED ? (gen ? b_tsolve_kernel<true, true> : b_tsolve_kernel<true, false>)
+                                        : (gen ? b_tsolve_kernel<false, true> : b_tsolve_kernel<false, false>);
+    k<<<blocks(tot[w], 1), n * kWave, tri_lds_doubles(lmax, n) * 8, s>>>(hdr, rq, w);
   }
   if (ev_b) HIPCHK(hipEventRecord(ev_b, s));
   b_finish_kernel<<<blocks(tot[W_FTILE], 1), kFinC * kFinL, 0, s>>>(hdr, rq);
