@@ -1566,9 +1566,11 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
 // takes a wave per round, the shortest chain (4096 x 90 SW + LW, FP64: 1.20 ms
 // per step with 8192 waves per call, 1.18 ms with 2048 to 4096).
 constexpr long long kSolveWaves = 2048;
-static void solve_layout(CallDims &d, const SgSpec &S) {
+// A call near a workspace limit takes fewer waves and so fewer partial sums
+// (max_waves), down to one per column.
+static void solve_layout(CallDims &d, const SgSpec &S, int max_waves = INT32_MAX) {
   const int rounds = (S.n_g + kRows - 1) / kRows;
-  const long long most = d.P < 16 ? rounds : (rounds + 2) / 3;
+  const long long most = std::min(max_waves, d.P < 16 ? rounds : (rounds + 2) / 3);
   const long long want = std::max<long long>(1, std::min<long long>(most, (kSolveWaves + d.P - 1) / d.P));
   d.rpw = (int)((rounds + want - 1) / want);
   d.nw = (rounds + d.rpw - 1) / d.rpw;
@@ -1790,7 +1792,7 @@ static void place_request(ReqDesc &q, const SgSpec &S, double *base, size_t *cur
 }
 
 static size_t padded_ws_doubles(const CallDims &d, const SgSpec &S) {
-  return request_ws_doubles(d, S) + 13 * 4;  // per-array alignment padding
+  return request_ws_doubles(d, S) + 13 * 3;  // per-array alignment padding
 }
 
 static void fill_desc(ReqDesc &q, const CallDims &d, const SpecEntry &e, const SocgpuRunesArgs &dv,
@@ -2000,6 +2002,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   if (int rc = resolve_request(spectrum_name, a, precision, &e, &d)) return rc;
   const SgSpec &S = e->host;
   const size_t ws_off = (sizeof(DescBlob) + 255) & ~(size_t)255;
+  while (ws_off + padded_ws_doubles(d, S) * 8 > kScratchBytes && d.nw > 1) solve_layout(d, S, d.nw - 1);
   const size_t need = ws_off + padded_ws_doubles(d, S) * 8;
   if (need > kScratchBytes)
     return fail(SOCGPU_ENOMEM, "call needs %zu bytes of workspace, above the %zu-byte fixed workspace of "
@@ -2111,9 +2114,10 @@ struct Resolved {
 };
 
 // Sizes of a batch (workspace, staging, outputs) without placing it; the
-// plan keeps the request list (with the clear-sky companions).
+// plan keeps the request list (with the clear-sky companions). max_waves: of
+// each caller's request, where given.
 static int plan_sizes(int n_caller, const SocgpuRequest *caller_req, int precision, std::vector<Resolved> &res,
-                      Plan &pl) {
+                      Plan &pl, const std::vector<int> *max_waves = nullptr) {
   for (int i = 0; i < n_caller; i++)
     if (!caller_req[i].args || !caller_req[i].diag) return fail(SOCGPU_EINVAL, "request %d: null args or diag", i);
   if (int rc = expand_clear(n_caller, caller_req, pl.x)) return rc;
@@ -2125,6 +2129,7 @@ static int plan_sizes(int n_caller, const SocgpuRequest *caller_req, int precisi
   for (int i = 0; i < n; i++) {
     if (int rc = resolve_request(req[i].spectrum_name, req[i].args, precision, &res[i].e, &res[i].d))
       return rc;
+    if (max_waves) solve_layout(res[i].d, res[i].e->host, (*max_waves)[pl.x.caller[i]]);
     const CallDims &d = res[i].d;
     pl.ws_doubles += padded_ws_doubles(d, res[i].e->host);
     pl.in_bytes += stage_bytes(req[i].args, d.NB);
@@ -2415,6 +2420,7 @@ struct ServeItem {
   SocgpuDiag diag;
   std::string name;
   size_t footprint = 0;
+  int max_waves = INT32_MAX;  // 1 for a call whose footprint is above the budget otherwise
   std::chrono::steady_clock::time_point t_submit;
   int status = 1;  // 1 pending, 0 done, < 0 error
 };
@@ -2490,9 +2496,13 @@ static void serve_finish_slot(SocgpuServer *sv, ServeSlot &sl, int status) {
 static int serve_launch(SocgpuServer *sv, ServeSlot &sl) {
   const int n = (int)sl.items.size();
   std::vector<SocgpuRequest> req(n);
-  for (int i = 0; i < n; i++) req[i] = sl.items[i]->req;
+  std::vector<int> max_waves(n);
+  for (int i = 0; i < n; i++) {
+    req[i] = sl.items[i]->req;
+    max_waves[i] = sl.items[i]->max_waves;
+  }
   std::vector<Resolved> res;
-  if (int rc = plan_sizes(n, req.data(), sv->cfg.precision, res, sl.plan)) return rc;
+  if (int rc = plan_sizes(n, req.data(), sv->cfg.precision, res, sl.plan, &max_waves)) return rc;
   const int nq = sl.plan.n();
   if (sl.ws.ensure(sl.plan.ws_doubles * 8) || sl.in_stage.ensure(sl.plan.in_bytes + 256) ||
       sl.out_stage.ensure(sl.plan.out_doubles * 8 + 64) || sl.desc.ensure(desc_bytes(nq)))
@@ -2620,9 +2630,16 @@ int socgpu_serve_submit(SocgpuServer *sv, const SocgpuRequest *request, long lon
     // with its clear-sky companion, if it asks for clear-sky fluxes
     Expanded x;
     if (int rc = expand_clear(1, &r, x)) return rc;
+    size_t least = 0;
     for (const SocgpuRequest &q : x.req) {
       if (int rc = resolve_request(q.spectrum_name, q.args, sv->cfg.precision, &e, &d)) return rc;
       it->footprint += footprint_bytes(q, d, e->host);
+      solve_layout(d, e->host, 1);
+      least += footprint_bytes(q, d, e->host);
+    }
+    if (it->footprint > sv->cfg.hbm_budget_bytes) {
+      it->footprint = least;
+      it->max_waves = 1;
     }
   }
   it->req = SocgpuRequest{it->name.c_str(), &it->args, &it->diag};
