@@ -434,7 +434,7 @@ __global__ __launch_bounds__(kWave * kBandWaves, KMAX == 6 ? 2 : 1) void b_band_
   double *buf = lds + kBandQ * kRows * lp + wv * 3 * KMAX * kWave;
   const long long tot = h->tot[W];
   for (long long w = blockIdx.x; w < tot; w += gridDim.x) {
-    const ReqDesc &q = rq[__builtin_amdgcn_readfirstlane(find_req(h, rq, W, w))];
+    const ReqDesc &q = rq[find_req(h, rq, W, w)];
     const CallDims d = U_struct(q.d);
     const int c0 = (int)(w - U(q.s[W])) * kRows, P = d.P, L = d.L;
     const double *colrec = G(U(q.colrec)), *tlev = G(U(q.tlev));

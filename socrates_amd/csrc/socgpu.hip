@@ -803,18 +803,6 @@ __device__ __forceinline__ void finish_body(const CallDims &d, const double *__r
   }
 }
 
-// Heating rate from flux divergence (socrates_set_diag.F90:140-210), K/s.
-__device__ __forceinline__ void heating_body(int P, int L, const double *__restrict__ up,
-                                             const double *__restrict__ down,
-                                             const double *__restrict__ heat_cap,
-                                             double *__restrict__ hr, int idx) {
-  if (idx >= P * L) return;
-  int col = idx % P, i = idx / P;  // layer i+1 lies between levels i and i+1
-  double fdiv = down[(size_t)i * P + col] - down[(size_t)(i + 1) * P + col] +
-                up[(size_t)(i + 1) * P + col] - up[(size_t)i * P + col];
-  hr[idx] = heat_cap ? fdiv / heat_cap[idx] : fdiv;
-}
-
 // ------------------------------------------------------------ triple column
 // Maximum-random overlap transfer coefficients of the triple-column
 // representation (overlap_coupled.F90:150-453 with full correlation; the
@@ -903,7 +891,7 @@ __device__ __forceinline__ void overlap_body(const CallDims &d, const double *__
 // W_TSOLVE + 2 i + odd: columns of the triple-column solve, i = 0 and 1 as there,
 // 2 for calls of more layers (they differ in the LDS a block takes); odd: blocks
 // of three waves instead of two (an odd number of waves' k-terms)
-enum { W_LAY, W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE,
+enum { W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE,
        W_PTILE = W_TSOLVE + 6, W_CCOL, W_FTILE, W_GEN, kNWork };
 
 struct ReqDesc {
@@ -947,16 +935,38 @@ __device__ __forceinline__ SocgpuRunesArgs gargs(const SocgpuRunesArgs &a) {
   return g;
 }
 
+// The request of work item g (the same for all 64 lanes) of space w: every round
+// the lanes probe 64 starts, so 64 requests take one round of memory latency and
+// 4096 two (a binary search, 8 for 216 requests, made every block of a short
+// kernel wait for about 4 us).
 __device__ __forceinline__ int find_req(const BatchHdr *h, const ReqDesc *rq, int w, long long g) {
-  int lo = 0, hi = h->R - 1;
+  const int lane = threadIdx.x & (kWave - 1);
+  int lo = 0, n = U(h->R);
+  while (n > 1) {
+    const int step = (n + kWave - 1) / kWave, at = lane * step;
+    const bool le = at < n && rq[lo + (at < n ? at : 0)].s[w] <= g;
+    const int skip = (__popcll(__ballot(le)) - 1) * step;
+    lo += skip;
+    n = min(step, n - skip);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// The same for items base + lane of one wave, each lane its own request.
+__device__ __forceinline__ int find_req_lane(const BatchHdr *h, const ReqDesc *rq, int w, long long base,
+                                             long long tot) {
+  const long long end = base + kWave < tot ? base + kWave : tot;
+  int lo = find_req(h, rq, w, base), hi = find_req(h, rq, w, end - 1);
+  const long long g = base + (threadIdx.x & (kWave - 1));
   while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
+    const int mid = (lo + hi + 1) >> 1;
     if (rq[mid].s[w] <= g) lo = mid;
     else hi = mid - 1;
   }
   return lo;
 }
 
+// (the pack kernel does this for calls that run it)
 __global__ void b_init_kernel(const BatchHdr *h, const ReqDesc *rq) {
   int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= h->R) return;
@@ -1011,13 +1021,17 @@ __global__ __launch_bounds__(kPackC * kPackL) void b_pack_kernel(const BatchHdr 
   const long long tot = h->tot[W_PTILE];
   const int tx = threadIdx.x % kPackC, ty = threadIdx.x / kPackC;
   for (long long tile = blockIdx.x; tile < tot; tile += gridDim.x) {
-    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W_PTILE, tile));
+    const int r = find_req(h, rq, W_PTILE, tile);
     const ReqDesc &q = rq[r];
     const SocgpuRunesArgs a = gargs(q.a);
     const SgSpec *spec = G(q.spec);
     double *colrec = G(q.colrec), *grec = G(q.grec), *tlev = G(q.tlev);
     const int P = q.d.P, L = q.d.L;
     const int t = (int)(tile - q.s[W_PTILE]);
+    if (t == 0 && threadIdx.x == 0) {   // no cloud yet: the range kernel lowers and raises these
+      G(q.krange)[0] = L + 1;
+      G(q.krange)[1] = 0;
+    }
     const int ntc = (P + kPackC - 1) / kPackC;
     const int c0 = (t % ntc) * kPackC, i0 = (t / ntc) * kPackL;
     const int col = c0 + tx, i = i0 + ty;
@@ -1079,8 +1093,9 @@ __global__ void b_cldrange_kernel(const BatchHdr *h, const ReqDesc *rq) {
        base += stride) {
     const long long g = base + lane;
     int r = -1, kmin = INT32_MAX, kmax = 0;
+    const int rl = find_req_lane(h, rq, W_CCOL, base, tot);
     if (g < tot) {
-      r = find_req(h, rq, W_CCOL, g);
+      r = rl;
       const ReqDesc &q = rq[r];
       const SocgpuRunesArgs a = gargs(q.a);
       const int idx = (int)(g - q.s[W_CCOL]), P = q.d.P, L = q.d.L;
@@ -1131,7 +1146,7 @@ __global__ __launch_bounds__(64 * kCgWaves) void b_cloudgen_kernel(const BatchHd
   const long long tot = h->tot[W_CG];
   const double *loaded = nullptr;
   for (long long base = (long long)blockIdx.x * kCgWaves; base < tot; base += (long long)gridDim.x * kCgWaves) {
-    const ReqDesc &q0 = rq[__builtin_amdgcn_readfirstlane(find_req(h, rq, W_CG, base))];
+    const ReqDesc &q0 = rq[find_req(h, rq, W_CG, base)];
     const int nx0 = q0.n1 * q0.n2;
     if (q0.xcw != loaded && nx0 <= kXcwMax) {
       const double *x0 = G(q0.xcw);
@@ -1141,7 +1156,7 @@ __global__ __launch_bounds__(64 * kCgWaves) void b_cloudgen_kernel(const BatchHd
     __syncthreads();
     const long long w = base + wv;
     if (w < tot) {
-      const ReqDesc &q = rq[__builtin_amdgcn_readfirstlane(find_req(h, rq, W_CG, w))];
+      const ReqDesc &q = rq[find_req(h, rq, W_CG, w)];
       const double *tab = (q.xcw == loaded && q.n1 * q.n2 <= kXcwMax) ? sx : q.xcw;
       cloudgen_body(q.d, G(q.colrec), G(q.a.rand_seed), q.dp_cf, q.dp_cw, G(q.krange), tab, q.n1, q.n2,
                     G(q.csub), G(q.colscal), (int)(w - q.s[W_CG]), lane);
@@ -1155,12 +1170,16 @@ __global__ __launch_bounds__(64 * kCgWaves) void b_cloudgen_kernel(const BatchHd
 #include "tri_rows.h"
 
 // Outputs in tiles of kFinC columns x kFinL levels per block and iteration:
-// partials read along the levels of a column, transposed through LDS,
-// written along the profiles of a level.
+// partials read along the levels of a column, transposed through LDS, written
+// along the profiles of a level. A tile's last level is the next one's first, so
+// that each tile has both levels of its kFinL - 1 layers and forms their heating
+// rates from flux divergence (socrates_set_diag.F90:140-210, K/s): 7 % more sums
+// against a kernel of its own that read the fluxes again (9 us of a 4096 x 90
+// step, and a launch).
 constexpr int kFinC = 16, kFinL = 16;
 
 __host__ __device__ inline int finish_tiles(const CallDims &d) {
-  return ((d.P + kFinC - 1) / kFinC) * ((d.L + 1 + kFinL - 1) / kFinL);
+  return ((d.P + kFinC - 1) / kFinC) * ((d.L + kFinL - 2) / (kFinL - 1));
 }
 
 __global__ __launch_bounds__(kFinC * kFinL) void b_finish_kernel(const BatchHdr *h, const ReqDesc *rq) {
@@ -1168,12 +1187,12 @@ __global__ __launch_bounds__(kFinC * kFinL) void b_finish_kernel(const BatchHdr 
   const long long tot = h->tot[W_FTILE];
   const int ta = threadIdx.x % kFinL, tb = threadIdx.x / kFinL;
   for (long long tile = blockIdx.x; tile < tot; tile += gridDim.x) {
-    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W_FTILE, tile));
+    const int r = find_req(h, rq, W_FTILE, tile);
     const ReqDesc &q = rq[r];
     const int P = q.d.P, L = q.d.L;
     const int t = (int)(tile - q.s[W_FTILE]);
     const int ntc = (P + kFinC - 1) / kFinC;
-    const int c0 = (t % ntc) * kFinC, l0 = (t / ntc) * kFinL;
+    const int c0 = (t % ntc) * kFinC, l0 = (t / ntc) * (kFinL - 1);
     {
       const int col = c0 + tb, lev = l0 + ta;   // levels fastest
       if (col < P && lev <= L)
@@ -1183,11 +1202,16 @@ __global__ __launch_bounds__(kFinC * kFinL) void b_finish_kernel(const BatchHdr 
     __syncthreads();
     {
       const int col = c0 + ta, lev = l0 + tb;   // profiles fastest
-      if (col < P && lev <= L) {
+      if (col < P && lev <= L && (tb < kFinL - 1 || lev == L)) {
         const size_t idx = (size_t)lev * P + col;
         G(q.up)[idx] = sh[0][ta][tb];
         G(q.dn)[idx] = sh[1][ta][tb];
         if (q.dir) G(q.dir)[idx] = sh[2][ta][tb];
+        if (q.hr && lev < L) {                  // layer lev + 1, between levels lev and lev + 1
+          const double fdiv = sh[1][ta][tb] - sh[1][ta][tb + 1] + sh[0][ta][tb + 1] - sh[0][ta][tb];
+          const double *cap = G(q.a.layer_heat_capacity);
+          G(q.hr)[idx] = cap ? fdiv / cap[idx] : fdiv;
+        }
       }
     }
     __syncthreads();
@@ -1196,21 +1220,13 @@ __global__ __launch_bounds__(kFinC * kFinL) void b_finish_kernel(const BatchHdr 
 
 __global__ void b_overlap_kernel(const BatchHdr *h, const ReqDesc *rq) {
   const long long tot = h->tot[W_TOVL];
-  for (long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x; g < tot;
-       g += (long long)gridDim.x * blockDim.x) {
-    const ReqDesc &q = rq[find_req(h, rq, W_TOVL, g)];
-    overlap_body(q.d, G(q.colrec), G(q.krange), q.a.cloud_vertical_decorr, q.a.conv_vertical_decorr, G(q.ovl),
-                 (int)(g - q.s[W_TOVL]));
-  }
-}
-
-__global__ void b_heating_kernel(const BatchHdr *h, const ReqDesc *rq) {
-  const long long tot = h->tot[W_LAY];
-  for (long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x; g < tot;
-       g += (long long)gridDim.x * blockDim.x) {
-    const ReqDesc &q = rq[find_req(h, rq, W_LAY, g)];
-    if (q.hr)
-      heating_body(q.d.P, q.d.L, G(q.up), G(q.dn), G(q.a.layer_heat_capacity), G(q.hr), (int)(g - q.s[W_LAY]));
+  const int lane = threadIdx.x & (kWave - 1);
+  for (long long base = blockIdx.x * (long long)blockDim.x + threadIdx.x - lane; base < tot;
+       base += (long long)gridDim.x * blockDim.x) {
+    const ReqDesc &q = rq[find_req_lane(h, rq, W_TOVL, base, tot)];
+    if (base + lane < tot)
+      overlap_body(q.d, G(q.colrec), G(q.krange), q.a.cloud_vertical_decorr, q.a.conv_vertical_decorr, G(q.ovl),
+                   (int)(base + lane - q.s[W_TOVL]));
   }
 }
 
@@ -1748,7 +1764,6 @@ static size_t request_ws_doubles(const CallDims &d, const SgSpec &S) {
 
 static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]) {
   const long long P = d.P, L = d.L;
-  w[W_LAY] = P * L;
   w[W_CG] = d.mcica ? P : 0;
   for (int k = 0; k < 6; k++) w[W_BAND + k] = 0;
   w[W_BAND + 2 * ((L > kShortL) + (L > kLongL)) + (d.ggen ? 1 : 0)] = band_quads(d);
@@ -1813,15 +1828,14 @@ static void fill_desc(ReqDesc &q, const CallDims &d, const SpecEntry &e, const S
 // Launches the kernel sequence of a packed batch on stream s. hdr/rq are
 // device copies of the batch header and descriptors; tot is the host copy of
 // the work totals (grid sizes); solve-kernel time between ev_a and ev_b.
-static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long tot[kNWork], int R,
-                        int precision, hipStream_t s, const Fork *fk, hipEvent_t ev_a, hipEvent_t ev_b) {
+static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long tot[kNWork], int precision,
+                        hipStream_t s, const Fork *fk, hipEvent_t ev_a, hipEvent_t ev_b) {
   const int T = 256;
   const bool gen = tot[W_GEN] > 0;
   auto blocks = [](long long n, int per) {
     long long b = (n + per - 1) / per;
     return (int)(b < 1 ? 1 : (b > 1048576 ? 1048576 : b));
   };
-  b_init_kernel<<<(R + 63) / 64, 64, 0, s>>>(hdr, rq);
   b_pack_kernel<<<blocks(tot[W_PTILE], 1), kPackC * kPackL, 0, s>>>(hdr, rq);
   if (tot[W_CCOL] > 0) b_cldrange_kernel<<<blocks(tot[W_CCOL], T), T, 0, s>>>(hdr, rq);
   // the cloud generator on the side stream when there is one, beside the
@@ -1877,7 +1891,6 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   }
   if (ev_b) HIPCHK(hipEventRecord(ev_b, s));
   b_finish_kernel<<<blocks(tot[W_FTILE], 1), kFinC * kFinL, 0, s>>>(hdr, rq);
-  b_heating_kernel<<<blocks(tot[W_LAY], T), T, 0, s>>>(hdr, rq);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1928,7 +1941,7 @@ int socgpu_runes(const char *spectrum_name, const SocgpuRunesArgs *a, SocgpuDiag
   HIPCHK(hipMemcpyAsync(g_ctx.desc.p, &host, sizeof host, hipMemcpyHostToDevice, s));
   const BatchHdr *dh = (const BatchHdr *)g_ctx.desc.p;
   const ReqDesc *dq = (const ReqDesc *)((char *)g_ctx.desc.p + offsetof(decltype(host), q));
-  if (int rc = launch_batch(dh, (ReqDesc *)dq, host.h.tot, 1, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
+  if (int rc = launch_batch(dh, (ReqDesc *)dq, host.h.tot, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
   HIPCHK(hipEventRecord(g_ctx.ev3, s));
   int herr = 0;
   HIPCHK(hipMemcpyAsync(&herr, &dh->err, sizeof herr, hipMemcpyDeviceToHost, s));
@@ -2020,7 +2033,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   DescBlob *dd = (DescBlob *)g_ctx.scratch_dev;
   HIPCHK(hipEventRecord(g_ctx.ev0, s));
   b_desc_store_kernel<<<1, 64, 0, s>>>(host, dd);
-  if (int rc = launch_batch(&dd->h, &dd->q, host.h.tot, 1, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
+  if (int rc = launch_batch(&dd->h, &dd->q, host.h.tot, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
   HIPCHK(hipEventRecord(g_ctx.ev3, s));
   HIPCHK(hipMemcpyAsync(g_ctx.err_host, &dd->h.err, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
@@ -2270,7 +2283,7 @@ int socgpu_runes_batch(int n_request, const SocgpuRequest *requests, int precisi
   HIPCHK(hipMemcpyAsync(g_ctx.desc.p, blob.data(), blob.size(), hipMemcpyHostToDevice, s));
   const BatchHdr *dh = (const BatchHdr *)g_ctx.desc.p;
   ReqDesc *dq = (ReqDesc *)((char *)g_ctx.desc.p + sizeof(BatchHdr));
-  if (int rc = launch_batch(dh, dq, pl.h.tot, pl.n(), precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
+  if (int rc = launch_batch(dh, dq, pl.h.tot, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
   HIPCHK(hipEventRecord(g_ctx.ev3, s));
   int herr = 0;
   HIPCHK(hipMemcpyAsync(&herr, &dh->err, sizeof herr, hipMemcpyDeviceToHost, s));
@@ -2350,7 +2363,7 @@ int socgpu_batch_run(SocgpuBatch *b, int n_request, const SocgpuRequest *request
     batch_drop_graph(b);
     HIPCHK(hipStreamSynchronize(s));
     HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int rc = launch_batch(dh, dq, b->cap, b->cap_desc / sizeof(ReqDesc) + 1, b->precision, s, &b->fork, nullptr, nullptr);
+    int rc = launch_batch(dh, dq, b->cap, b->precision, s, &b->fork, nullptr, nullptr);
     hipGraph_t g = nullptr;
     hipError_t ec = hipStreamEndCapture(s, &g);
     if (rc) return rc;
@@ -2526,7 +2539,7 @@ static int serve_launch(SocgpuServer *sv, ServeSlot &sl) {
   HIPCHK(hipMemcpyAsync(sl.desc.p, sl.pinned, desc_bytes(nq), hipMemcpyHostToDevice, s));
   const BatchHdr *dh = (const BatchHdr *)sl.desc.p;
   ReqDesc *dq = (ReqDesc *)((char *)sl.desc.p + sizeof(BatchHdr));
-  if (int rc = launch_batch(dh, dq, sl.plan.h.tot, nq, sv->cfg.precision, s, &sl.fork, nullptr, nullptr)) return rc;
+  if (int rc = launch_batch(dh, dq, sl.plan.h.tot, sv->cfg.precision, s, &sl.fork, nullptr, nullptr)) return rc;
   HIPCHK(hipMemcpyAsync(&((BatchHdr *)sl.pinned)->err, &dh->err, sizeof(int), hipMemcpyDeviceToHost, s));
   if (int rc = copy_back_issue(sl.plan, sl.out_stage.as<double>(), sl.out_host_used, s)) return rc;
   HIPCHK(hipEventRecord(sl.done, s));
@@ -2919,7 +2932,6 @@ int socgpu_cloud_gen(int n_profile, int n_layer, int n_subcol, int n_req, int ip
     return fail(SOCGPU_ENOMEM, "allocation failed");
   std::memset(&host, 0, sizeof host);
   host.h.R = 1;
-  host.h.tot[W_LAY] = (long long)P * L;
   host.h.tot[W_CG] = P;
   host.h.tot[W_CCOL] = (long long)P * ((L + kRangeChunk - 1) / kRangeChunk);
   host.q.a.cloud_frac = dcf.as<double>();

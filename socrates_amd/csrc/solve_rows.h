@@ -663,7 +663,7 @@ __global__ __launch_bounds__(256, KMAX <= 9 ? 2 : 1) void b_solve_kernel(const B
   const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
   for (long long w0 = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w0 < tot; w0 += nw) {
     const int w = __builtin_amdgcn_readfirstlane((int)w0);
-    const int r = __builtin_amdgcn_readfirstlane(find_req(h, rq, W, w));
+    const int r = find_req(h, rq, W, w);
     const ReqDesc &q = rq[r];
     const int wave = w - (int)q.s[W];
     if (q.d.isolir == SOCGPU_SOURCE_SOLAR)

@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kTriWaves * kWave, 3) void b_tsolve_kernel(const Ba
   const int nwv = blockDim.x / kWave;
   const long long tot = h->tot[space];
   for (long long w = blockIdx.x; w < tot; w += gridDim.x) {
-    const ReqDesc &q = rq[__builtin_amdgcn_readfirstlane(find_req(h, rq, space, w))];
+    const ReqDesc &q = rq[find_req(h, rq, space, w)];
     const CallDims d = U_struct(q.d);
     const int col = (int)(w - U(q.s[space])), L = d.L, lp = L + 1;
     const SgSpec *spec = G(U(q.spec));
