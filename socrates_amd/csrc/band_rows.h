@@ -173,19 +173,21 @@ __device__ __forceinline__ void band_rows(const ReqDesc &q, const CallDims &d, c
   // the absorption of a term in layer i. Further gases (general gas optics): the
   // call's field, clamped at 0, else its well-mixed ratio
   // (socrates_set_atm.F90:535-622)
-  const auto absorb = [&](const SgTerm &t, int i) -> double {
-    double mmr;
+  const auto amount = [&](const SgTerm &t, int i) -> double {
     if (GEN && t.gas >= SG_GAS_WM0) {
       const double *fld = G(U(q.a.gas_field[t.gas - SG_GAS_WM0]));
-      mmr = fld ? fmax(fld[(size_t)i * d.P + col], 0.0) : U(q.a.gas_mix_ratio[t.gas - SG_GAS_WM0]);
-    } else {
-      mmr = t.gas == SG_GAS_ZERO ? 0.0 : x(3 + t.gas, i);
+      return fld ? fmax(fld[(size_t)i * d.P + col], 0.0) : U(q.a.gas_mix_ratio[t.gas - SG_GAS_WM0]);
     }
+    return t.gas == SG_GAS_ZERO ? 0.0 : x(3 + t.gas, i);
+  };
+  const auto absorb = [&](const SgTerm &t, int i) -> double {
+    const double mmr = amount(t, i);
     if (GEN && t.fnc != SG_FNC_POWER_LAW)
       return k_scaled(t, spec, x(0, i), rec[(size_t)i * SG_NQ + SG_Q_P], x(6, i),
                       grec ? grec + (size_t)i * SG_NGQ : nullptr, mmr);
     return k_term(t, x(0, i), x(1, i), mmr);
   };
+  const int nt = GEN ? U(spec->n_tmp) : 0;
   int t0 = minor0;
   for (int j = 0; j < n_gas; j++) {
     const int nk = U(B.minor_nk[j]);
@@ -202,11 +204,24 @@ __device__ __forceinline__ void band_rows(const ReqDesc &q, const CallDims &d, c
     for (int qt = 0; qt < nk; qt++) {
       const SgTerm t = U_term(spec->minor[t0 + qt]);
       double kk[KMAX];
-      if (GEN)
-        for (int c = 0; c < K; c++) buf[c * kWave + lane] = absorb(t, layer(c));
+      if (GEN && t.fnc == SG_FNC_LOOKUP) {
+        // (unrolled, so that the layers' table entries are read together: one at a
+        // time, each layer waited for its record and then for its entries, and the
+        // kernel took 220 us of a 1024 x 70 infra-red segment with look-up tables)
+        const double *kl = G(U(spec->klut)) + (size_t)t.lut * U(spec->n_pre) * nt;
+        int o0[KMAX], o1[KMAX];
 #pragma unroll
-      for (int c = 0; c < KMAX; c++) {
-        {
+        for (int c = 0; c < KMAX; c++) lut_at(grec[(size_t)layer(c) * SG_NGQ + SG_G_IDX], nt, o0[c], o1[c]);
+#pragma unroll
+        for (int c = 0; c < KMAX; c++) {
+          const double v = lut_k(kl, o0[c], o1[c], grec + (size_t)layer(c) * SG_NGQ, amount(t, layer(c)));
+          kk[c] = has(c) ? v : 0.0;
+        }
+      } else {
+        if (GEN)
+          for (int c = 0; c < K; c++) buf[c * kWave + lane] = absorb(t, layer(c));
+#pragma unroll
+        for (int c = 0; c < KMAX; c++) {
           const double v = GEN ? (c < K ? buf[c * kWave + lane] : 0.0) : absorb(t, layer(c));
           kk[c] = has(c) ? v : 0.0;
         }

@@ -194,6 +194,21 @@ SG_HD double k_term(const SgTerm &t, double lnp, double lnt, double mmr) {
   return t.k * fmax(0.0, s * mmr);
 }
 
+// A look-up term's k_abs of one layer (below): the offsets of its pairs of table
+// entries, from the layer's packed indices, and the weighted sum.
+SG_HD void lut_at(double packed, int nt, int &o0, int &o1) {
+  const int idx = (int)packed;
+  const int jp = idx & 255, jt = (idx >> 8) & 255, jtt = idx >> 16;
+  o0 = jp * nt + jt;
+  o1 = (jp + 1) * nt + jtt;
+}
+SG_HD double lut_k(const double *kl, int o0, int o1, const double *g, double mmr) {
+#pragma clang fp contract(off)
+  const double ke = fmax(0.0, g[SG_G_F00] * kl[o0] + g[SG_G_F10] * kl[o1] + g[SG_G_F01] * kl[o0 + 1] +
+                                  g[SG_G_F11] * kl[o1 + 1]);
+  return fmax(0.0, ke * mmr);
+}
+
 // k_abs of one term at one layer for the other scalings on the path:
 //  - power quadratic, k * max(0, (p/p_ref)^a (1 + b x + c x^2) * mmr) with
 //    x = T/T_ref - 1 (scale_absorb.F90:176-193);
@@ -208,13 +223,10 @@ SG_HD double k_scaled(const SgTerm &t, const SgSpec *spec, double lnp, double p,
                       const double *g, double mmr) {
 #pragma clang fp contract(off)
   if (t.fnc == SG_FNC_LOOKUP) {
-    const int idx = (int)g[SG_G_IDX];
-    const int jp = idx & 255, jt = (idx >> 8) & 255, jtt = idx >> 16, nt = U(spec->n_tmp);
-    const double *kl = G(U(spec->klut)) + (size_t)t.lut * U(spec->n_pre) * nt;
-    const double ke = fmax(0.0, g[SG_G_F00] * kl[jp * nt + jt] + g[SG_G_F10] * kl[(jp + 1) * nt + jtt] +
-                                    g[SG_G_F01] * kl[jp * nt + jt + 1] +
-                                    g[SG_G_F11] * kl[(jp + 1) * nt + jtt + 1]);
-    return fmax(0.0, ke * mmr);
+    const int nt = U(spec->n_tmp);
+    int o0, o1;
+    lut_at(g[SG_G_IDX], nt, o0, o1);
+    return lut_k(G(U(spec->klut)) + (size_t)t.lut * U(spec->n_pre) * nt, o0, o1, g, mmr);
   }
   double s;
   if (t.fnc == SG_FNC_POWER_QUAD) {

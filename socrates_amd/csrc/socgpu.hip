@@ -574,7 +574,7 @@ __device__ __forceinline__ void load_layer(const LaneSrc &s, int i, LayerIn &x) 
   x.lnt = s.hot[s.hp + i];
   x.mass = s.hot[2 * s.hp + i];
   x.mmr = s.mmr[i];
-  if (GEN && !CLR)
+  if (GEN && GAS)
     x.kx = s.fnc != SG_FNC_POWER_LAW
                ? k_scaled(*s.term, s.spec, x.lnp, r[SG_Q_P], r[SG_Q_T], s.grec ? s.grec + i * SG_NGQ : nullptr, x.mmr)
                : (MIXED ? (double)k_term_f32(*s.term, (float)x.lnp, (float)x.lnt, (float)x.mmr)
@@ -1871,7 +1871,7 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
 #define SG_SOLVE(KMAX, OPT, W)                                                                               \
   if (tot[W] > 0) {                                                                                         \
     auto *k = precision == SOCGPU_MIXED ? b_solve_kernel<true, OPT, KMAX, W> : b_solve_kernel<false, OPT, KMAX, W>; \
-    k<<<blocks(tot[W], wpb), wpb * kWave, wpb * solve_lds_doubles<KMAX>() * 8, s>>>(hdr, rq);                \
+    k<<<blocks(tot[W], wpb), wpb * kWave, wpb * solve_lds_doubles<KMAX, OPT>() * 8, s>>>(hdr, rq);                \
   }
   SG_SOLVE(6, kOptPlain, W_SOLVE + kOptPlain)
   SG_SOLVE(6, kOptGen, W_SOLVE + kOptGen)

@@ -225,15 +225,45 @@ struct RowState {
 
 // General gas optics: the term's absorption in each of the lane's layers,
 // ahead of the unrolled layer code (which would hold every scaling K times).
-template <bool MIXED>
-__device__ __forceinline__ void row_gas(const SgTerm &t, const LaneSrc &src, int n, const RowMap &mp, double *low,
-                                        int lane) {
-  for (int k = 0; k < mp.K; k++) {
-    const int i = min(mp.i0 + k, n - 1);
-    LayerIn x;
-    load_layer<MIXED, true, false, true>(src, i, x);
-    low[k * kWave + lane] = x.kx;
+// Look-up terms three layers at a time, so that their loads overlap (one at a
+// time, each layer waited for its record and then for its table entries).
+// layer(k): the lane's k-th layer; put(k, v): keeps its absorption.
+template <bool MIXED, class Layer, class Put>
+__device__ __forceinline__ void row_gas(const SgTerm &t, const LaneSrc &src, int K, const Layer &layer,
+                                        const Put &put) {
+  const bool lut = t.fnc == SG_FNC_LOOKUP;
+  if (__any(lut)) {
+    const int nt = U(src.spec->n_tmp);
+    const double *kl = G(U(src.spec->klut)) + (size_t)(lut ? t.lut : 0) * U(src.spec->n_pre) * nt;
+    for (int k0 = 0; k0 < K; k0 += 3) {
+      int i[3], o0[3], o1[3];
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        i[j] = layer(min(k0 + j, K - 1));
+        lut_at(src.grec[(size_t)i[j] * SG_NGQ + SG_G_IDX], nt, o0[j], o1[j]);
+      }
+      double v[3];
+#pragma unroll
+      for (int j = 0; j < 3; j++) v[j] = lut_k(kl, o0[j], o1[j], src.grec + (size_t)i[j] * SG_NGQ, src.mmr[i[j]]);
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+        if (k0 + j < K) put(k0 + j, v[j]);
+    }
   }
+  if (!lut)
+    for (int k = 0; k < K; k++) {
+      LayerIn x;
+      load_layer<MIXED, true, false, true>(src, layer(k), x);
+      put(k, x.kx);
+    }
+}
+
+// The same of a clear run of n layers, into low.
+template <bool MIXED>
+__device__ __forceinline__ void row_gas_clear(const SgTerm &t, const LaneSrc &src, int n, const RowMap &mp,
+                                              double *low, int lane) {
+  row_gas<MIXED>(t, src, mp.K, [&](int k) { return max(min(mp.i0 + k, n - 1), 0); },
+                 [&](int k, double v) { low[k * kWave + lane] = v; });
 }
 
 // Down the first n layers of the column, all clear: eliminates the lane's K
@@ -248,7 +278,7 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
 #pragma clang fp contract(on)
   Slab S{1.0, 0.0, 0.0, 0.0, 0.0};
   double f = 1.0, fr[SOLAR ? KMAX : 1];
-  if (GEN) row_gas<MIXED>(t, src, n, mp, low, lane);
+  if (GEN) row_gas_clear<MIXED>(t, src, n, mp, low, lane);
   // each layer's inputs are loaded while the one before is computed
   LayerIn x, nx;
   load_layer<MIXED, GEN, true>(src, max(min(mp.i0, n - 1), 0), nx);
@@ -310,7 +340,7 @@ __device__ __forceinline__ void row_down_absorb(const LaneCtx &c, const SgTerm &
                                                 const RowMap &mp, int s, double finc, RowState<KMAX, true> &w,
                                                 double &dn, double *low, int lane) {
 #pragma clang fp contract(on)
-  if (GEN) row_gas<false>(t, src, n, mp, low, lane);
+  if (GEN) row_gas_clear<false>(t, src, n, mp, low, lane);
   LayerIn x, nx;
   load_layer<false, GEN, true>(src, max(min(mp.i0, n - 1), 0), nx);
   double A = 1.0, C = 0.0;
@@ -424,9 +454,13 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
   const bool first = p == 0, last = p == NP - 1;
   const int n_clear = g.n_clear;
   double *m = low + lane;
-  double priv[KPRIV > 0 ? KPRIV * kLowQ : 1];
-#define SG_LOW(k, j) (*(KPRIV > 0 ? &priv[(k) * kLowQ + (j)] : &m[((k) * kLowQ + (j)) * kWave]))
+  constexpr int Q = GEN ? kLowQ + 1 : kLowQ;   // the last one the gas absorption
+  double priv[KPRIV > 0 ? KPRIV * Q : 1];
+#define SG_LOW(k, j) (*(KPRIV > 0 ? &priv[(k) * Q + (j)] : &m[((k) * Q + (j)) * kWave]))
   double xsum = 0.0;
+  if (GEN)
+    row_gas<MIXED>(t, src, K, [&](int k) { return ic + min(p * K + k, nl - 1); },
+                   [&](int k, double v) { SG_LOW(k, kLowQ) = v; });
   for (int it = 0; it < n_it; it++) {
     const int j = it * NS + q, jc = j - n_clear;
     const bool clr = n_clear && j == 0, act = clr || (jc >= 0 && jc < g.n_s);
@@ -441,6 +475,7 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
       const int r = p * K + k;
       LayerIn x;
       load_layer<MIXED, GEN>(sj, ic + min(r, nl - 1), x);
+      if (GEN) x.kx = SG_LOW(k, kLowQ);
       Slab B;
       if (SOLAR) SG_LOW(k, 4) = f;
       row_layer<MIXED, GEN, SOLAR, false>(c, t, x, r < nl, f, B.T, B.Rt, B.Su, B.Sd);
@@ -647,9 +682,13 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
 }
 
 // LDS of one wave: the cloudy part's layers, the level sums and the column.
-template <int KMAX>
+// (general gas optics keep a cloudy layer's absorption beside its state)
+__host__ __device__ constexpr int solve_low(int opt) {
+  return kLowK * (opt == kOptPlain ? kLowQ : kLowQ + 1) * kWave;
+}
+template <int KMAX, int OPT>
 __host__ __device__ constexpr int solve_lds_doubles() {
-  return kLowK * kLowQ * kWave + (3 + kHotQ) * (KMAX * kRowLanes + 1);
+  return solve_low(OPT) + (3 + kHotQ) * (KMAX * kRowLanes + 1);
 }
 
 // Waves (64 threads each) of the calls of one build: W the work space.
@@ -659,7 +698,7 @@ __global__ __launch_bounds__(256, KMAX <= 9 ? 2 : 1) void b_solve_kernel(const B
   constexpr int lp = KMAX * kRowLanes + 1;
   const long long tot = h->tot[W];
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
-  double *low = lds + wv * solve_lds_doubles<KMAX>(), *acc = low + kLowK * kLowQ * kWave, *hot = acc + 3 * lp;
+  double *low = lds + wv * solve_lds_doubles<KMAX, OPT>(), *acc = low + solve_low(OPT), *hot = acc + 3 * lp;
   const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
   for (long long w0 = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w0 < tot; w0 += nw) {
     const int w = __builtin_amdgcn_readfirstlane((int)w0);
