@@ -5,9 +5,8 @@
 // Contraction of a*b+c into fused multiply-adds is fixed per function: off in
 // the FP64 forms of the reference's formulas (as the reference is built), on
 // within one expression in the mixed form's. Either way the code gives the
-// same bits wherever it is inlined, so a layer recomputed by the recomputing
-// solve tile, or solved in another kernel variant of a batch, equals its
-// first computation.
+// same bits wherever it is inlined, so a layer solved in another kernel
+// variant of a batch has the same coefficients.
 #pragma once
 
 #include <float.h>
@@ -422,8 +421,8 @@ SG_HD int lcg_step(int x) {
 
 // The mixed form's functions fuse a*b+c into FMAs within one expression
 // only (contract(on)): the backend then makes the same choice wherever the
-// code is inlined, so a layer recomputed by the recomputing solve tile gives
-// the bits of its first computation.
+// code is inlined, so a layer has the same coefficients in every kernel
+// variant.
 //
 // FP32 transcendentals of the mixed form: single hardware instructions on
 // the device (v_exp_f32 after the scaling, v_rcp_f32 then a multiply, about

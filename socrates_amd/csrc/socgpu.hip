@@ -4,13 +4,13 @@
 //   pack      (col,layer) lanes: caller arrays -> per-column layer records
 //   cldrange  (col,layer) lanes: cloud top/base over the call (cloud_gen)
 //   cloudgen  one wave per column, one lane per McICA sub-column
-//   band      one wave per (col,band): minor-gas equivalent extinction, solar
-//             direct-beam adjustment, Planck terms, grey and cloud optics
+//   band      16 lanes per column, the bands over the waves of a block: minor-gas
+//             equivalent extinction, solar direct-beam adjustment, Planck terms,
+//             grey and cloud optics
 //   solve     16 lanes per (col,g-point), over the layers: gas optics, single
 //             scattering, two-stream coefficients, sources and the column
 //             solve; g-point-weighted sums, one partial per wave
-//   finish    (col,level) lanes: sum of partials, Planck
-//   heating   (col,layer) lanes: heating rates
+//   finish    (col,level) lanes: sum of partials, Planck, heating rates
 // The spectral tables live on the device from registration on.
 #include <hip/hip_runtime.h>
 
@@ -879,7 +879,7 @@ __device__ __forceinline__ void overlap_body(const CallDims &d, const double *__
 // A batch is a list of radiation calls ("requests"), each with its own
 // spectrum, source, shape and options, packed into one launch sequence:
 // every kernel loops over the concatenated work of all requests and finds
-// the request of a work item by binary search over per-request starts. A
+// the request of a work item among the per-request starts (find_req). A
 // request's results are those of the same call made alone.
 // W_BAND + 2 i + gen: blocks (4 columns) of the band kernel by the build that
 // runs them, i = 0, 1, 2 for calls of up to kShortL layers, up to kLongL and
@@ -1592,6 +1592,10 @@ static void solve_layout(CallDims &d, const SgSpec &S, int max_waves = INT32_MAX
   d.nw = (rounds + d.rpw - 1) / d.rpw;
 }
 
+// Bytes of the fixed workspace a call takes: its descriptor, then its arrays.
+static size_t noalloc_offset();
+static size_t noalloc_bytes(const CallDims &d, const SgSpec &S);
+
 // Checks one call's arguments and resolves its options (socrates_set_control
 // defaults on the two-stream path); fills the request's shapes.
 static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, int precision,
@@ -1738,6 +1742,14 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
   }
   d.n_g = S.n_g;
   solve_layout(d, S);
+  // a call that fits the fixed workspace with fewer waves takes that many, in every
+  // entry point: the same sums, so the same bits, in all of them
+  if (noalloc_bytes(d, S) > kScratchBytes) {
+    CallDims least = d;
+    solve_layout(least, S, 1);
+    if (noalloc_bytes(least, S) <= kScratchBytes)
+      while (noalloc_bytes(d, S) > kScratchBytes) solve_layout(d, S, d.nw - 1);
+  }
   *entry = &e;
   *dout = d;
   return 0;
@@ -1809,6 +1821,20 @@ static void place_request(ReqDesc &q, const SgSpec &S, double *base, size_t *cur
 static size_t padded_ws_doubles(const CallDims &d, const SgSpec &S) {
   return request_ws_doubles(d, S) + 13 * 3;  // per-array alignment padding
 }
+
+// A one-call descriptor block written into device memory by a kernel that
+// takes it by value (the allocation-free entry point copies nothing across
+// with the runtime's copy engines: no staging buffer is involved).
+struct DescBlob {
+  BatchHdr h;
+  ReqDesc q;
+};
+
+static size_t noalloc_offset() { return (sizeof(DescBlob) + 255) & ~(size_t)255; }
+static size_t noalloc_bytes(const CallDims &d, const SgSpec &S) {
+  return noalloc_offset() + padded_ws_doubles(d, S) * 8;
+}
+static_assert(sizeof(DescBlob) % 8 == 0, "descriptor block is copied in 8-byte words");
 
 static void fill_desc(ReqDesc &q, const CallDims &d, const SpecEntry &e, const SocgpuRunesArgs &dv,
                       double *up, double *dn, double *dir, double *hr) {
@@ -1978,15 +2004,6 @@ int socgpu_runes(const char *spectrum_name, const SocgpuRunesArgs *a, SocgpuDiag
 
 namespace sg {
 
-// A one-call descriptor block written into device memory by a kernel that
-// takes it by value (the allocation-free entry point copies nothing across
-// with the runtime's copy engines: no staging buffer is involved).
-struct DescBlob {
-  BatchHdr h;
-  ReqDesc q;
-};
-static_assert(sizeof(DescBlob) % 8 == 0, "descriptor block is copied in 8-byte words");
-
 __global__ void b_desc_store_kernel(DescBlob v, DescBlob *dst) {
   const unsigned long long *src = (const unsigned long long *)&v;
   unsigned long long *d = (unsigned long long *)dst;
@@ -2014,9 +2031,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   CallDims d;
   if (int rc = resolve_request(spectrum_name, a, precision, &e, &d)) return rc;
   const SgSpec &S = e->host;
-  const size_t ws_off = (sizeof(DescBlob) + 255) & ~(size_t)255;
-  while (ws_off + padded_ws_doubles(d, S) * 8 > kScratchBytes && d.nw > 1) solve_layout(d, S, d.nw - 1);
-  const size_t need = ws_off + padded_ws_doubles(d, S) * 8;
+  const size_t need = noalloc_bytes(d, S);
   if (need > kScratchBytes)
     return fail(SOCGPU_ENOMEM, "call needs %zu bytes of workspace, above the %zu-byte fixed workspace of "
                                "socgpu_runes_noalloc (use socgpu_runes)", need, kScratchBytes);
@@ -2024,7 +2039,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   std::memset(&host, 0, sizeof host);
   fill_desc(host.q, d, *e, *a, diag->flux_up, diag->flux_down, diag->flux_direct, diag->heating_rate);
   size_t cursor = 0;
-  place_request(host.q, S, (double *)(g_ctx.scratch_dev + ws_off), &cursor);
+  place_request(host.q, S, (double *)(g_ctx.scratch_dev + noalloc_offset()), &cursor);
   long long w[kNWork];
   request_work(d, S, w);
   host.h.R = 1;
@@ -2434,6 +2449,7 @@ struct ServeItem {
   std::string name;
   size_t footprint = 0;
   int max_waves = INT32_MAX;  // 1 for a call whose footprint is above the budget otherwise
+                              // (its level sums are grouped otherwise then)
   std::chrono::steady_clock::time_point t_submit;
   int status = 1;  // 1 pending, 0 done, < 0 error
 };
