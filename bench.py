@@ -35,9 +35,8 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--precision mixed|fp
                       [--no-autotune] [--serve-seconds S] [--no-cpu-baseline]
                       [--no-ragged] [--no-c1] [--tile R,B,S]
 
---tile fixes the solve tile of the --precision form (recompute 0/1, waves
-per block, waves per SIMD) instead of the autotuned one; a profiled run uses
-it to count the instructions of a given tile.
+--tile fixes the solve tile of the --precision form (waves per block; the
+first and third number change nothing any more) instead of the autotuned one.
 """
 import argparse
 import json
@@ -71,7 +70,7 @@ HBM_PEAK = 8000.0                          # GB/s
 # FETCH_SIZE and WRITE_SIZE runs of this script on the same build, each scaled
 # by what the counter reads for a plain copy of known size; the summary, its
 # commands and the scale factors are in TRAFFIC_SOURCE
-TRAFFIC = {"mixed": 2.959e9, "fp64": 3.164e9}
+TRAFFIC = {"mixed": 0.410e9, "fp64": 0.528e9}
 TRAFFIC_SOURCE = "profiles/c2_solve_traffic.md"
 
 
