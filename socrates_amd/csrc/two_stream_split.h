@@ -9,6 +9,7 @@ struct TwoStreamArgs {
   const double *tau, *omega, *asym, *sec0, *finc_down, *finc_dir, *alb_diff, *alb_dir;
   const double *dpl, *dpl2, *dsurf, *adjust;
   double *fdir, *fup, *fdown;
+  long long first;   // the launch's first solve
 };
 
 // One lane per (term, profile), profile fastest, so every per-layer read and
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(kTsWaves *kWave) void two_stream_kernel(TwoStreamAr
   const int lane = threadIdx.x % kWave;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int P = a.P, L = a.L;
-  const long long n = (long long)P * a.G, idx = (long long)blockIdx.x * kWave + lane;
+  const long long n = (long long)P * a.G, idx = a.first + (long long)blockIdx.x * kWave + lane;
   const bool act = idx < n;
   // lanes past the last solve repeat it and store nothing
   const long long id = act ? idx : n - 1;
@@ -154,12 +155,19 @@ __global__ __launch_bounds__(kTsWaves *kWave) void two_stream_kernel(TwoStreamAr
   }
 }
 
+// A launch's work-items, 16 per solve, have to be fewer than 2^32, and the entry
+// point takes up to 2^31 solves: 2^27 of them (2^31 work-items) a launch.
+constexpr long long kTsPerLaunch = 1LL << 27;
+
 template <bool MIXED, bool SOLAR>
-static void two_stream_launch(const TwoStreamArgs &a, hipStream_t s) {
+static void two_stream_launch(TwoStreamArgs a, hipStream_t s) {
   const long long n = (long long)a.P * a.G;
-  const int blocks = (int)((n + kWave - 1) / kWave), T = kTsWaves * kWave;
-  if (a.L <= 3 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 3><<<blocks, T, 0, s>>>(a);
-  else if (a.L <= 6 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 6><<<blocks, T, 0, s>>>(a);
-  else if (a.L <= 9 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 9><<<blocks, T, 0, s>>>(a);
-  else two_stream_kernel<MIXED, SOLAR, 12><<<blocks, T, 0, s>>>(a);
+  constexpr int T = kTsWaves * kWave;
+  for (a.first = 0; a.first < n; a.first += kTsPerLaunch) {
+    const int blocks = (int)((std::min(n - a.first, kTsPerLaunch) + kWave - 1) / kWave);
+    if (a.L <= 3 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 3><<<blocks, T, 0, s>>>(a);
+    else if (a.L <= 6 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 6><<<blocks, T, 0, s>>>(a);
+    else if (a.L <= 9 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 9><<<blocks, T, 0, s>>>(a);
+    else two_stream_kernel<MIXED, SOLAR, 12><<<blocks, T, 0, s>>>(a);
+  }
 }

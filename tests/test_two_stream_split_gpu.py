@@ -24,3 +24,21 @@ def test_split_sizes_match_oracle(isolir, shape):
     _check(gpu, ref, _spread(tsc, ref) if isolir == 2 else None, "fp64 isolir=%d %s" % (isolir, shape))
     if isolir == 1:
         assert np.abs(np.asarray(gpu["flux_direct"]) - ref[2]).max() <= 1e-10 * np.abs(ref[2]).max()
+
+
+def test_more_solves_than_one_launch_holds():
+    """2^28 + 2^14 solves take three launches; every term has the same inputs,
+    so all have the bits of a one-term call."""
+    import torch
+    P, G = 1 << 14, (1 << 14) + 1
+    tsc = synth.make_two_stream_case(P, 2, 2, seed=79, n_term=1, omc_range=(-3.0, 0.0))
+    dev = {k: torch.as_tensor(v).cuda() if isinstance(v, np.ndarray) else v for k, v in tsc.items()}
+    torch.cuda.synchronize()   # the library has a stream of its own
+    one = R.two_stream_case(dev, "fp64")
+    many = dict(dev, n_term=G, **{k: dev[k].reshape(1, 2, P).repeat(G, 1, 1) for k in ("tau", "omega", "asymmetry")})
+    out = {k: torch.full((G, 3, P), float("nan"), dtype=torch.float64, device="cuda") for k in ("flux_up", "flux_down")}
+    out["flux_direct"] = None
+    torch.cuda.synchronize()
+    R.two_stream_case(many, "fp64", out=out)
+    for k in ("flux_up", "flux_down"):
+        assert bool((out[k] == one[k].reshape(1, 3, P)).all()), k
