@@ -13,10 +13,10 @@ struct TwoStreamArgs {
 };
 
 // One lane per (term, profile), profile fastest, so every per-layer read and
-// per-level write is coalesced; the layers of 64 such solves are split over the
-// kTsWaves waves of a block, at most KMAX consecutive ones each, whose state
-// stays in registers. Each wave composes its layers into one slab; the slabs
-// pass through LDS, every wave eliminates down those above its own to find the
+// per-level write is coalesced; the layers of COLS such solves are split over
+// kTsGroups groups of a block's lanes (a wave each, or half of one), at most KMAX
+// consecutive ones each, whose state stays in registers. Each group composes its
+// layers into one slab; the slabs pass through LDS, every group eliminates down those above its own to find the
 // state at its top, and after the local elimination the affine maps of the
 // waves below pass the upward flux back the same way. With the whole column in
 // one lane the elimination state went through lane-private memory (64 B a layer
@@ -24,22 +24,22 @@ struct TwoStreamArgs {
 // its layers.
 // (two_coeff, ir_source.F90:93-120, solar_source.F90:104-162, the surface source
 // of column_solver.F90:160-185, solver_homogen_direct.F90:93-127.)
-constexpr int kTsWaves = 16;
+constexpr int kTsGroups = 16;
 
-template <bool MIXED, bool SOLAR, int KMAX>
-__global__ __launch_bounds__(kTsWaves *kWave) void two_stream_kernel(TwoStreamArgs a) {
+template <bool MIXED, bool SOLAR, int KMAX, int COLS>
+__global__ __launch_bounds__(kTsGroups *COLS, 4) void two_stream_kernel(TwoStreamArgs a) {
 #pragma clang fp contract(on)
   constexpr int kQ = 6;
-  __shared__ double sh[kTsWaves][kQ][kWave];
-  const int lane = threadIdx.x % kWave;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  __shared__ double sh[kTsGroups][kQ][COLS];
+  const int lane = threadIdx.x % COLS;
+  const int wv = COLS == kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / COLS) : threadIdx.x / COLS;
   const int P = a.P, L = a.L;
-  const long long n = (long long)P * a.G, idx = a.first + (long long)blockIdx.x * kWave + lane;
+  const long long n = (long long)P * a.G, idx = a.first + (long long)blockIdx.x * COLS + lane;
   const bool act = idx < n;
   // lanes past the last solve repeat it and store nothing
   const long long id = act ? idx : n - 1;
   const int g = (int)(id / P), l = (int)(id - (long long)g * P);
-  const int K = (L + kTsWaves - 1) / kTsWaves, i0 = wv * K, nk = max(0, min(K, L - i0));
+  const int K = (L + kTsGroups - 1) / kTsGroups, i0 = wv * K, nk = max(0, min(K, L - i0));
   const int n_wave = (L + K - 1) / K;   // waves with layers
   const double sec0 = SOLAR ? a.sec0[l] : 1.0;
   const size_t t0 = (size_t)g * L * P + l, o0 = (size_t)g * (L + 1) * P + l;
@@ -159,15 +159,28 @@ __global__ __launch_bounds__(kTsWaves *kWave) void two_stream_kernel(TwoStreamAr
 // point takes up to 2^31 solves: 2^27 of them (2^31 work-items) a launch.
 constexpr long long kTsPerLaunch = 1LL << 27;
 
-template <bool MIXED, bool SOLAR>
-static void two_stream_launch(TwoStreamArgs a, hipStream_t s) {
+// Columns per block: 64, a wave per group of layers; 32, two groups per wave, where
+// that still gives every CU (256) at most one block, so that twice as many of them
+// work. FP64, a call in us with 64 and with 32 columns: solar 2997 solves of 137
+// layers 55 and 51, 8000 of 90 48 and 44, but 12288 of 60 43 and 45, where some CUs
+// have two blocks; infra-red 2997 of 137 50 and 44 (mixed 47 and 42); 65536 of 90
+// solar 119 and 121.
+constexpr long long kTsFew = 256 * 32;
+
+template <bool MIXED, bool SOLAR, int COLS>
+static void two_stream_cols(TwoStreamArgs a, hipStream_t s) {
   const long long n = (long long)a.P * a.G;
-  constexpr int T = kTsWaves * kWave;
+  constexpr int T = kTsGroups * COLS;
   for (a.first = 0; a.first < n; a.first += kTsPerLaunch) {
-    const int blocks = (int)((std::min(n - a.first, kTsPerLaunch) + kWave - 1) / kWave);
-    if (a.L <= 3 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 3><<<blocks, T, 0, s>>>(a);
-    else if (a.L <= 6 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 6><<<blocks, T, 0, s>>>(a);
-    else if (a.L <= 9 * kTsWaves) two_stream_kernel<MIXED, SOLAR, 9><<<blocks, T, 0, s>>>(a);
-    else two_stream_kernel<MIXED, SOLAR, 12><<<blocks, T, 0, s>>>(a);
+    const int blocks = (int)((std::min(n - a.first, kTsPerLaunch) + COLS - 1) / COLS);
+    if (a.L <= 3 * kTsGroups) two_stream_kernel<MIXED, SOLAR, 3, COLS><<<blocks, T, 0, s>>>(a);
+    else if (a.L <= 6 * kTsGroups) two_stream_kernel<MIXED, SOLAR, 6, COLS><<<blocks, T, 0, s>>>(a);
+    else if (a.L <= 9 * kTsGroups) two_stream_kernel<MIXED, SOLAR, 9, COLS><<<blocks, T, 0, s>>>(a);
+    else two_stream_kernel<MIXED, SOLAR, 12, COLS><<<blocks, T, 0, s>>>(a);
   }
+}
+template <bool MIXED, bool SOLAR>
+static void two_stream_launch(const TwoStreamArgs &a, hipStream_t s) {
+  if ((long long)a.P * a.G <= kTsFew) two_stream_cols<MIXED, SOLAR, 32>(a, s);
+  else two_stream_cols<MIXED, SOLAR, kWave>(a, s);
 }

@@ -26,6 +26,14 @@ def test_split_sizes_match_oracle(isolir, shape):
         assert np.abs(np.asarray(gpu["flux_direct"]) - ref[2]).max() <= 1e-10 * np.abs(ref[2]).max()
 
 
+@pytest.mark.parametrize("isolir", [1, 2])
+@pytest.mark.parametrize("shape", [(2731, 17, 3), (2048, 49, 4), (2731, 97, 3), (2731, 145, 3)])
+def test_block_widths_match_oracle(isolir, shape):
+    """8192 solves are the most that blocks of 32 columns take; 8193 fill 64-column
+    blocks but for one column in the last."""
+    test_split_sizes_match_oracle(isolir, shape)
+
+
 def test_more_solves_than_one_launch_holds():
     """2^28 + 2^14 solves take three launches; every term has the same inputs,
     so all have the bits of a one-term call."""
