@@ -120,7 +120,8 @@ struct CallDims {
   int mcica, mode;   // McICA on, sampling table (0 single, 1 optimal)
   int drop;          // droplet type index (0-based; the stratiform type)
   int n_g;           // major k-terms
-  int nw, rpw;       // waves per column of the solve, and rounds of g-points per wave
+  int nw, rpw;       // groups of a column's rounds of g-points, and rounds per group
+  int fold;          // one solve wave takes a column's groups in turn (else a wave each)
   int n_gen, n_fill, ipph, ioverlap;
   int triple, drop2; // triple-column representation; convective droplet type
   int raw_range;     // cloud range on the fractions as given (kernel-level cloud_gen)
@@ -143,6 +144,9 @@ struct CallDims {
   int n_aer;         // modal aerosols: modes (0: none; the general solve build)
   int ggen;          // the spectrum needs the general gas optics (band kernel build)
 };
+
+// Waves per column of the solve.
+__host__ __device__ inline int solve_waves(const CallDims &d) { return d.fold ? 1 : d.nw; }
 
 // Modal aerosol inputs of a call (device pointers: mixing ratio
 // [mode][layer][profile], absorption, scattering and asymmetry
@@ -775,15 +779,16 @@ __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm 
 // Sum of the per-wave partials, the Planck flux added back for the
 // infra-red (adjust_ir_radiance.F90:186-200, weight_band = 1), output in the
 // caller's [level][profile] layout. A column's partials come from its waves,
-// partial[col][wave], summed in wave order (the solve writes no direct flux for
-// an infra-red call: it is zero).
+// partial[col][wave], summed in wave order (one that has folded the column's
+// groups has summed them in that order; the solve writes no direct flux for an
+// infra-red call: it is zero).
 __device__ __forceinline__ void finish_body(const CallDims &d, const double *__restrict__ partial,
                                             const double *__restrict__ bandrec,
                                             const double *__restrict__ bandscal, int col, int lev,
                                             double &su, double &sd, double &sx) {
   const int L = d.L;
   su = 0.0; sd = 0.0; sx = 0.0;
-  const int nw = d.triple ? 1 : d.nw;
+  const int nw = d.triple ? 1 : solve_waves(d);
   const bool direct = d.triple || d.isolir == SOCGPU_SOURCE_SOLAR;
   for (int c = 0; c < nw; c++) {
     const double *o = partial + ((size_t)col * nw + c) * 3 * (L + 1);
@@ -887,11 +892,12 @@ __device__ __forceinline__ void overlap_body(const CallDims &d, const double *__
 // W_GEN counts the calls that need the general build of the triple-column solve.
 // W_SOLVE + 3 i + opt: waves of the solve, by the build that runs them (i = 0
 // for calls of up to kShortL layers, 1 up to kLongL; opt: kOptPlain, kOptGen,
-// kOptAer); W_SOLVE_ANY: calls of more layers
+// kOptAer); W_SOLVE_ANY: calls of more layers; W_SOLVE_FOLD: any call whose columns'
+// groups of g-points one wave takes in turn (CallDims::fold)
 // W_TSOLVE + 2 i + odd: columns of the triple-column solve, i = 0 and 1 as there,
 // 2 for calls of more layers (they differ in the LDS a block takes); odd: blocks
 // of three waves instead of two (an odd number of waves' k-terms)
-enum { W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_TOVL, W_TSOLVE,
+enum { W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_SOLVE_FOLD, W_TOVL, W_TSOLVE,
        W_PTILE = W_TSOLVE + 6, W_CCOL, W_FTILE, W_GEN, kNWork };
 
 struct ReqDesc {
@@ -1573,7 +1579,7 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
   return 0;
 }
 
-// Waves per column of the solve, each taking some rounds of 4 g-points. A wave
+// Groups of a column's rounds of 4 g-points, a solve wave each. A wave
 // first brings its column into LDS and at its end writes its partial sums, so it
 // should have several rounds; the chip holds 2048 waves of this kernel (two per
 // SIMD), so a call should have about as many. From 16 columns a wave has 3
@@ -1582,19 +1588,15 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
 // takes a wave per round, the shortest chain (4096 x 90 SW + LW, FP64: 1.20 ms
 // per step with 8192 waves per call, 1.18 ms with 2048 to 4096).
 constexpr long long kSolveWaves = 2048;
-// A call near a workspace limit takes fewer waves and so fewer partial sums
-// (max_waves), down to one per column.
-static void solve_layout(CallDims &d, const SgSpec &S, int max_waves = INT32_MAX) {
-  const int rounds = (S.n_g + kRows - 1) / kRows;
-  const long long most = std::min(max_waves, d.P < 16 ? rounds : (rounds + 2) / 3);
+// The groups fix the order in which the g-points are summed, so they are the same
+// wherever the call is made. Where a wave each needs too much room for the partial
+// sums (the fixed workspace, a serving budget), one wave takes them in turn (fold).
+static void solve_layout(CallDims &d, const SgSpec &S) {
+  const int rounds = (S.n_g + kRows - 1) / kRows, most = d.P < 16 ? rounds : (rounds + 2) / 3;
   const long long want = std::max<long long>(1, std::min<long long>(most, (kSolveWaves + d.P - 1) / d.P));
   d.rpw = (int)((rounds + want - 1) / want);
   d.nw = (rounds + d.rpw - 1) / d.rpw;
 }
-
-// Bytes of the fixed workspace a call takes: its descriptor, then its arrays.
-static size_t noalloc_offset();
-static size_t noalloc_bytes(const CallDims &d, const SgSpec &S);
 
 // Checks one call's arguments and resolves its options (socrates_set_control
 // defaults on the two-stream path); fills the request's shapes.
@@ -1742,14 +1744,6 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
   }
   d.n_g = S.n_g;
   solve_layout(d, S);
-  // a call that fits the fixed workspace with fewer waves takes that many, in every
-  // entry point: the same sums, so the same bits, in all of them
-  if (noalloc_bytes(d, S) > kScratchBytes) {
-    CallDims least = d;
-    solve_layout(least, S, 1);
-    if (noalloc_bytes(least, S) <= kScratchBytes)
-      while (noalloc_bytes(d, S) > kScratchBytes) solve_layout(d, S, d.nw - 1);
-  }
   *entry = &e;
   *dout = d;
   return 0;
@@ -1758,7 +1752,7 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
 // Per-wave partial sums of a request's solve.
 static size_t partial_doubles(const CallDims &d) {
   if (d.triple) return (size_t)d.P * 3 * (d.L + 1);
-  return (size_t)d.P * d.nw * 3 * (d.L + 1);
+  return (size_t)d.P * solve_waves(d) * 3 * (d.L + 1);
 }
 
 // Device workspace of one request, in doubles (8-byte units), and its work
@@ -1779,10 +1773,11 @@ static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]
   w[W_CG] = d.mcica ? P : 0;
   for (int k = 0; k < 6; k++) w[W_BAND + k] = 0;
   w[W_BAND + 2 * ((L > kShortL) + (L > kLongL)) + (d.ggen ? 1 : 0)] = band_quads(d);
-  for (int k = W_SOLVE; k <= W_SOLVE_ANY; k++) w[k] = 0;
+  for (int k = W_SOLVE; k <= W_SOLVE_FOLD; k++) w[k] = 0;
   if (!d.triple) {
     const int opt = d.n_aer > 0 ? kOptAer : (d.gen ? kOptGen : kOptPlain);
-    w[L > kLongL ? (int)W_SOLVE_ANY : W_SOLVE + 3 * (L > kShortL) + opt] = P * d.nw;
+    const int build = L > kLongL ? (int)W_SOLVE_ANY : W_SOLVE + 3 * (L > kShortL) + opt;
+    w[d.fold ? (int)W_SOLVE_FOLD : build] = P * solve_waves(d);
   }
   w[W_TOVL] = d.triple ? P * (L + 1) : 0;
   for (int k = 0; k < 6; k++) w[W_TSOLVE + k] = 0;
@@ -1830,10 +1825,6 @@ struct DescBlob {
   ReqDesc q;
 };
 
-static size_t noalloc_offset() { return (sizeof(DescBlob) + 255) & ~(size_t)255; }
-static size_t noalloc_bytes(const CallDims &d, const SgSpec &S) {
-  return noalloc_offset() + padded_ws_doubles(d, S) * 8;
-}
 static_assert(sizeof(DescBlob) % 8 == 0, "descriptor block is copied in 8-byte words");
 
 static void fill_desc(ReqDesc &q, const CallDims &d, const SpecEntry &e, const SocgpuRunesArgs &dv,
@@ -1906,6 +1897,7 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   SG_SOLVE(9, kOptGen, W_SOLVE + 3 + kOptGen)
   SG_SOLVE(9, kOptAer, W_SOLVE + 3 + kOptAer)
   SG_SOLVE(12, kOptAny, W_SOLVE_ANY)
+  SG_SOLVE(12, kOptAny, W_SOLVE_FOLD)
 #undef SG_SOLVE
   for (int w = W_TSOLVE; w < W_TSOLVE + 6; w++) {
     if (tot[w] == 0) continue;
@@ -2031,7 +2023,9 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   CallDims d;
   if (int rc = resolve_request(spectrum_name, a, precision, &e, &d)) return rc;
   const SgSpec &S = e->host;
-  const size_t need = noalloc_bytes(d, S);
+  const size_t ws_off = (sizeof(DescBlob) + 255) & ~(size_t)255;
+  d.fold = ws_off + padded_ws_doubles(d, S) * 8 > kScratchBytes;
+  const size_t need = ws_off + padded_ws_doubles(d, S) * 8;
   if (need > kScratchBytes)
     return fail(SOCGPU_ENOMEM, "call needs %zu bytes of workspace, above the %zu-byte fixed workspace of "
                                "socgpu_runes_noalloc (use socgpu_runes)", need, kScratchBytes);
@@ -2039,7 +2033,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   std::memset(&host, 0, sizeof host);
   fill_desc(host.q, d, *e, *a, diag->flux_up, diag->flux_down, diag->flux_direct, diag->heating_rate);
   size_t cursor = 0;
-  place_request(host.q, S, (double *)(g_ctx.scratch_dev + noalloc_offset()), &cursor);
+  place_request(host.q, S, (double *)(g_ctx.scratch_dev + ws_off), &cursor);
   long long w[kNWork];
   request_work(d, S, w);
   host.h.R = 1;
@@ -2142,10 +2136,10 @@ struct Resolved {
 };
 
 // Sizes of a batch (workspace, staging, outputs) without placing it; the
-// plan keeps the request list (with the clear-sky companions). max_waves: of
-// each caller's request, where given.
+// plan keeps the request list (with the clear-sky companions). fold: of each
+// caller's request, where given.
 static int plan_sizes(int n_caller, const SocgpuRequest *caller_req, int precision, std::vector<Resolved> &res,
-                      Plan &pl, const std::vector<int> *max_waves = nullptr) {
+                      Plan &pl, const std::vector<int> *fold = nullptr) {
   for (int i = 0; i < n_caller; i++)
     if (!caller_req[i].args || !caller_req[i].diag) return fail(SOCGPU_EINVAL, "request %d: null args or diag", i);
   if (int rc = expand_clear(n_caller, caller_req, pl.x)) return rc;
@@ -2157,7 +2151,7 @@ static int plan_sizes(int n_caller, const SocgpuRequest *caller_req, int precisi
   for (int i = 0; i < n; i++) {
     if (int rc = resolve_request(req[i].spectrum_name, req[i].args, precision, &res[i].e, &res[i].d))
       return rc;
-    if (max_waves) solve_layout(res[i].d, res[i].e->host, (*max_waves)[pl.x.caller[i]]);
+    if (fold) res[i].d.fold = (*fold)[pl.x.caller[i]];
     const CallDims &d = res[i].d;
     pl.ws_doubles += padded_ws_doubles(d, res[i].e->host);
     pl.in_bytes += stage_bytes(req[i].args, d.NB);
@@ -2448,8 +2442,7 @@ struct ServeItem {
   SocgpuDiag diag;
   std::string name;
   size_t footprint = 0;
-  int max_waves = INT32_MAX;  // 1 for a call whose footprint is above the budget otherwise
-                              // (its level sums are grouped otherwise then)
+  int fold = 0;  // 1 for a call whose footprint is above the budget otherwise (CallDims)
   std::chrono::steady_clock::time_point t_submit;
   int status = 1;  // 1 pending, 0 done, < 0 error
 };
@@ -2525,13 +2518,13 @@ static void serve_finish_slot(SocgpuServer *sv, ServeSlot &sl, int status) {
 static int serve_launch(SocgpuServer *sv, ServeSlot &sl) {
   const int n = (int)sl.items.size();
   std::vector<SocgpuRequest> req(n);
-  std::vector<int> max_waves(n);
+  std::vector<int> fold(n);
   for (int i = 0; i < n; i++) {
     req[i] = sl.items[i]->req;
-    max_waves[i] = sl.items[i]->max_waves;
+    fold[i] = sl.items[i]->fold;
   }
   std::vector<Resolved> res;
-  if (int rc = plan_sizes(n, req.data(), sv->cfg.precision, res, sl.plan, &max_waves)) return rc;
+  if (int rc = plan_sizes(n, req.data(), sv->cfg.precision, res, sl.plan, &fold)) return rc;
   const int nq = sl.plan.n();
   if (sl.ws.ensure(sl.plan.ws_doubles * 8) || sl.in_stage.ensure(sl.plan.in_bytes + 256) ||
       sl.out_stage.ensure(sl.plan.out_doubles * 8 + 64) || sl.desc.ensure(desc_bytes(nq)))
@@ -2663,12 +2656,12 @@ int socgpu_serve_submit(SocgpuServer *sv, const SocgpuRequest *request, long lon
     for (const SocgpuRequest &q : x.req) {
       if (int rc = resolve_request(q.spectrum_name, q.args, sv->cfg.precision, &e, &d)) return rc;
       it->footprint += footprint_bytes(q, d, e->host);
-      solve_layout(d, e->host, 1);
+      d.fold = 1;
       least += footprint_bytes(q, d, e->host);
     }
     if (it->footprint > sv->cfg.hbm_budget_bytes) {
       it->footprint = least;
-      it->max_waves = 1;
+      it->fold = 1;
     }
   }
   it->req = SocgpuRequest{it->name.c_str(), &it->args, &it->diag};

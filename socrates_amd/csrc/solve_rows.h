@@ -547,7 +547,7 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
   return dpp_or0<kBcast + 0>(xsum);
 }
 
-// The solves of one wave: rounds r0..r1-1 of the column's g-points, 4 a round.
+// The solves of one group of a column: some of its rounds of 4 g-points.
 // (mcica_sample.F90:453-930; monochromatic_radiance.F90:429-691;
 // mcica_column.F90:255-622; solver_homogen_direct.F90:93-127.)
 //
@@ -559,20 +559,20 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
 // a(i) X(i+1) + b(i) W with W the sum of the weights. (mcica_column.F90:266-298
 // recomputes those layers for every sample.)
 //
-// Output: partial[wave][up, down, direct][L+1] of this wave's weighted sums
-// (direct: solar calls only).
-template <bool MIXED, int OPT, bool SOLAR, int KMAX>
+// Output: partial[wave][up, down, direct][L+1] of the group's weighted sums
+// (direct: solar calls only), FOLD: added to those of the groups before it.
+template <bool MIXED, int OPT, bool SOLAR, int KMAX, bool FOLD>
 __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__restrict__ spec, int l_rayleigh,
                                            const double *__restrict__ colrec, const double *__restrict__ grec,
                                            const double *__restrict__ colscal, const double *__restrict__ bandrec,
                                            const double *__restrict__ bandscal, const double *__restrict__ c_sub,
                                            const double *__restrict__ cldopt, const double *__restrict__ aerrec,
-                                           double *__restrict__ partial, int wave, int lane, double *acc, int lp,
-                                           double *low, double *hot) {
+                                           double *__restrict__ partial, int wave, int group, int lane, double *acc,
+                                           int lp, double *low, double *hot) {
 #pragma clang fp contract(on)
   constexpr bool GEN = OPT != kOptPlain;
   const int L = d.L, NB = d.NB, G = spec->n_g;
-  const int col = wave / d.nw, part = wave - col * d.nw;
+  const int col = FOLD ? wave : wave / d.nw, part = FOLD ? group : wave - col * d.nw;
   const int s = lane % kRowLanes, row = lane / kRowLanes;
   const double *cs = colscal + (size_t)col * SG_NS;
   const double fc = d.mcica ? cs[SG_S_FC] : 0.0;
@@ -676,11 +676,14 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   double *out = partial + (size_t)wave * 3 * (L + 1);
-  for (int i = lane; i <= L; i += kWave) {
-    out[i] = acc[i];
-    out[(L + 1) + i] = acc[lp + i];
-    if (SOLAR) out[2 * (L + 1) + i] = acc[2 * lp + i];
-  }
+  const bool add = FOLD && group > 0;
+  for (int i = lane; i <= L; i += kWave)
+#pragma unroll
+    for (int v = 0; v < (SOLAR ? 3 : 2); v++) {
+      double *o = out + v * (L + 1) + i;
+      *o = add ? *o + acc[v * lp + i] : acc[v * lp + i];
+    }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
 }
 
 // LDS of one wave: the cloudy part's layers, the level sums and the column.
@@ -693,11 +696,15 @@ __host__ __device__ constexpr int solve_lds_doubles() {
   return solve_low(OPT) + (3 + kHotQ) * (KMAX * kRowLanes + 1);
 }
 
-// Waves (64 threads each) of the calls of one build: W the work space.
+// Waves (64 threads each) of the calls of one build: W the work space. In
+// W_SOLVE_FOLD a wave takes a column's groups in turn, and sums them in the order in
+// which the output kernel sums those of a wave each. (A loop over the groups in every
+// build took 0.5 to 2 % of a step.)
 template <bool MIXED, int OPT, int KMAX, int W>
 __global__ __launch_bounds__(256, KMAX <= 9 ? 2 : 1) void b_solve_kernel(const BatchHdr *h, const ReqDesc *rq) {
   extern __shared__ double lds[];
   constexpr int lp = KMAX * kRowLanes + 1;
+  constexpr bool FOLD = W == W_SOLVE_FOLD;
   const long long tot = h->tot[W];
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
   double *low = lds + wv * solve_lds_doubles<KMAX, OPT>(), *acc = low + solve_low(OPT), *hot = acc + 3 * lp;
@@ -707,13 +714,16 @@ __global__ __launch_bounds__(256, KMAX <= 9 ? 2 : 1) void b_solve_kernel(const B
     const int r = find_req(h, rq, W, w);
     const ReqDesc &q = rq[r];
     const int wave = w - (int)q.s[W];
-    if (q.d.isolir == SOCGPU_SOURCE_SOLAR)
-      solve_rows<MIXED, OPT, true, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
-                                         G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                         G(q.partial), wave, lane, acc, lp, low, hot);
-    else
-      solve_rows<MIXED, OPT, false, KMAX>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
-                                          G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                          G(q.partial), wave, lane, acc, lp, low, hot);
+    const int n = FOLD ? q.d.nw : 1;
+    for (int g = 0; g < n; g++) {
+      if (q.d.isolir == SOCGPU_SOURCE_SOLAR)
+        solve_rows<MIXED, OPT, true, KMAX, FOLD>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+                                                 G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
+                                                 G(q.partial), wave, g, lane, acc, lp, low, hot);
+      else
+        solve_rows<MIXED, OPT, false, KMAX, FOLD>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+                                                  G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
+                                                  G(q.partial), wave, g, lane, acc, lp, low, hot);
+    }
   }
 }
