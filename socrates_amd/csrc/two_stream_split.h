@@ -14,23 +14,24 @@ struct TwoStreamArgs {
 
 // One lane per (term, profile), profile fastest, so every per-layer read and
 // per-level write is coalesced; the layers of COLS such solves are split over
-// kTsGroups groups of a block's lanes (a wave each, or half of one), at most KMAX
-// consecutive ones each, whose state stays in registers. Each group composes its
-// layers into one slab; the slabs pass through LDS, every group eliminates down those above its own to find the
-// state at its top, and after the local elimination the affine maps of the
-// waves below pass the upward flux back the same way. With the whole column in
+// GROUPS groups of a block's lanes (a wave each, or half of one), at most KMAX
+// consecutive ones each, whose state stays in registers (128 a lane, which four waves
+// per SIMD allow: the solar builds of 9 layers spill 16 to 48 of them, 68 to 84 B a
+// lane, those of 12 80 to 110, up to 228 B, the infra-red ones of 12 40 to 48, up to
+// 84 B). Each group composes its layers into one slab; the slabs pass through LDS,
+// every group eliminates down those above its own to find the state at its top, and
+// after the local elimination the affine maps of the groups below pass the upward
+// flux back the same way. With the whole column in
 // one lane the elimination state went through lane-private memory (64 B a layer
 // beside the 48 B the solve has to move) and a small call was one chain of all
 // its layers.
 // (two_coeff, ir_source.F90:93-120, solar_source.F90:104-162, the surface source
 // of column_solver.F90:160-185, solver_homogen_direct.F90:93-127.)
-constexpr int kTsGroups = 16;
-
-template <bool MIXED, bool SOLAR, int KMAX, int COLS>
-__global__ __launch_bounds__(kTsGroups *COLS, 4) void two_stream_kernel(TwoStreamArgs a) {
+template <bool MIXED, bool SOLAR, int KMAX, int COLS, int GROUPS>
+__global__ __launch_bounds__(GROUPS *COLS, 4) void two_stream_kernel(TwoStreamArgs a) {
 #pragma clang fp contract(on)
   constexpr int kQ = 6;
-  __shared__ double sh[kTsGroups][kQ][COLS];
+  __shared__ double sh[GROUPS][kQ][COLS];
   const int lane = threadIdx.x % COLS;
   const int wv = COLS == kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / COLS) : threadIdx.x / COLS;
   const int P = a.P, L = a.L;
@@ -39,7 +40,7 @@ __global__ __launch_bounds__(kTsGroups *COLS, 4) void two_stream_kernel(TwoStrea
   // lanes past the last solve repeat it and store nothing
   const long long id = act ? idx : n - 1;
   const int g = (int)(id / P), l = (int)(id - (long long)g * P);
-  const int K = (L + kTsGroups - 1) / kTsGroups, i0 = wv * K, nk = max(0, min(K, L - i0));
+  const int K = (L + GROUPS - 1) / GROUPS, i0 = wv * K, nk = max(0, min(K, L - i0));
   const int n_wave = (L + K - 1) / K;   // waves with layers
   const double sec0 = SOLAR ? a.sec0[l] : 1.0;
   const size_t t0 = (size_t)g * L * P + l, o0 = (size_t)g * (L + 1) * P + l;
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(kTsGroups *COLS, 4) void two_stream_kernel(TwoStrea
       w2[k] = su;
       w3[k] = sd;
       const Slab B{o.T, o.R, o.R, su, sd};
-      S = k == 0 ? B : slab_add(S, B);
+      if (GROUPS > 1) S = k == 0 ? B : slab_add(S, B);
     }
   }
   sh[wv][0][lane] = S.T;
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(kTsGroups *COLS, 4) void two_stream_kernel(TwoStrea
   }
 }
 
-// A launch's work-items, 16 per solve, have to be fewer than 2^32, and the entry
+// A launch's work-items, up to 16 per solve, have to be fewer than 2^32, and the entry
 // point takes up to 2^31 solves: 2^27 of them (2^31 work-items) a launch.
 constexpr long long kTsPerLaunch = 1LL << 27;
 
@@ -167,20 +168,30 @@ constexpr long long kTsPerLaunch = 1LL << 27;
 // solar 119 and 121.
 constexpr long long kTsFew = 256 * 32;
 
-template <bool MIXED, bool SOLAR, int COLS>
-static void two_stream_cols(TwoStreamArgs a, hipStream_t s) {
+template <bool MIXED, bool SOLAR, int KMAX, int COLS, int GROUPS = 16>
+static void two_stream_run(TwoStreamArgs a, hipStream_t s) {
   const long long n = (long long)a.P * a.G;
-  constexpr int T = kTsGroups * COLS;
   for (a.first = 0; a.first < n; a.first += kTsPerLaunch) {
     const int blocks = (int)((std::min(n - a.first, kTsPerLaunch) + COLS - 1) / COLS);
-    if (a.L <= 3 * kTsGroups) two_stream_kernel<MIXED, SOLAR, 3, COLS><<<blocks, T, 0, s>>>(a);
-    else if (a.L <= 6 * kTsGroups) two_stream_kernel<MIXED, SOLAR, 6, COLS><<<blocks, T, 0, s>>>(a);
-    else if (a.L <= 9 * kTsGroups) two_stream_kernel<MIXED, SOLAR, 9, COLS><<<blocks, T, 0, s>>>(a);
-    else two_stream_kernel<MIXED, SOLAR, 12, COLS><<<blocks, T, 0, s>>>(a);
+    two_stream_kernel<MIXED, SOLAR, KMAX, COLS, GROUPS><<<blocks, GROUPS * COLS, 0, s>>>(a);
   }
 }
+template <bool MIXED, bool SOLAR, int COLS>
+static void two_stream_cols(const TwoStreamArgs &a, hipStream_t s) {
+  if (a.L <= 48) two_stream_run<MIXED, SOLAR, 3, COLS>(a, s);
+  else if (a.L <= 96) two_stream_run<MIXED, SOLAR, 6, COLS>(a, s);
+  else if (a.L <= 144) two_stream_run<MIXED, SOLAR, 9, COLS>(a, s);
+  else two_stream_run<MIXED, SOLAR, 12, COLS>(a, s);
+}
+
+// Few layers: one lane per solve up to 3, 4 groups up to 12, since 16 groups would be
+// idle for the most part. FP64, a call in us with 16 groups and so: solar 65536 x 16
+// solves of 2 layers 186 and 51, of 5 264 and 109, of 10 379 and 174; infra-red 113,
+// 146, 173 and 48, 80, 132; 4096 x 16 solar solves of 12 layers 48 and 39.
 template <bool MIXED, bool SOLAR>
 static void two_stream_launch(const TwoStreamArgs &a, hipStream_t s) {
-  if ((long long)a.P * a.G <= kTsFew) two_stream_cols<MIXED, SOLAR, 32>(a, s);
+  if (a.L <= 3) two_stream_run<MIXED, SOLAR, 3, kWave, 1>(a, s);
+  else if (a.L <= 12) two_stream_run<MIXED, SOLAR, 3, kWave, 4>(a, s);
+  else if ((long long)a.P * a.G <= kTsFew) two_stream_cols<MIXED, SOLAR, 32>(a, s);
   else two_stream_cols<MIXED, SOLAR, kWave>(a, s);
 }
