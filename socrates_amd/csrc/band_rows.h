@@ -236,7 +236,7 @@ __device__ __forceinline__ void band_rows(const ReqDesc &q, const CallDims &d, c
         for (int c = 0; c < KMAX; c++) {
           {
             const double e = exp(-kk[c] * x(2, layer(c)) * sec0);
-            double p = product_scan<1>(has(c) ? e : 1.0);
+            double p = product_scan<kRowLanes, 1>(has(c) ? e : 1.0, s);
             const double tot = dpp_or0<kBcast + 15>(p);
             if (c % 4 == 1 || c % 4 == 3) p = p * t02;
             if (c % 4 >= 2) p = p * p31;

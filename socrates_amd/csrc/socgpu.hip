@@ -891,13 +891,13 @@ __device__ __forceinline__ void overlap_body(const CallDims &d, const double *__
 // more; gen: the spectrum needs the general gas optics.
 // W_GEN counts the calls that need the general build of the triple-column solve.
 // W_SOLVE + 3 i + opt: waves of the solve, by the build that runs them (i = 0
-// for calls of up to kShortL layers, 1 up to kLongL; opt: kOptPlain, kOptGen,
+// for calls of up to kFewL layers, 1 up to kShortL, 2 up to kLongL; opt: kOptPlain, kOptGen,
 // kOptAer); W_SOLVE_ANY: calls of more layers; W_SOLVE_FOLD: any call whose columns'
 // groups of g-points one wave takes in turn (CallDims::fold)
 // W_TSOLVE + 2 i + odd: columns of the triple-column solve, i = 0 and 1 as there,
 // 2 for calls of more layers (they differ in the LDS a block takes); odd: blocks
 // of three waves instead of two (an odd number of waves' k-terms)
-enum { W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 6, W_SOLVE_FOLD, W_TOVL, W_TSOLVE,
+enum { W_CG, W_BAND, W_SOLVE = W_BAND + 6, W_SOLVE_ANY = W_SOLVE + 9, W_SOLVE_FOLD, W_TOVL, W_TSOLVE,
        W_PTILE = W_TSOLVE + 6, W_CCOL, W_FTILE, W_GEN, kNWork };
 
 struct ReqDesc {
@@ -912,7 +912,8 @@ struct ReqDesc {
   double *ovl, *tws;            // triple column: overlap coefficients, solve workspace
   double *aerrec;               // modal aerosols: clear-air scattering, moment products
   int *krange;
-  long long s[kNWork];          // first work item of this request in each space
+  int s[kNWork];                // first work item of this request in each space (fewer than
+                                // 2^31: the records behind them would not fit the device)
 };
 
 // err: 0, or 1 + the (descriptor-order) index of a request whose input the
@@ -1579,7 +1580,7 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
   return 0;
 }
 
-// Groups of a column's rounds of 4 g-points, a solve wave each. A wave
+// Groups of a column's rounds of 4 (few layers: 16) g-points, a solve wave each. A wave
 // first brings its column into LDS and at its end writes its partial sums, so it
 // should have several rounds; the chip holds 2048 waves of this kernel (two per
 // SIMD), so a call should have about as many. From 16 columns a wave has 3
@@ -1592,7 +1593,8 @@ constexpr long long kSolveWaves = 2048;
 // wherever the call is made. Where a wave each needs too much room for the partial
 // sums (the fixed workspace, a serving budget), one wave takes them in turn (fold).
 static void solve_layout(CallDims &d, const SgSpec &S) {
-  const int rounds = (S.n_g + kRows - 1) / kRows, most = d.P < 16 ? rounds : (rounds + 2) / 3;
+  const int per = kWave / (d.L <= kFewL ? kFewLanes : kRowLanes), rounds = (S.n_g + per - 1) / per;
+  const int most = d.P < 16 ? rounds : (rounds + 2) / 3;
   const long long want = std::max<long long>(1, std::min<long long>(most, (kSolveWaves + d.P - 1) / d.P));
   d.rpw = (int)((rounds + want - 1) / want);
   d.nw = (rounds + d.rpw - 1) / d.rpw;
@@ -1776,8 +1778,8 @@ static void request_work(const CallDims &d, const SgSpec &S, long long w[kNWork]
   for (int k = W_SOLVE; k <= W_SOLVE_FOLD; k++) w[k] = 0;
   if (!d.triple) {
     const int opt = d.n_aer > 0 ? kOptAer : (d.gen ? kOptGen : kOptPlain);
-    const int build = L > kLongL ? (int)W_SOLVE_ANY : W_SOLVE + 3 * (L > kShortL) + opt;
-    w[d.fold ? (int)W_SOLVE_FOLD : build] = P * solve_waves(d);
+    const int build = L > kLongL ? (int)W_SOLVE_ANY : W_SOLVE + 3 * ((L > kFewL) + (L > kShortL)) + opt;
+    w[d.fold && L > kFewL ? (int)W_SOLVE_FOLD : build] = P * solve_waves(d);
   }
   w[W_TOVL] = d.triple ? P * (L + 1) : 0;
   for (int k = 0; k < 6; k++) w[W_TSOLVE + k] = 0;
@@ -1885,19 +1887,23 @@ static int launch_batch(const BatchHdr *hdr, const ReqDesc *rq, const long long 
   if (ev_a) HIPCHK(hipEventRecord(ev_a, s));
   const SocgpuTile &tile = g_tile[precision == SOCGPU_MIXED ? 1 : 0];
   const int wpb = tile.waves_per_block;
-#define SG_SOLVE(KMAX, OPT, W)                                                                               \
-  if (tot[W] > 0) {                                                                                         \
-    auto *k = precision == SOCGPU_MIXED ? b_solve_kernel<true, OPT, KMAX, W> : b_solve_kernel<false, OPT, KMAX, W>; \
-    k<<<blocks(tot[W], wpb), wpb * kWave, wpb * solve_lds_doubles<KMAX, OPT>() * 8, s>>>(hdr, rq);                \
+#define SG_SOLVE(KMAX, OPT, LN, W)                                                                             \
+  if (tot[W] > 0) {                                                                                           \
+    auto *k = precision == SOCGPU_MIXED ? b_solve_kernel<true, OPT, KMAX, LN, W>                               \
+                                        : b_solve_kernel<false, OPT, KMAX, LN, W>;                             \
+    k<<<blocks(tot[W], wpb), wpb * kWave, wpb * solve_lds_doubles<KMAX, OPT, LN>() * 8, s>>>(hdr, rq);          \
   }
-  SG_SOLVE(6, kOptPlain, W_SOLVE + kOptPlain)
-  SG_SOLVE(6, kOptGen, W_SOLVE + kOptGen)
-  SG_SOLVE(6, kOptAer, W_SOLVE + kOptAer)
-  SG_SOLVE(9, kOptPlain, W_SOLVE + 3 + kOptPlain)
-  SG_SOLVE(9, kOptGen, W_SOLVE + 3 + kOptGen)
-  SG_SOLVE(9, kOptAer, W_SOLVE + 3 + kOptAer)
-  SG_SOLVE(12, kOptAny, W_SOLVE_ANY)
-  SG_SOLVE(12, kOptAny, W_SOLVE_FOLD)
+  SG_SOLVE(6, kOptPlain, kFewLanes, W_SOLVE + kOptPlain)
+  SG_SOLVE(6, kOptGen, kFewLanes, W_SOLVE + kOptGen)
+  SG_SOLVE(6, kOptAer, kFewLanes, W_SOLVE + kOptAer)
+  SG_SOLVE(6, kOptPlain, kRowLanes, W_SOLVE + 3 + kOptPlain)
+  SG_SOLVE(6, kOptGen, kRowLanes, W_SOLVE + 3 + kOptGen)
+  SG_SOLVE(6, kOptAer, kRowLanes, W_SOLVE + 3 + kOptAer)
+  SG_SOLVE(9, kOptPlain, kRowLanes, W_SOLVE + 6 + kOptPlain)
+  SG_SOLVE(9, kOptGen, kRowLanes, W_SOLVE + 6 + kOptGen)
+  SG_SOLVE(9, kOptAer, kRowLanes, W_SOLVE + 6 + kOptAer)
+  SG_SOLVE(12, kOptAny, kRowLanes, W_SOLVE_ANY)
+  SG_SOLVE(12, kOptAny, kRowLanes, W_SOLVE_FOLD)
 #undef SG_SOLVE
   for (int w = W_TSOLVE; w < W_TSOLVE + 6; w++) {
     if (tot[w] == 0) continue;
@@ -2133,6 +2139,7 @@ static int batch_err(const Plan &pl, int err) {
 struct Resolved {
   SpecEntry *e;
   CallDims d;
+  long long w[kNWork];  // work items
 };
 
 // Sizes of a batch (workspace, staging, outputs) without placing it; the
@@ -2156,9 +2163,8 @@ static int plan_sizes(int n_caller, const SocgpuRequest *caller_req, int precisi
     pl.ws_doubles += padded_ws_doubles(d, res[i].e->host);
     pl.in_bytes += stage_bytes(req[i].args, d.NB);
     if (!req[i].diag->l_outputs_on_device) pl.out_doubles += (size_t)d.P * (3 * (d.L + 1) + d.L) + 16;
-    long long w[kNWork];
-    request_work(d, res[i].e->host, w);
-    for (int k = 0; k < kNWork; k++) pl.need[k] += w[k];
+    request_work(d, res[i].e->host, res[i].w);
+    for (int k = 0; k < kNWork; k++) pl.need[k] += res[i].w[k];
   }
   return 0;
 }
@@ -2207,11 +2213,9 @@ static int plan_place(const std::vector<Resolved> &res, Plan &pl, double *ws, ch
     ReqDesc &q = pl.rq[j];
     fill_desc(q, d, e, dv, up, dn, dir, hr);
     place_request(q, e.host, ws, &ws_cur);
-    long long w[kNWork];
-    request_work(d, e.host, w);
     for (int k = 0; k < kNWork; k++) {
-      q.s[k] = start[k];
-      start[k] += w[k];
+      q.s[k] = (int)start[k];
+      start[k] += res[i].w[k];
     }
   }
   for (int k = 0; k < kNWork; k++) pl.h.tot[k] = start[k];

@@ -3,9 +3,9 @@
 // layer_coef*) and lane exchanges it uses.
 //
 // A solve is one (column, g-point) clear or McICA profile: the two-stream
-// system of L layers. 16 consecutive lanes (a DPP row) share one solve, each
-// lane taking K = ceil(layers / 16) consecutive layers in registers, so a
-// wave holds 4 solves of one column. The layers' coefficients are independent
+// system of L layers. LN consecutive lanes share one solve, 16 (a DPP row) or, for
+// calls of few layers, 4 (kFewL), each lane taking K = ceil(layers / LN) consecutive
+// layers in registers, so a wave holds 4 or 16 solves of one column. The layers' coefficients are independent
 // and are most of the work; the elimination down the column and the
 // back-substitution up it are recurrences, made parallel across the lanes:
 //  - each lane composes its layers into one slab (transmission, reflection
@@ -34,6 +34,11 @@ constexpr int kHotQ = 7;                      // column record slots a wave keep
 // gases without aerosols; any gas scaling and treatment of scattering; that with
 // aerosols. Calls of more layers than kLongL are few: one build for all optics.
 constexpr int kShortL = 6 * kRowLanes, kLongL = 9 * kRowLanes;
+// Calls of few layers (also three builds by optics): 16 lanes would be idle for the
+// most part. Call of 16384 columns in us, FP64 solar, with 16 lanes per solve and with
+// 4: 2 layers clear 433 and 285, 5 layers all-sky 752 and 438, 24 all-sky 922 and 704;
+// infra-red, 24 all-sky 1125 and 881. (One column of 20 layers 145 and 149.)
+constexpr int kFewLanes = 4, kFewL = 6 * kFewLanes;
 enum { kOptPlain, kOptGen, kOptAer, kOptAny };
 
 // v of the lane CTRL selects, 0 where there is none; and with 1 there.
@@ -48,6 +53,32 @@ __device__ __forceinline__ double dpp_or1(double v) { return dpp_f64<CTRL, 0xf>(
 
 // row_shr:N (from the lane N below), row_shl:N (N above), row_newbcast:N
 constexpr int kShr = 0x110, kShl = 0x100, kBcast = 0x150, kXor1 = 0xB1;
+
+// v of the lane N below or N above in the group of LN lanes, s the lane's place in
+// it; 0 (or 1) where there is none; and v of the group's first or last lane.
+template <int LN, int N>
+__device__ __forceinline__ double below0(double v, int s) {
+  const double x = dpp_or0<kShr + N>(v);
+  return LN == kRowLanes || s >= N ? x : 0.0;
+}
+template <int LN, int N>
+__device__ __forceinline__ double below1(double v, int s) {
+  const double x = dpp_or1<kShr + N>(v);
+  return LN == kRowLanes || s >= N ? x : 1.0;
+}
+template <int LN, int N>
+__device__ __forceinline__ double above0(double v, int s) {
+  const double x = dpp_or0<kShl + N>(v);
+  return LN == kRowLanes || s + N < LN ? x : 0.0;
+}
+template <int LN>
+__device__ __forceinline__ double of_first(double v) {
+  return LN == kRowLanes ? dpp_or0<kBcast + 0>(v) : dpp_move<0x00>(v);   // quad_perm [0, 0, 0, 0]
+}
+template <int LN>
+__device__ __forceinline__ double of_last(double v) {
+  return LN == kRowLanes ? dpp_or0<kBcast + 15>(v) : dpp_move<0xFF>(v);  // quad_perm [3, 3, 3, 3]
+}
 
 // 1 / x of a denominator in (0, 1]: the hardware estimate and two Newton steps
 // (within an ulp or two).
@@ -87,81 +118,99 @@ __device__ __forceinline__ void slab_below(double Rb, double Sd, const Slab &B, 
   sd = B.Sd + tb * (Sd + Rb * B.Su);
 }
 
-// One step of the prefix scan of slabs: the slab N lanes below in the row
+// One step of the prefix scan of slabs: the slab N lanes below in the group
 // (zeros where there is none: such a lane's slab already starts at the top of
 // the scanned layers, its state is absolute and only Rb and Sd of it are
 // used again).
-template <int N>
-__device__ __forceinline__ void slab_step(Slab &S) {
+template <int LN, int N>
+__device__ __forceinline__ void slab_step(Slab &S, int s) {
   Slab A;
-  A.T = dpp_or0<kShr + N>(S.T);
-  A.Rt = dpp_or0<kShr + N>(S.Rt);
-  A.Rb = dpp_or0<kShr + N>(S.Rb);
-  A.Su = dpp_or0<kShr + N>(S.Su);
-  A.Sd = dpp_or0<kShr + N>(S.Sd);
+  A.T = below0<LN, N>(S.T, s);
+  A.Rt = below0<LN, N>(S.Rt, s);
+  A.Rb = below0<LN, N>(S.Rb, s);
+  A.Su = below0<LN, N>(S.Su, s);
+  A.Sd = below0<LN, N>(S.Sd, s);
   S = slab_add(A, S);
 }
 
-// The scan over a row whose consecutive slabs lie NS lanes apart.
-template <int NS>
-__device__ __forceinline__ void slab_scan(Slab &S) {
-  if (NS == 1) slab_step<1>(S);
-  slab_step<2>(S);
-  slab_step<4>(S);
+// The scan over a group whose consecutive slabs lie NS lanes apart.
+template <int LN, int NS>
+__device__ __forceinline__ void slab_scan(Slab &S, int s) {
+  if (NS == 1) slab_step<LN, 1>(S, s);
+  if (LN == kRowLanes) {
+    slab_step<LN, 2>(S, s);
+    slab_step<LN, 4>(S, s);
+  }
   double rb, sd;
-  slab_below(dpp_or0<kShr + 8>(S.Rb), dpp_or0<kShr + 8>(S.Sd), S, rb, sd);
+  slab_below(below0<LN, LN / 2>(S.Rb, s), below0<LN, LN / 2>(S.Sd, s), S, rb, sd);
   S.Rb = rb;
   S.Sd = sd;
 }
 
-template <int NS>
-__device__ __forceinline__ double product_scan(double p) {
-  if (NS == 1) p = p * dpp_or1<kShr + 1>(p);
-  p = p * dpp_or1<kShr + 2>(p);
-  p = p * dpp_or1<kShr + 4>(p);
-  p = p * dpp_or1<kShr + 8>(p);
+template <int LN, int NS>
+__device__ __forceinline__ double product_scan(double p, int s) {
+  if (NS == 1) p = p * below1<LN, 1>(p, s);
+  p = p * below1<LN, 2>(p, s);
+  if (LN == kRowLanes) {
+    p = p * below1<LN, 4>(p, s);
+    p = p * below1<LN, 8>(p, s);
+  }
   return p;
 }
 
-// Suffix scan of the affine maps x -> A x + C, the last of the row's maps
+// Suffix scan of the affine maps x -> A x + C, the last of the group's maps
 // being absolute (A unused).
-template <int N>
-__device__ __forceinline__ void affine_up_step(double &A, double &C) {
+template <int LN, int N>
+__device__ __forceinline__ void affine_up_step(double &A, double &C, int s) {
 #pragma clang fp contract(on)
-  const double A1 = dpp_or0<kShl + N>(A), C1 = dpp_or0<kShl + N>(C);
+  const double A1 = above0<LN, N>(A, s), C1 = above0<LN, N>(C, s);
   C = A * C1 + C;
   A = A * A1;
 }
-template <int NS>
-__device__ __forceinline__ void affine_up_scan(double A, double &C) {
+template <int LN, int NS>
+__device__ __forceinline__ void affine_up_scan(double A, double &C, int s) {
 #pragma clang fp contract(on)
-  if (NS == 1) affine_up_step<1>(A, C);
-  affine_up_step<2>(A, C);
-  affine_up_step<4>(A, C);
-  C = A * dpp_or0<kShl + 8>(C) + C;
+  if (NS == 1) affine_up_step<LN, 1>(A, C, s);
+  if (LN == kRowLanes) {
+    affine_up_step<LN, 2>(A, C, s);
+    affine_up_step<LN, 4>(A, C, s);
+  }
+  C = A * above0<LN, LN / 2>(C, s) + C;
 }
 
-// The same down the row, the first of its maps being absolute.
-template <int N>
-__device__ __forceinline__ void affine_down_step(double &A, double &C) {
+// The same down the group, the first of its maps being absolute.
+template <int LN, int N>
+__device__ __forceinline__ void affine_down_step(double &A, double &C, int s) {
 #pragma clang fp contract(on)
-  const double A1 = dpp_or0<kShr + N>(A), C1 = dpp_or0<kShr + N>(C);
+  const double A1 = below0<LN, N>(A, s), C1 = below0<LN, N>(C, s);
   C = A * C1 + C;
   A = A * A1;
 }
-__device__ __forceinline__ void affine_down_scan(double A, double &C) {
+template <int LN>
+__device__ __forceinline__ void affine_down_scan(double A, double &C, int s) {
 #pragma clang fp contract(on)
-  affine_down_step<1>(A, C);
-  affine_down_step<2>(A, C);
-  affine_down_step<4>(A, C);
-  C = A * dpp_or0<kShr + 8>(C) + C;
+  affine_down_step<LN, 1>(A, C, s);
+  if (LN == kRowLanes) {
+    affine_down_step<LN, 2>(A, C, s);
+    affine_down_step<LN, 4>(A, C, s);
+  }
+  C = A * below0<LN, LN / 2>(C, s) + C;
 }
 
-// Four values per lane summed over the wave's 4 rows, lane by lane: row r
-// gets the sum of value row_value(r).
+// Four values per lane summed over the wave's solves, lane by lane of their
+// groups: row r gets the sum of value row_value(r) (groups of 4: each of its quads;
+// the first adds it to the level sums, leads).
+template <int LN>
 __device__ __forceinline__ double sum_rows(double v0, double v1, double v2, double v3) {
-  return swap16_sum(swap32_sum(v0, v1), swap32_sum(v2, v3));
+  double z = swap16_sum(swap32_sum(v0, v1), swap32_sum(v2, v3));
+  if (LN != kRowLanes) {
+    z = z + dpp_move<0x128>(z);   // row_ror:8
+    z = z + dpp_move<0x124>(z);   // row_ror:4
+  }
+  return z;
 }
+template <int LN>
+__device__ __forceinline__ bool leads(int lane) { return LN == kRowLanes || lane % kRowLanes < LN; }
 __device__ __forceinline__ int row_value(int row) { return (row & 1) * 2 + (row >> 1); }
 
 // A wave's level sums in LDS: [up, down, direct][lp], each added to by one
@@ -206,15 +255,16 @@ __device__ __forceinline__ void row_elim(double T, double R, double su, double s
   rho = rho_n;
 }
 
-// The layers of a run of n that lane s of its row takes: K on the first lanes,
+// The layers of a run of n that lane s of its group takes: K on the first lanes,
 // K - 1 on the others, from layer i0.
 struct RowMap {
   int K, i0;
   bool full;
   __device__ __forceinline__ bool has(int k) const { return k + 1 < K || full; }
 };
+template <int LN>
 __device__ __forceinline__ RowMap row_map(int n, int s) {
-  const int K = (n + kRowLanes - 1) / kRowLanes, rem = n - kRowLanes * (K - 1);
+  const int K = (n + LN - 1) / LN, rem = n - LN * (K - 1);
   return RowMap{K, s * (K - 1) + min(s, rem), s < rem};
 }
 
@@ -270,11 +320,11 @@ __device__ __forceinline__ void row_gas_clear(const SgTerm &t, const LaneSrc &sr
 
 // Down the first n layers of the column, all clear: eliminates the lane's K
 // layers; (rho, dn, fdir) become those at the bottom of the lane's layers
-// (lane 15's: at level n). Adds the direct flux at the levels above n, with
+// (the last lane's: at level n). Adds the direct flux at the levels above n, with
 // weight W, to acc.
-template <bool MIXED, bool GEN, bool SOLAR, int KMAX>
+template <bool MIXED, bool GEN, bool SOLAR, int KMAX, int LN>
 __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, const LaneSrc &src, int n,
-                                         const RowMap &mp, int s, int row, double finc, double W,
+                                         const RowMap &mp, int s, double finc, double W,
                                          RowState<KMAX, false> &w, double &rho, double &dn, double &fdir, double *acc,
                                          int lp, double *low, int lane) {
 #pragma clang fp contract(on)
@@ -298,11 +348,11 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
   }
   double F = 1.0;
   if (SOLAR) {
-    F = finc * dpp_or1<kShr + 1>(product_scan<1>(f));
+    F = finc * below1<LN, 1>(product_scan<LN, 1>(f, s), s);
     S.Su = S.Su * F;
     S.Sd = S.Sd * F;
     const double WF = W * F;
-    const int v = row_value(row);
+    const int v = row_value(lane / kRowLanes);
 #pragma unroll
     for (int k0 = 0; k0 < KMAX; k0 += 4) {
       if (k0 < mp.K) {
@@ -310,16 +360,16 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
 #pragma unroll
         for (int j = 0; j < 4; j++)
           d[j] = (k0 + j < KMAX && k0 + j < mp.K) ? WF * fr[k0 + j < KMAX ? k0 + j : 0] : 0.0;
-        const double z = sum_rows(d[0], d[1], d[2], d[3]);
+        const double z = sum_rows<LN>(d[0], d[1], d[2], d[3]);
         const int k = k0 + v;
-        if (k < mp.K && mp.has(k)) acc_add(acc + 2 * lp + mp.i0 + k, z);
+        if (k < mp.K && mp.has(k) && leads<LN>(lane)) acc_add(acc + 2 * lp + mp.i0 + k, z);
       }
     }
   }
   if (s == 0) S.Sd = S.Sd + S.T * finc;
-  slab_scan<1>(S);
-  rho = dpp_or0<kShr + 1>(S.Rb);
-  dn = dpp_or0<kShr + 1>(S.Sd);
+  slab_scan<LN, 1>(S, s);
+  rho = below0<LN, 1>(S.Rb, s);
+  dn = below0<LN, 1>(S.Sd, s);
   if (s == 0) dn = finc;
 #pragma unroll
   for (int k = 0; k < KMAX; k++) {
@@ -337,7 +387,7 @@ __device__ __forceinline__ void row_down(const LaneCtx &c, const SgTerm &t, cons
 
 // row_down of infra-red layers that do not scatter, FP64 form: the flux goes
 // down them by one affine recurrence, and fu(top) = T fu(bottom) + su.
-template <bool GEN, int KMAX>
+template <bool GEN, int KMAX, int LN>
 __device__ __forceinline__ void row_down_absorb(const LaneCtx &c, const SgTerm &t, const LaneSrc &src, int n,
                                                 const RowMap &mp, int s, double finc, RowState<KMAX, true> &w,
                                                 double &dn, double *low, int lane) {
@@ -363,8 +413,8 @@ __device__ __forceinline__ void row_down_absorb(const LaneCtx &c, const SgTerm &
     }
   }
   if (s == 0) C = A * finc + C;
-  affine_down_scan(A, C);
-  dn = dpp_or0<kShr + 1>(C);
+  affine_down_scan<LN>(A, C, s);
+  dn = below0<LN, 1>(C, s);
   if (s == 0) dn = finc;
 #pragma unroll
   for (int k = 0; k < KMAX; k++) {
@@ -379,8 +429,8 @@ __device__ __forceinline__ void row_down_absorb(const LaneCtx &c, const SgTerm &
 // Up the same layers: X the (weighted) upward flux at level n, W the weight
 // of the sources; adds the weighted upward and downward fluxes of the levels
 // above n to acc.
-template <int KMAX, bool ABS>
-__device__ __forceinline__ void row_up(const RowMap &mp, int s, int row, double X, double W,
+template <int KMAX, bool ABS, int LN>
+__device__ __forceinline__ void row_up(const RowMap &mp, int s, int lane, double X, double W,
                                        const RowState<KMAX, ABS> &w, double *acc, int lp) {
 #pragma clang fp contract(on)
   double A = 1.0, C = 0.0;
@@ -392,11 +442,11 @@ __device__ __forceinline__ void row_up(const RowMap &mp, int s, int row, double 
     }
   }
   C = C * W;
-  if (s == kRowLanes - 1) C = A * X + C;
-  affine_up_scan<1>(A, C);
-  double x = dpp_or0<kShl + 1>(C);
-  if (s == kRowLanes - 1) x = X;
-  const int v = row_value(row);
+  if (s == LN - 1) C = A * X + C;
+  affine_up_scan<LN, 1>(A, C, s);
+  double x = above0<LN, 1>(C, s);
+  if (s == LN - 1) x = X;
+  const int v = row_value(lane / kRowLanes);
 #pragma unroll
   for (int k0 = ((KMAX - 1) / 2) * 2; k0 >= 0; k0 -= 2) {
     if (k0 < mp.K) {
@@ -410,9 +460,9 @@ __device__ __forceinline__ void row_up(const RowMap &mp, int s, int row, double 
           dw[j] = ABS ? w.dn[k < KMAX ? k : 0] * W : w.rho[ABS ? 0 : (k < KMAX ? k : 0)] * x + w.dn[k < KMAX ? k : 0] * W;
         }
       }
-      const double z = sum_rows(up[0], dw[0], up[1], dw[1]);
+      const double z = sum_rows<LN>(up[0], dw[0], up[1], dw[1]);
       const int k = k0 + (v >> 1);
-      if (k < mp.K && mp.has(k)) acc_add(acc + (v & 1) * lp + mp.i0 + k, z);
+      if (k < mp.K && mp.has(k) && leads<LN>(lane)) acc_add(acc + (v & 1) * lp + mp.i0 + k, z);
     }
   }
 }
@@ -442,18 +492,18 @@ struct RowItem {
 // to kLowK layers per lane), or for cloud that reaches higher lane-private
 // memory (KPRIV layers per lane). Adds the weighted fluxes of levels ic..L to
 // acc; returns the weighted upward flux at level ic.
-template <bool MIXED, bool GEN, bool SOLAR, int NS, int KPRIV>
+template <bool MIXED, bool GEN, bool SOLAR, int NS, int KPRIV, int LN>
 __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, const LaneSrc &src,
                                              const SgSpec *__restrict__ spec, int mode, const RowItem &g, int n_it,
-                                             int L, int ic, int s, int row, int lane, double rho_ic, double dn_ic,
+                                             int L, int ic, int s, int lane, double rho_ic, double dn_ic,
                                              double f_ic, double alb_diff, double alb_dir, double sg_lw, double *acc,
                                              int lp, double *low) {
 #pragma clang fp contract(on)
-  constexpr int NP = kRowLanes / NS;   // positions
+  constexpr int NP = LN / NS;   // positions
   const int p = s / NS, q = s % NS, nl = L - ic;
   const int K = (nl + NP - 1) / NP;
-  const int v = row_value(row);
-  const bool first = p == 0, last = p == NP - 1;
+  const int v = row_value(lane / kRowLanes);
+  const bool first = p == 0, last = p == NP - 1, lead = q == 0 && leads<LN>(lane);
   const int n_clear = g.n_clear;
   double *m = low + lane;
   constexpr int Q = GEN ? kLowQ + 1 : kLowQ;   // the last one the gas absorption
@@ -490,7 +540,7 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
     }
     double F = 1.0;
     if (SOLAR) {
-      const double e = dpp_or1<kShr + NS>(product_scan<NS>(f));
+      const double e = below1<LN, NS>(product_scan<LN, NS>(f, s), s);
       F = f_ic * e;
       S.Su = S.Su * F;
       S.Sd = S.Sd * F;
@@ -501,8 +551,8 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
       S.Rb = first ? rb : S.Rb;
       S.Sd = first ? sd : S.Sd;
     }
-    slab_scan<NS>(S);
-    double rho = dpp_or0<kShr + NS>(S.Rb), dn = dpp_or0<kShr + NS>(S.Sd);
+    slab_scan<LN, NS>(S, s);
+    double rho = below0<LN, NS>(S.Rb, s), dn = below0<LN, NS>(S.Sd, s);
     if (first) { rho = rho_ic; dn = dn_ic; }
     double A = 1.0, C = 0.0;   // fu(top of the lane) = A fu(bottom) + C
     for (int k = 0; k < K; k++) {
@@ -523,31 +573,31 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
     {
       // level L, from the last position's lanes
       const double wl = last ? wj : 0.0;
-      double z = sum_rows(wl * fus, wl * (rho * fus + dn), wl * fdir, 0.0);
+      double z = sum_rows<LN>(wl * fus, wl * (rho * fus + dn), wl * fdir, 0.0);
       if (NS == 2) z = z + dpp_move<kXor1>(z);
-      if (last && q == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
+      if (last && lead && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
     }
     if (last) C = A * fus + C;
-    affine_up_scan<NS>(A, C);
-    double fu = dpp_or0<kShl + NS>(C);
+    affine_up_scan<LN, NS>(A, C, s);
+    double fu = above0<LN, NS>(C, s);
     if (last) fu = fus;
     for (int k = K - 1; k >= 0; k--) {
       fu = SG_LOW(k, 0) * fu + SG_LOW(k, 1);
       const double fd = SG_LOW(k, 2) * fu + SG_LOW(k, 3);
       const double fb = SOLAR ? F * SG_LOW(k, 4) : 0.0;
-      double z = sum_rows(wj * fu, wj * fd, wj * fb, 0.0);
+      double z = sum_rows<LN>(wj * fu, wj * fd, wj * fb, 0.0);
       if (NS == 2) z = z + dpp_move<kXor1>(z);
       const int r = p * K + k;
-      if (r < nl && q == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + ic + r, z);
+      if (r < nl && lead && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + ic + r, z);
     }
     if (first) xsum = xsum + wj * fu;
   }
 #undef SG_LOW
   if (NS == 2) xsum = xsum + dpp_move<kXor1>(xsum);
-  return dpp_or0<kBcast + 0>(xsum);
+  return of_first<LN>(xsum);
 }
 
-// The solves of one group of a column: some of its rounds of 4 g-points.
+// The solves of one group of a column: some of its rounds of 4 (or 16) g-points.
 // (mcica_sample.F90:453-930; monochromatic_radiance.F90:429-691;
 // mcica_column.F90:255-622; solver_homogen_direct.F90:93-127.)
 //
@@ -560,20 +610,21 @@ __device__ __forceinline__ double row_cloudy(const LaneCtx &c, const SgTerm &t, 
 // recomputes those layers for every sample.)
 //
 // Output: partial[wave][up, down, direct][L+1] of the group's weighted sums
-// (direct: solar calls only), FOLD: added to those of the groups before it.
-template <bool MIXED, int OPT, bool SOLAR, int KMAX, bool FOLD>
+// (direct: solar calls only); fold: of the wave's groups 0 to group.
+template <bool MIXED, int OPT, bool SOLAR, int KMAX, int LN>
 __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__restrict__ spec, int l_rayleigh,
                                            const double *__restrict__ colrec, const double *__restrict__ grec,
                                            const double *__restrict__ colscal, const double *__restrict__ bandrec,
                                            const double *__restrict__ bandscal, const double *__restrict__ c_sub,
                                            const double *__restrict__ cldopt, const double *__restrict__ aerrec,
-                                           double *__restrict__ partial, int wave, int group, int lane, double *acc,
-                                           int lp, double *low, double *hot) {
+                                           double *__restrict__ partial, int wave, bool fold, int group, int lane,
+                                           double *acc, int lp, double *low, double *hot) {
 #pragma clang fp contract(on)
   constexpr bool GEN = OPT != kOptPlain;
   const int L = d.L, NB = d.NB, G = spec->n_g;
-  const int col = FOLD ? wave : wave / d.nw, part = FOLD ? group : wave - col * d.nw;
-  const int s = lane % kRowLanes, row = lane / kRowLanes;
+  constexpr int kSolves = kWave / LN;
+  const int col = fold ? wave : wave / d.nw, part = fold ? group : wave - col * d.nw;
+  const int s = lane % LN;
   const double *cs = colscal + (size_t)col * SG_NS;
   const double fc = d.mcica ? cs[SG_S_FC] : 0.0;
   const bool cloudy = d.mcica && fc > 0.0;
@@ -587,10 +638,10 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
     for (int j = 0; j < kHotQ; j++) hot[j * lp + i] = r[j];
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-  const int n_round = (G + kRows - 1) / kRows;
+  const int n_round = (G + kSolves - 1) / kSolves;
   const int r1 = min(n_round, (part + 1) * d.rpw);
   for (int rd = part * d.rpw; rd < r1; rd++) {
-    const int item = rd * kRows + row;
+    const int item = rd * kSolves + lane / LN;
     const bool act = item < G;
     const int gi = act ? item : 0;
     const SgTerm t = spec->g[gi];
@@ -632,51 +683,52 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
     const double alb_diff = bs[2], alb_dir = bs[3];
     const double finc = SOLAR ? bs[0] / c.sec0 : -bs[0];   // flux_inc_down, flux_inc_direct
     const double sg_lw = SOLAR ? 0.0 : (1.0 - alb_diff) * (bs[1] - br[(L - 1) * SG_NBQ + 3]);
-    // the row's solves, and the most any row of the wave has
+    // the group's solves, and the most any group of the wave has
     const int n_clear = g.n_clear;
     int n_solve = n_clear + g.n_s;
-    n_solve = max(n_solve, __shfl_xor(n_solve, 16, kWave));
-    n_solve = __builtin_amdgcn_readfirstlane(max(n_solve, __shfl_xor(n_solve, 32, kWave)));
+#pragma unroll
+    for (int o = LN; o < kWave; o *= 2) n_solve = max(n_solve, __shfl_xor(n_solve, o, kWave));
+    n_solve = __builtin_amdgcn_readfirstlane(n_solve);
     const int nl = L - ic;
-    const RowMap mp = row_map(ic, s);
+    const RowMap mp = row_map<LN>(ic, s);
     const double W = g.w_clear + g.n_s * g.w_sub;
     // the layers from ic down: the surface, or the cloudy part first
     const auto below = [&](double rho, double dn, double fdir) -> double {
       if (nl == 0) {
         const double fus = surface_up<SOLAR>(alb_diff, alb_dir, sg_lw, rho, dn, fdir);
         const double X = W * fus;
-        const double z = sum_rows(X, W * (rho * fus + dn), W * fdir, 0.0);
-        const int v = row_value(row);
-        if (s == 0 && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
+        const double z = sum_rows<LN>(X, W * (rho * fus + dn), W * fdir, 0.0);
+        const int v = row_value(lane / kRowLanes);
+        if (s == 0 && leads<LN>(lane) && v < (SOLAR ? 3 : 2)) acc_add(acc + v * lp + L, z);
         return X;
       }
-      // two solves side by side where the cloudy layers fit 8 lanes of the row
-      if (nl <= 8 * kLowK)
-        return row_cloudy<MIXED, GEN, SOLAR, 2, 0>(c, t, src, spec, d.mode, g, (n_solve + 1) / 2, L, ic, s, row, lane,
-                                                   rho, dn, fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
-      return row_cloudy<MIXED, GEN, SOLAR, 1, KMAX>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, row, lane, rho, dn,
-                                                    fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+      // two solves side by side where the cloudy layers fit half of the group's lanes
+      if (nl <= LN / 2 * kLowK)
+        return row_cloudy<MIXED, GEN, SOLAR, 2, 0, LN>(c, t, src, spec, d.mode, g, (n_solve + 1) / 2, L, ic, s, lane,
+                                                       rho, dn, fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
+      return row_cloudy<MIXED, GEN, SOLAR, 1, KMAX, LN>(c, t, src, spec, d.mode, g, n_solve, L, ic, s, lane, rho, dn,
+                                                        fdir, alb_diff, alb_dir, sg_lw, acc, lp, low);
     };
     double rho, dn, fdir;
     if (!MIXED && !SOLAR && !c.aer) {
       // infra-red clear air without aerosols does not scatter
       RowState<KMAX, true> w;
-      row_down_absorb<GEN, KMAX>(c, t, src, ic, mp, s, finc, w, dn, low, lane);
-      const double X = below(0.0, dpp_or0<kBcast + 15>(dn), 0.0);
-      row_up<KMAX, true>(mp, s, row, X, W, w, acc, lp);
+      row_down_absorb<GEN, KMAX, LN>(c, t, src, ic, mp, s, finc, w, dn, low, lane);
+      const double X = below(0.0, of_last<LN>(dn), 0.0);
+      row_up<KMAX, true, LN>(mp, s, lane, X, W, w, acc, lp);
     } else {
       RowState<KMAX, false> w;
-      row_down<MIXED, GEN, SOLAR, KMAX>(c, t, src, ic, mp, s, row, finc, W, w, rho, dn, fdir, acc, lp, low, lane);
-      rho = dpp_or0<kBcast + 15>(rho);
-      dn = dpp_or0<kBcast + 15>(dn);
-      if (SOLAR) fdir = dpp_or0<kBcast + 15>(fdir);
+      row_down<MIXED, GEN, SOLAR, KMAX, LN>(c, t, src, ic, mp, s, finc, W, w, rho, dn, fdir, acc, lp, low, lane);
+      rho = of_last<LN>(rho);
+      dn = of_last<LN>(dn);
+      if (SOLAR) fdir = of_last<LN>(fdir);
       const double X = below(rho, dn, fdir);
-      row_up<KMAX, false>(mp, s, row, X, W, w, acc, lp);
+      row_up<KMAX, false, LN>(mp, s, lane, X, W, w, acc, lp);
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   double *out = partial + (size_t)wave * 3 * (L + 1);
-  const bool add = FOLD && group > 0;
+  const bool add = fold && group > 0;
   for (int i = lane; i <= L; i += kWave)
 #pragma unroll
     for (int v = 0; v < (SOLAR ? 3 : 2); v++) {
@@ -691,39 +743,40 @@ __device__ __forceinline__ void solve_rows(const CallDims &d, const SgSpec *__re
 __host__ __device__ constexpr int solve_low(int opt) {
   return kLowK * (opt == kOptPlain ? kLowQ : kLowQ + 1) * kWave;
 }
-template <int KMAX, int OPT>
+template <int KMAX, int OPT, int LN>
 __host__ __device__ constexpr int solve_lds_doubles() {
-  return solve_low(OPT) + (3 + kHotQ) * (KMAX * kRowLanes + 1);
+  return solve_low(OPT) + (3 + kHotQ) * (KMAX * LN + 1);
 }
 
-// Waves (64 threads each) of the calls of one build: W the work space. In
-// W_SOLVE_FOLD a wave takes a column's groups in turn, and sums them in the order in
-// which the output kernel sums those of a wave each. (A loop over the groups in every
-// build took 0.5 to 2 % of a step.)
-template <bool MIXED, int OPT, int KMAX, int W>
+// Waves (64 threads each) of the calls of one build: W the work space. Where FOLD is
+// set, a wave of a folding call takes a column's groups in turn, and sums them in the
+// order in which the output kernel sums those of a wave each. (A loop over the groups
+// in every build took 0.5 to 2 % of a step.)
+template <bool MIXED, int OPT, int KMAX, int LN, int W>
 __global__ __launch_bounds__(256, KMAX <= 9 ? 2 : 1) void b_solve_kernel(const BatchHdr *h, const ReqDesc *rq) {
   extern __shared__ double lds[];
-  constexpr int lp = KMAX * kRowLanes + 1;
-  constexpr bool FOLD = W == W_SOLVE_FOLD;
+  constexpr int lp = KMAX * LN + 1;
+  constexpr bool FOLD = W == W_SOLVE_FOLD || LN == kFewLanes;
   const long long tot = h->tot[W];
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
-  double *low = lds + wv * solve_lds_doubles<KMAX, OPT>(), *acc = low + solve_low(OPT), *hot = acc + 3 * lp;
+  double *low = lds + wv * solve_lds_doubles<KMAX, OPT, LN>(), *acc = low + solve_low(OPT), *hot = acc + 3 * lp;
   const long long nw = (long long)gridDim.x * (blockDim.x / kWave);
   for (long long w0 = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave; w0 < tot; w0 += nw) {
     const int w = __builtin_amdgcn_readfirstlane((int)w0);
     const int r = find_req(h, rq, W, w);
     const ReqDesc &q = rq[r];
     const int wave = w - (int)q.s[W];
-    const int n = FOLD ? q.d.nw : 1;
+    const bool fold = FOLD && q.d.fold;
+    const int n = fold ? q.d.nw : 1;
     for (int g = 0; g < n; g++) {
       if (q.d.isolir == SOCGPU_SOURCE_SOLAR)
-        solve_rows<MIXED, OPT, true, KMAX, FOLD>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
-                                                 G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                                 G(q.partial), wave, g, lane, acc, lp, low, hot);
+        solve_rows<MIXED, OPT, true, KMAX, LN>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+                                               G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
+                                               G(q.partial), wave, fold, g, lane, acc, lp, low, hot);
       else
-        solve_rows<MIXED, OPT, false, KMAX, FOLD>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
-                                                  G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
-                                                  G(q.partial), wave, g, lane, acc, lp, low, hot);
+        solve_rows<MIXED, OPT, false, KMAX, LN>(q.d, G(q.spec), q.l_rayleigh, G(q.colrec), G(q.grec), G(q.colscal),
+                                                G(q.bandrec), G(q.bandscal), G(q.csub), G(q.cldopt), G(q.aerrec),
+                                                G(q.partial), wave, fold, g, lane, acc, lp, low, hot);
     }
   }
 }

@@ -187,7 +187,7 @@ static void two_stream_cols(const TwoStreamArgs &a, hipStream_t s) {
 // Few layers: one lane per solve up to 3, 4 groups up to 12, since 16 groups would be
 // idle for the most part. FP64, a call in us with 16 groups and so: solar 65536 x 16
 // solves of 2 layers 186 and 51, of 5 264 and 109, of 10 379 and 174; infra-red 113,
-// 146, 173 and 48, 80, 132; 4096 x 16 solar solves of 12 layers 48 and 39.
+// 146, 222 and 48, 80, 132; 4096 x 16 solar solves of 12 layers 48 and 39.
 template <bool MIXED, bool SOLAR>
 static void two_stream_launch(const TwoStreamArgs &a, hipStream_t s) {
   if (a.L <= 3) two_stream_run<MIXED, SOLAR, 3, kWave, 1>(a, s);

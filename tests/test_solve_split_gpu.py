@@ -45,7 +45,8 @@ def least_gb(case, src, precision):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("src,P,L,kind", [("lw", 550, 90, "cloud"), ("sw", 8, 60, "cloud"), ("lw", 8, 100, "cloud"),
                                           ("sw", 40, 60, "cloud"), ("lw", 8, 50, "clear"), ("sw", 8, 70, "aerosol"),
-                                          ("lw", 17, 150, "aerosol")])
+                                          ("lw", 17, 150, "aerosol"), ("lw", 8, 20, "cloud"),
+                                          ("sw", 40, 10, "cloud")])
 def test_server_has_the_bits_of_the_call_alone(src, P, L, kind, precision):
     case = synth.make_case(P, L, src, NBAND[src], seed=P + L, cloudy=kind != "clear")
     if kind == "aerosol":
