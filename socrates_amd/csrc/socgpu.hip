@@ -1583,7 +1583,10 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
 // Groups of a column's rounds of 4 (few layers: 16) g-points, a solve wave each. A wave
 // first brings its column into LDS and at its end writes its partial sums, so it
 // should have several rounds; the chip holds 2048 waves of this kernel (two per
-// SIMD), so a call should have about as many. From 16 columns a wave has 3
+// SIMD), so a call should have about as many. (That is for calls of up to 96 layers.
+// The LDS of a wave of the longer builds leaves a CU 7, with general optics or
+// aerosols 6, and above 144 layers 5 of them; the split was not tuned for these.)
+// From 16 columns a wave has 3
 // rounds at least (10 000 columns in 216 calls of about 46, mixed: 2.66 ms per
 // batch with one round per wave, 2.45 ms with three); a call of fewer columns
 // takes a wave per round, the shortest chain (4096 x 90 SW + LW, FP64: 1.20 ms
@@ -1811,12 +1814,13 @@ static void place_request(ReqDesc &q, const SgSpec &S, double *base, size_t *cur
   q.csub = d.mcica ? take(P * L * SG_MAXSUBCOL) : nullptr;
   q.cldopt = d.mcica ? take(P * NB * L * d.co_stride) : (d.triple ? take(P * NB * L * 8) : nullptr);
   q.ovl = d.triple ? take(P * (L + 1) * kOv) : nullptr;
+  if (d.triple) *cursor = (*cursor + 15) & ~(size_t)15;   // its rows on lines (tri_row)
   q.tws = d.triple ? take(P * L * kTriQ * tri_row(d.n_g)) : nullptr;
   q.aerrec = d.n_aer ? take(P * NB * L * 4) : nullptr;
 }
 
 static size_t padded_ws_doubles(const CallDims &d, const SgSpec &S) {
-  return request_ws_doubles(d, S) + 13 * 3;  // per-array alignment padding
+  return request_ws_doubles(d, S) + 13 * 3 + 12;  // alignment of each array
 }
 
 // A one-call descriptor block written into device memory by a kernel that

@@ -30,10 +30,12 @@ constexpr int kTriHot = 12;               // column record slots in LDS: lnp, ln
                                           // cloud fraction, the two types' fractions, their reciprocals
 
 __host__ __device__ inline int tri_chunks(int n_g) { return (n_g + kTriTerms - 1) / kTriTerms; }
-// Doubles per layer and state of a column's workspace: whole 128-byte lines for
-// each wave (rows of 3 n_g, whose lines two waves write in part, had the 4096 x 90
-// step at 2515 us instead of 1578), but never more than the 64 lanes per 64 k-terms
-// and three regions that callers' workspaces have held.
+// Doubles per layer and state of a column's workspace, which starts on a line: whole
+// 128-byte lines for each wave (rows of 3 n_g, whose lines two waves write in part, had
+// the 4096 x 90 step at 2515 us instead of 1578; whole lines of a workspace that began
+// within one 1506 instead of 1489), but never more than the 64 lanes per 64 k-terms and
+// three regions that callers' workspaces have held: 64 k-terms, whose padded row would
+// be longer, take rows of 3 n_g.
 __host__ __device__ inline int tri_row(int n_g) {
   const int full = n_g / kTriTerms, last = 3 * (n_g - full * kTriTerms);
   const int row = kWave * full + (last + 15) / 16 * 16, most = 3 * kWave * ((n_g + kWave - 1) / kWave);
