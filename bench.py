@@ -294,6 +294,8 @@ def main():
             tiles[prec] = R.autotune(calls, prec)
         else:
             tiles[prec] = R.get_tile(prec)
+        # (the tile's other fields change nothing)
+        tiles[prec] = {"waves_per_block": tiles[prec]["waves_per_block"]}
         # solve-kernel time (HIP events on the library stream) from the
         # stream form of the same batch
         ks = []

@@ -107,8 +107,6 @@ struct SgSpec {
   // [0] single and [1] optimal sampling
   int has_mcica, n_gen, ipph, n1, n2;
   int n_req[2];
-  int n_sub_items[2];
-  int sub_g[2][SG_MAXSUB];      // g-point of each sub item
   int sub_isub[2][SG_MAXSUB];   // generated sub-column (1-based) it samples
   double sub_inv_s[2][SG_MAXSUB];
   int g_n_sub[2][SG_MAXG];      // sub items per g-point

@@ -626,13 +626,11 @@ int attach_mcica(SgSpec *s, const McicaData &m, bool solar, std::string *err) {
         if (item >= SG_MAXSUB) { *err = "too many McICA samples"; return -3; }
         int idx = msamp % n_req;
         if (idx == 0) idx = n_req;
-        s->sub_g[mode][item] = gi;
         s->sub_isub[mode][item] = reorder[idx];
         s->sub_inv_s[mode][item] = 1.0 / (double)nsub;
         item++;
       }
     }
-    s->n_sub_items[mode] = item;
   }
   return 0;
 }
