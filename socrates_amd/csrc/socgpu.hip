@@ -919,9 +919,9 @@ struct ReqDesc {
 // err: 0, or 1 + the (descriptor-order) index of a request whose input the
 // kernels found invalid (a cloud fraction above 1.001); the host writes 0
 // with every descriptor upload and reads it back after the launch.
-struct BatchHdr {
+struct alignas(8) BatchHdr {   // descriptors follow it
   int R, err;
-  long long tot[kNWork];
+  int tot[kNWork];
 };
 
 // A call's arguments with every input pointer seen as global (G).
@@ -1963,13 +1963,13 @@ int socgpu_runes(const char *spectrum_name, const SocgpuRunesArgs *a, SocgpuDiag
   long long w[kNWork];
   request_work(d, S, w);
   host.h.R = 1;
-  for (int k = 0; k < kNWork; k++) { host.q.s[k] = 0; host.h.tot[k] = w[k]; }
+  for (int k = 0; k < kNWork; k++) { host.q.s[k] = 0; host.h.tot[k] = (int)w[k]; }
   hipStream_t s = g_ctx.stream;
   HIPCHK(hipEventRecord(g_ctx.ev0, s));
   HIPCHK(hipMemcpyAsync(g_ctx.desc.p, &host, sizeof host, hipMemcpyHostToDevice, s));
   const BatchHdr *dh = (const BatchHdr *)g_ctx.desc.p;
   const ReqDesc *dq = (const ReqDesc *)((char *)g_ctx.desc.p + offsetof(decltype(host), q));
-  if (int rc = launch_batch(dh, (ReqDesc *)dq, host.h.tot, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
+  if (int rc = launch_batch(dh, (ReqDesc *)dq, w, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
   HIPCHK(hipEventRecord(g_ctx.ev3, s));
   int herr = 0;
   HIPCHK(hipMemcpyAsync(&herr, &dh->err, sizeof herr, hipMemcpyDeviceToHost, s));
@@ -2047,12 +2047,12 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   long long w[kNWork];
   request_work(d, S, w);
   host.h.R = 1;
-  for (int k = 0; k < kNWork; k++) { host.q.s[k] = 0; host.h.tot[k] = w[k]; }
+  for (int k = 0; k < kNWork; k++) { host.q.s[k] = 0; host.h.tot[k] = (int)w[k]; }
   hipStream_t s = g_ctx.stream;
   DescBlob *dd = (DescBlob *)g_ctx.scratch_dev;
   HIPCHK(hipEventRecord(g_ctx.ev0, s));
   b_desc_store_kernel<<<1, 64, 0, s>>>(host, dd);
-  if (int rc = launch_batch(&dd->h, &dd->q, host.h.tot, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
+  if (int rc = launch_batch(&dd->h, &dd->q, w, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
   HIPCHK(hipEventRecord(g_ctx.ev3, s));
   HIPCHK(hipMemcpyAsync(g_ctx.err_host, &dd->h.err, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
@@ -2222,7 +2222,7 @@ static int plan_place(const std::vector<Resolved> &res, Plan &pl, double *ws, ch
       start[k] += res[i].w[k];
     }
   }
-  for (int k = 0; k < kNWork; k++) pl.h.tot[k] = start[k];
+  for (int k = 0; k < kNWork; k++) pl.h.tot[k] = (int)start[k];
   pl.out_used = out_cur;
   pl.in_used = in_off;
   if (in_host && in_off > 0) HIPCHK(hipMemcpyAsync(in_stage, in_host, in_off, hipMemcpyHostToDevice, s));
@@ -2300,7 +2300,7 @@ int socgpu_runes_batch(int n_request, const SocgpuRequest *requests, int precisi
   HIPCHK(hipMemcpyAsync(g_ctx.desc.p, blob.data(), blob.size(), hipMemcpyHostToDevice, s));
   const BatchHdr *dh = (const BatchHdr *)g_ctx.desc.p;
   ReqDesc *dq = (ReqDesc *)((char *)g_ctx.desc.p + sizeof(BatchHdr));
-  if (int rc = launch_batch(dh, dq, pl.h.tot, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
+  if (int rc = launch_batch(dh, dq, pl.need, precision, s, &g_ctx.fork, g_ctx.ev1, g_ctx.ev2)) return rc;
   HIPCHK(hipEventRecord(g_ctx.ev3, s));
   int herr = 0;
   HIPCHK(hipMemcpyAsync(&herr, &dh->err, sizeof herr, hipMemcpyDeviceToHost, s));
@@ -2556,7 +2556,7 @@ static int serve_launch(SocgpuServer *sv, ServeSlot &sl) {
   HIPCHK(hipMemcpyAsync(sl.desc.p, sl.pinned, desc_bytes(nq), hipMemcpyHostToDevice, s));
   const BatchHdr *dh = (const BatchHdr *)sl.desc.p;
   ReqDesc *dq = (ReqDesc *)((char *)sl.desc.p + sizeof(BatchHdr));
-  if (int rc = launch_batch(dh, dq, sl.plan.h.tot, sv->cfg.precision, s, &sl.fork, nullptr, nullptr)) return rc;
+  if (int rc = launch_batch(dh, dq, sl.plan.need, sv->cfg.precision, s, &sl.fork, nullptr, nullptr)) return rc;
   HIPCHK(hipMemcpyAsync(&((BatchHdr *)sl.pinned)->err, &dh->err, sizeof(int), hipMemcpyDeviceToHost, s));
   if (int rc = copy_back_issue(sl.plan, sl.out_stage.as<double>(), sl.out_host_used, s)) return rc;
   HIPCHK(hipEventRecord(sl.done, s));
@@ -2950,7 +2950,7 @@ int socgpu_cloud_gen(int n_profile, int n_layer, int n_subcol, int n_req, int ip
   std::memset(&host, 0, sizeof host);
   host.h.R = 1;
   host.h.tot[W_CG] = P;
-  host.h.tot[W_CCOL] = (long long)P * ((L + kRangeChunk - 1) / kRangeChunk);
+  host.h.tot[W_CCOL] = P * ((L + kRangeChunk - 1) / kRangeChunk);
   host.q.a.cloud_frac = dcf.as<double>();
   host.q.d = d;
   host.q.colrec = drec.as<double>();

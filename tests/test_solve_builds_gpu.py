@@ -9,6 +9,7 @@ column's largest; check_mixed), in FP64 plus twice the oracle's own largest move
 in the column under one-ulp changes of its exponentials (exp_spread of
 test_aerosol_gpu). Columns with cloud up to their top are compared in FP64 only: the
 mixed form's heating-rate bound is that of cloud in the troposphere."""
+import numpy as np
 import pytest
 
 import test_solve_rows_gpu
@@ -79,3 +80,21 @@ def test_triple_mixed(src, shape):
     case = test_tri_rows_gpu.make(src, P, L, n, 6000 + 10 * L + n + (src == "sw"))
     ref = oracle.runes(case, files_of("synth")[src], None)
     check_mixed(R.runes_case(case, src, precision="mixed"), ref, "triple mixed %s %s" % (src, shape))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("L", [20, 97, 145])
+def test_waves_per_block(L, precision):
+    """Blocks of 1, 2 and 4 waves (more LDS than 64 KB above 96 layers) give the same bits."""
+    case = synth.add_aerosols(test_solve_rows_gpu.make("sw", 7, L, L // 3, 8900 + L), 2, 8901)
+    saved = R.get_tile(precision)
+    try:
+        out = []
+        for waves in (1, 2, 4):
+            R.set_tile(precision, 0, waves)
+            out.append(R.runes_case(case, "sw", precision=precision))
+    finally:
+        R.set_tile(precision, saved["recompute"], saved["waves_per_block"], saved["waves_per_simd"])
+    for o in out[1:]:
+        for k in o:
+            assert np.array_equal(o[k], out[0][k]), k

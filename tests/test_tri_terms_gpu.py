@@ -9,11 +9,13 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
 import test_tri_rows_gpu
 from oracle import oracle
 from socrates_amd import runes as R
 from test_gpu_parity import SPEC, check_fp64, check_mixed
+from test_zz_no_alloc import FIELDS, _outs
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
 import make_spectra  # noqa: E402
@@ -48,3 +50,24 @@ def test_rows_by_number_of_terms(tmp_path, n_g):
     check_fp64(R.runes_case(case, name, precision="fp64"), ref, "triple %d terms" % n_g, "lw",
                case.layer_heat_capacity, spread=sp)
     check_mixed(R.runes_case(case, name, precision="mixed"), ref, "triple %d terms mixed" % n_g)
+
+
+def test_room_of_a_call(tmp_path):
+    """A 64-term call needs no more room in the fixed workspace than with a lane per
+    k-term and three regions of 4 words: records of 21 words per layer and its level
+    temperature, scalars, band and cloud records, overlaps, level sums, the solve's
+    state, 52 words of alignment and 1280 bytes of descriptor."""
+    P, L, NB = 400, 90, 9
+    name = "lw_64_terms"
+    R.set_spectrum(name, spectrum(tmp_path / "sp", 64))
+    case = test_tri_rows_gpu.make("lw", P, L, 17, 7100)
+    arrs = {k: torch.from_numpy(np.ascontiguousarray(getattr(case, k))).cuda()
+            for k in FIELDS + ("conv_frac", "liq_conv_mmr", "liq_conv_dim")}
+    arrs["cos_zenith_angle"] = torch.from_numpy(np.ascontiguousarray(case.cos_zen)).cuda()
+    _, kw = R.case_call(case, name, device_arrays=arrs, out=_outs(case))
+    with pytest.raises(R.SocgpuError) as e:
+        R.runes_noalloc(kw.pop("n_profile"), kw.pop("n_layer"), name, kw.pop("i_source"), **kw)
+    need = int(re.search(r"needs (\d+) bytes", str(e.value)).group(1))
+    words = (P * L * 21 + P * (L + 1) + P * 7 + P * NB * L * 4 + P * NB * 4 + 2 + P * NB * L * 8 + P * (L + 1) * 18 +
+             P * (L + 1) * 3 + P * L * 3 * 4 * 64)
+    assert need <= 1280 + 8 * (words + 52)
