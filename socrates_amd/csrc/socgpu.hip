@@ -1593,15 +1593,20 @@ static int stage_inputs(const SocgpuRunesArgs *a, SocgpuRunesArgs *dv, int NB) {
 // per step with 8192 waves per call, 1.18 ms with 2048 to 4096).
 constexpr long long kSolveWaves = 2048;
 // The groups fix the order in which the g-points are summed, so they are the same
-// wherever the call is made. Where a wave each needs too much room for the partial
-// sums (the fixed workspace, a serving budget), one wave takes them in turn (fold).
-static void solve_layout(CallDims &d, const SgSpec &S) {
+// wherever the call is made: a call that fits the fixed workspace with fewer groups,
+// and so fewer partial sums (max_groups), takes that many in every entry point. Where
+// they need more room than a serving budget has, one wave takes them in turn (fold).
+static void solve_layout(CallDims &d, const SgSpec &S, int max_groups = INT32_MAX) {
   const int per = kWave / (d.L <= kFewL ? kFewLanes : kRowLanes), rounds = (S.n_g + per - 1) / per;
-  const int most = d.P < 16 ? rounds : (rounds + 2) / 3;
+  const int most = std::min(max_groups, d.P < 16 ? rounds : (rounds + 2) / 3);
   const long long want = std::max<long long>(1, std::min<long long>(most, (kSolveWaves + d.P - 1) / d.P));
   d.rpw = (int)((rounds + want - 1) / want);
   d.nw = (rounds + d.rpw - 1) / d.rpw;
 }
+
+// Bytes of the fixed workspace a call takes: its descriptor, then its arrays.
+static size_t noalloc_offset();
+static size_t noalloc_bytes(const CallDims &d, const SgSpec &S);
 
 // Checks one call's arguments and resolves its options (socrates_set_control
 // defaults on the two-stream path); fills the request's shapes.
@@ -1749,6 +1754,12 @@ static int resolve_request(const char *spectrum_name, const SocgpuRunesArgs *a, 
   }
   d.n_g = S.n_g;
   solve_layout(d, S);
+  if (noalloc_bytes(d, S) > kScratchBytes) {
+    CallDims least = d;
+    solve_layout(least, S, 1);
+    if (noalloc_bytes(least, S) <= kScratchBytes)
+      while (noalloc_bytes(d, S) > kScratchBytes) solve_layout(d, S, d.nw - 1);
+  }
   *entry = &e;
   *dout = d;
   return 0;
@@ -1831,6 +1842,10 @@ struct DescBlob {
   ReqDesc q;
 };
 
+static size_t noalloc_offset() { return (sizeof(DescBlob) + 255) & ~(size_t)255; }
+static size_t noalloc_bytes(const CallDims &d, const SgSpec &S) {
+  return noalloc_offset() + padded_ws_doubles(d, S) * 8;
+}
 static_assert(sizeof(DescBlob) % 8 == 0, "descriptor block is copied in 8-byte words");
 
 static void fill_desc(ReqDesc &q, const CallDims &d, const SpecEntry &e, const SocgpuRunesArgs &dv,
@@ -2033,9 +2048,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   CallDims d;
   if (int rc = resolve_request(spectrum_name, a, precision, &e, &d)) return rc;
   const SgSpec &S = e->host;
-  const size_t ws_off = (sizeof(DescBlob) + 255) & ~(size_t)255;
-  d.fold = ws_off + padded_ws_doubles(d, S) * 8 > kScratchBytes;
-  const size_t need = ws_off + padded_ws_doubles(d, S) * 8;
+  const size_t need = noalloc_bytes(d, S);
   if (need > kScratchBytes)
     return fail(SOCGPU_ENOMEM, "call needs %zu bytes of workspace, above the %zu-byte fixed workspace of "
                                "socgpu_runes_noalloc (use socgpu_runes)", need, kScratchBytes);
@@ -2043,7 +2056,7 @@ int socgpu_runes_noalloc(const char *spectrum_name, const SocgpuRunesArgs *a, So
   std::memset(&host, 0, sizeof host);
   fill_desc(host.q, d, *e, *a, diag->flux_up, diag->flux_down, diag->flux_direct, diag->heating_rate);
   size_t cursor = 0;
-  place_request(host.q, S, (double *)(g_ctx.scratch_dev + ws_off), &cursor);
+  place_request(host.q, S, (double *)(g_ctx.scratch_dev + noalloc_offset()), &cursor);
   long long w[kNWork];
   request_work(d, S, w);
   host.h.R = 1;

@@ -1,6 +1,6 @@
-"""A call's k-term sums are grouped alike wherever it is made: alone, in the server
-whatever its budget, and in the fixed workspace, where a wave that takes all of a
-column's groups in turn has the bits of a wave for each."""
+"""A call's k-term sums are grouped alike wherever it is made: alone, in a batch, in the
+fixed workspace, and in the server whatever its budget, where a wave that takes all of
+a column's groups in turn has the bits of a wave for each."""
 import re
 
 import numpy as np
@@ -40,8 +40,8 @@ def least_gb(case, src, precision):
     return (int(re.search(r"needs (\d+) bytes", str(e.value)).group(1)) + 8) / 2.0 ** 30
 
 
-# 550 x 90 infra-red: above the fixed workspace with a wave per group, below it
-# with one; 8 columns: a group per round; 40: three rounds a group
+# 550 x 90 infra-red: fits the fixed workspace with fewer groups than a call of its
+# size takes otherwise; 8 columns: a group per round; 40: three rounds a group
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("src,P,L,kind", [("lw", 550, 90, "cloud"), ("sw", 8, 60, "cloud"), ("lw", 8, 100, "cloud"),
                                           ("sw", 40, 60, "cloud"), ("lw", 8, 50, "clear"), ("sw", 8, 70, "aerosol"),
