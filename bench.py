@@ -70,7 +70,7 @@ HBM_PEAK = 8000.0                          # GB/s
 # FETCH_SIZE and WRITE_SIZE runs of this script on the same build, each scaled
 # by what the counter reads for a plain copy of known size; the summary, its
 # commands and the scale factors are in TRAFFIC_SOURCE
-TRAFFIC = {"mixed": 0.410e9, "fp64": 0.528e9}
+TRAFFIC = {"mixed": 0.409e9, "fp64": 0.527e9}
 TRAFFIC_SOURCE = "profiles/c2_solve_traffic.md"
 
 

@@ -164,7 +164,7 @@ struct SgSpec {
 #define SG_S_LFG 6     // 1: the ground source of each band is given (band scalar 1)
 #define SG_NS 7
 
-// per (col, band, layer) record from the preparation kernel, [col][band][layer][4]
+// per (col, band, layer) record from the band kernel, [col][band][layer][4]
 //  LW: k_grey_tot, planck diff, planck diff_2, planck at the bottom level
 //  SW: k_grey_tot, adjust_solar_ke, 0, 0
 // per (col, band) scalars [col][band][4]

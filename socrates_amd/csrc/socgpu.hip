@@ -711,7 +711,7 @@ __device__ __forceinline__ void layer_coef_mixed(const LaneCtx &c, const SgTerm 
   float tau, om, omc, g;
   const bool cloudy = !CLR && csub * frac1 > 0.0;
   if (cloudy) {
-    // absorption kext - kscat formed in FP64 by the prep kernel (relative
+    // absorption kext - kscat formed in FP64 by the band kernel (relative
     // accuracy ~1e-10 even for weakly absorbing droplets), kept in FP32
     const float kext = (float)co[0], kabs = (float)co[1];
     const float phf = (float)co[2], fwd = (float)co[3];
@@ -892,8 +892,9 @@ __device__ __forceinline__ void overlap_body(const CallDims &d, const double *__
 // W_GEN counts the calls that need the general build of the triple-column solve.
 // W_SOLVE + 3 i + opt: waves of the solve, by the build that runs them (i = 0
 // for calls of up to kFewL layers, 1 up to kShortL, 2 up to kLongL; opt: kOptPlain, kOptGen,
-// kOptAer); W_SOLVE_ANY: calls of more layers; W_SOLVE_FOLD: any call whose columns'
-// groups of g-points one wave takes in turn (CallDims::fold)
+// kOptAer); W_SOLVE_ANY: calls of more layers; W_SOLVE_FOLD: calls of more than
+// kFewL layers whose columns' groups of g-points one wave takes in turn
+// (CallDims::fold; shorter ones fold in their own build)
 // W_TSOLVE + 2 i + odd: columns of the triple-column solve, i = 0 and 1 as there,
 // 2 for calls of more layers (they differ in the LDS a block takes); odd: blocks
 // of three waves instead of two (an odd number of waves' k-terms)
@@ -1313,10 +1314,9 @@ __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // A second stream beside a launch stream, and the events that fork the cloud
 // generator onto it after the cloud range is known and join it back before
-// the solve: the generator (one wave per column) and the band kernel (one
-// wave per column and band) depend on the same inputs but not on each
-// other, and both spend most of their time waiting on memory, so they share
-// the device. Streams are created with the default priority.
+// the solve: the generator (one wave per column) and the band kernel (16 lanes
+// per column) depend on the same inputs but not on each other, and the generator
+// spends most of its time waiting, so they share the device. Streams are created with the default priority.
 struct Fork {
   hipStream_t side = nullptr;
   hipEvent_t f = nullptr, j = nullptr;
@@ -1349,9 +1349,9 @@ struct Context {
   std::mutex mu;
 };
 static Context g_ctx;
-// solve-kernel tile per precision form ([0] FP64, [1] mixed); the defaults
-// are the autotuner's picks on the 4096-column x 90-layer all-sky SW + LW
-// batch
+// solve-kernel tile per precision form ([0] FP64, [1] mixed): one wave per block,
+// the autotuner's pick on the 4096-column x 90-layer all-sky SW + LW batch (the
+// other two fields change nothing)
 static SocgpuTile g_tile[2] = {{0, 1, 3}, {1, 1, 3}};
 
 static int ensure_init() {

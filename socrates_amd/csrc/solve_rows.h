@@ -18,10 +18,10 @@
 //    scan gives every lane that flux.
 // Between the sweeps a lane's layers stay in its registers, as far as 256 of them go:
 // the builds of up to 24 layers spill none to 39, those of up to 96 none to 27, of up
-// to 144 20 to 93, and above 144 layers (512 registers) up to 20. Cloud that reaches above the LDS state is
-// in lane-private memory (240 to 576 B a lane). One lane per solve kept the
-// elimination state of all layers in lane-private memory (20 KB a lane): the
-// solve then moved 4.6 GB of scratch per 4096 x 90 SW + LW step, waited 63 % of its
+// to 144 20 to 93, and above 144 layers (512 registers) up to 20. The layers of deep
+// cloud, more of them than the LDS holds, are in lane-private memory (240 to 576 B a
+// lane). One lane per solve kept the elimination state of all layers there (20 KB a
+// lane): the solve then moved 4.6 GB of scratch per 4096 x 90 SW + LW step, waited 63 % of its
 // cycles and took 1157 us (FP64). Now it moves 0.5 GB (0.4 mixed) in 559 us (511) and
 // is bound by VALU issue: 74 % of the cycles with the two waves per SIMD that 256
 // registers a lane allow.

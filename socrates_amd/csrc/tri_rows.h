@@ -17,10 +17,11 @@
 // solar direct beam has a sweep of its own that forms its transmission again
 // (keeping all coefficients of that sweep for the elimination moved 28 % more
 // bytes and took 1578 us instead of 1516 in a 4096 x 90 FP64 step, SW + LW).
-// What bounds it: the workspace, 2.6 GB of that step's 1050 us, beside FP64
-// arithmetic (56 % of the cycles). One lane per k-term (all regions in turn, 64
-// k-terms a wave) took 1605 us, waiting 74 % of its cycles on the column's records
-// and the workspace with 2.7 waves per SIMD.
+// What bounds it: the workspace (2.0 GB read and 1.5 GB written in that step's two
+// solves of 1165 us together) beside FP64 arithmetic (VALU busy in 57 % of the
+// cycles). One lane per k-term (all regions in turn, 64 k-terms a wave) took 1605 us
+// there, waiting 74 % of its cycles on the column's records and the workspace with
+// 2.7 waves per SIMD.
 #pragma once
 
 constexpr int kTriTerms = kWave / 3;      // k-terms per wave

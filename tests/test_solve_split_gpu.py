@@ -9,6 +9,7 @@ import pytest
 from socrates_amd import runes as R
 from socrates_amd import synth
 from socrates_amd.serve import Server
+from test_ga9_gpu import MCICA_GA9, NAME, SPEC_GA9, WM
 from test_gpu_parity import NBAND
 from test_zz_no_alloc import _device, _outs
 
@@ -70,3 +71,17 @@ def test_batch_and_fixed_workspace_have_the_bits_of_the_call_alone():
         if k in res[0]:
             for r in res[1:]:
                 assert np.array_equal(r[k].cpu().numpy(), res[0][k].cpu().numpy()), k
+
+
+@pytest.mark.parametrize("src", ["sw", "lw"])
+def test_server_general_optics(src):
+    for s in ("sw", "lw"):
+        R.set_spectrum(NAME[s], SPEC_GA9[s])
+    R.set_mcica(MCICA_GA9, sw_spectrum_name=NAME["sw"], lw_spectrum_name=NAME["lw"])
+    for P, L in ((20, 60), (9, 100), (20, 20)):
+        case = synth.make_case(P, L, src, NBAND[src], seed=P + L, cloudy=True)
+        case.wm_mix_ratio = WM.copy()
+        ref = R.runes_case(case, NAME[src], precision="mixed")
+        out = served(case, NAME[src], "mixed", least_gb(case, NAME[src], "mixed"))
+        for k in FLUXES:
+            assert np.array_equal(np.asarray(out[k]), np.asarray(ref[k])), (k, P, L)
